@@ -14,6 +14,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <map>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -106,10 +107,12 @@ struct pdem_ctx {
   int mixed_tpb = 1024;    // mixed tile kernels' workgroup size (autotuned)
   int tile_nodes = TILE_NODES;
   std::vector<int> nbr_lo, nbr_hi;  // per-node neighbor id range (tile windows)
-  int* d_slot = nullptr;            // mixed thread slot -> node
-  int64_t* d_sp16 = nullptr;        // mixed 16-bit id slices, by slot
+  // lists of the mixed tiles (DevTile)
   uint16_t* d_col16 = nullptr;
-  size_t col16_cap = 0;
+  float* d_wgt = nullptr;
+  uint32_t* d_lnode = nullptr;
+  int* d_lslice = nullptr;
+  size_t col16_cap = 0, wgt_cap = 0, lnode_cap = 0, lslice_cap = 0;
   // learned pair-contact closure
   bool cl_ready = false;        // closure data allocated (pdem_closure_setup)
   ClosureArgs ca{};
@@ -156,6 +159,16 @@ struct pdem_ctx {
     auto it = std::find(allocs.begin(), allocs.end(), p);
     if (it != allocs.end()) allocs.erase(it);
     HIPCHK(hipFree(p));
+  }
+  // a buffer of at least n elements (contents lost when it grows)
+  template <class T>
+  void grow(T*& p, size_t& cap, size_t n) {
+    if (n <= cap) return;
+    if (p) dfree(p);
+    p = nullptr;
+    cap = 0;
+    p = dalloc<T>(n, false);
+    cap = n;
   }
   template <class T>
   T* upload(const T* h, size_t n) {
@@ -247,55 +260,60 @@ struct Launch {
     if (c->mixed.n_open_pids > 0)
       hipLaunchKernelGGL(k_mixed_umax<DIM>, dim3(c->mixed.n_open_pids), dim3(256), 0, st, c->ds, c->mixed);
   }
-  template <int INF, int T>
-  static void mixed_dilation(pdem_ctx* c) {
-    const MixedArgs& ma = c->mixed;
-    mixed_umax(c, c->stream);
-    if (ma.ntiles_hbm) {
-      fork(c);
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, false, T>), dim3(ma.ntiles_hbm), dim3(T), 0, c->side,
-                         c->ds, ma);
-      HIPCHK(hipEventRecord(c->ev_join, c->side));
-    }
-    if (ma.ntiles_lds && ma.small)
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, true, T, LDS_SMALL>), dim3(ma.ntiles_lds), dim3(T), 0, c->stream,
-                         c->ds, ma);
-    else if (ma.ntiles_lds)
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, true, T>), dim3(ma.ntiles_lds), dim3(T), 0, c->stream,
-                         c->ds, ma);
-    if (ma.ntiles_hbm) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
-  }
-  template <int INF, int T>
-  static void mixed_force(pdem_ctx* c) {
-    const MixedArgs& ma = c->mixed;
-    if (ma.ntiles_hbm) {
-      fork(c);
-      hipLaunchKernelGGL((k_mixed_force<DIM, INF, false, T>), dim3(ma.ntiles_hbm), dim3(T), 0, c->side,
-                         c->ds, ma);
-      HIPCHK(hipEventRecord(c->ev_join, c->side));
-    }
-    if (ma.ntiles_lds && ma.small)
-      hipLaunchKernelGGL((k_mixed_force<DIM, INF, true, T, LDS_SMALL>), dim3(ma.ntiles_lds), dim3(T), 0, c->stream,
-                         c->ds, ma);
-    else if (ma.ntiles_lds)
-      hipLaunchKernelGGL((k_mixed_force<DIM, INF, true, T>), dim3(ma.ntiles_lds), dim3(T), 0, c->stream,
-                         c->ds, ma);
-    if (ma.ntiles_hbm) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
-  }
   // The state-based passes of the mixed kernels: closed tiles (whole
   // particles) in the fused kernel on the engine stream; open LDS tiles and
-  // HBM tiles in the two-pass kernels (dilation of all, then force of all,
-  // since their force pass reads other tiles' dilation terms) on the side
-  // stream beside them.  Without closed tiles the open LDS tiles keep the
-  // engine stream and the HBM tiles the side stream.
-  template <int INF, int T>
+  // HBM tiles in the two-pass kernels (first pass of all, then second of all,
+  // since a tile's second pass reads other tiles' b terms).  Beside closed
+  // tiles the two-pass kernels run on the side stream; without them the open
+  // LDS tiles keep the engine stream and the HBM tiles the side stream.
+  // T: workgroup size.
+  // GEOM: the LDS tiles evaluate the weights (MixedArgs::geom).
+  template <int T, bool GEOM>
+  static void open_first(pdem_ctx* c, hipStream_t st) {
+    const MixedArgs& ma = c->mixed;
+    const dim3 g((unsigned)ma.ntiles_lds), t(T);
+    if (ma.ntiles_lds && ma.small)
+      hipLaunchKernelGGL((k_mixed_dilation<DIM, true, GEOM, T, LDS_SMALL>), g, t, 0, st, c->ds, ma);
+    else if (ma.ntiles_lds)
+      hipLaunchKernelGGL((k_mixed_dilation<DIM, true, GEOM, T>), g, t, 0, st, c->ds, ma);
+  }
+  template <int T, bool GEOM>
+  static void open_second(pdem_ctx* c, hipStream_t st) {
+    const MixedArgs& ma = c->mixed;
+    const dim3 g((unsigned)ma.ntiles_lds), t(T);
+    if (ma.ntiles_lds && ma.small)
+      hipLaunchKernelGGL((k_mixed_force<DIM, true, GEOM, T, LDS_SMALL>), g, t, 0, st, c->ds, ma);
+    else if (ma.ntiles_lds)
+      hipLaunchKernelGGL((k_mixed_force<DIM, true, GEOM, T>), g, t, 0, st, c->ds, ma);
+  }
+  static void hbm_first(pdem_ctx* c, hipStream_t st) {
+    const MixedArgs& ma = c->mixed;
+    if (ma.ntiles_hbm)
+      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB>), dim3((unsigned)(ma.ntiles_hbm * ma.hbm_split)),
+                         dim3(HBM_TPB), 0, st, c->ds, ma);
+  }
+  static void hbm_second(pdem_ctx* c, hipStream_t st) {
+    const MixedArgs& ma = c->mixed;
+    if (ma.ntiles_hbm)
+      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB>), dim3((unsigned)(ma.ntiles_hbm * ma.hbm_split)),
+                         dim3(HBM_TPB), 0, st, c->ds, ma);
+  }
+  template <int T, bool GEOM>
   static void mixed_state(pdem_ctx* c) {
     const MixedArgs& ma = c->mixed;
     const int grp = c->ev_next_group++;
     if (ma.ntiles_closed == 0) {
       auto ev = ev_begin(c, c->stream);
-      mixed_dilation<INF, T>(c);
-      mixed_force<INF, T>(c);
+      mixed_umax(c, c->stream);
+      for (int pass = 0; pass < 2; pass++) {
+        if (ma.ntiles_hbm) {
+          fork(c);
+          pass == 0 ? hbm_first(c, c->side) : hbm_second(c, c->side);
+          HIPCHK(hipEventRecord(c->ev_join, c->side));
+        }
+        pass == 0 ? open_first<T, GEOM>(c, c->stream) : open_second<T, GEOM>(c, c->stream);
+        if (ma.ntiles_hbm) HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
+      }
       ev_end(c, ev, c->stream, grp);
       return;
     }
@@ -305,32 +323,21 @@ struct Launch {
     // launches
     if (two_pass) fork(c);
     auto ev = ev_begin(c, c->stream);
+    const dim3 g((unsigned)ma.ntiles_closed);
     if (ma.small)
-      hipLaunchKernelGGL((k_mixed_state<DIM, INF, T, LDS_SMALL>), dim3(ma.ntiles_closed), dim3(T), 0, c->stream,
-                         c->ds, ma);
+      hipLaunchKernelGGL((k_mixed_state<DIM, GEOM, T, LDS_SMALL>), g, dim3(T), 0, c->stream, c->ds, ma);
+    else if (ma.mid && T > 512)
+      hipLaunchKernelGGL((k_mixed_state<DIM, GEOM, 512, LDS_MID>), g, dim3(512), 0, c->stream, c->ds, ma);
     else
-      hipLaunchKernelGGL((k_mixed_state<DIM, INF, T>), dim3(ma.ntiles_closed), dim3(T), 0, c->stream, c->ds, ma);
+      hipLaunchKernelGGL((k_mixed_state<DIM, GEOM, T>), g, dim3(T), 0, c->stream, c->ds, ma);
     ev_end(c, ev, c->stream, grp);
     if (two_pass) {
       auto es = ev_begin(c, c->side);
       mixed_umax(c, c->side);
-      if (ma.ntiles_lds && ma.small)
-        hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, true, T, LDS_SMALL>), dim3(ma.ntiles_lds), dim3(T), 0,
-                           c->side, c->ds, ma);
-      else if (ma.ntiles_lds)
-        hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, true, T>), dim3(ma.ntiles_lds), dim3(T), 0, c->side, c->ds,
-                           ma);
-      if (ma.ntiles_hbm)
-        hipLaunchKernelGGL((k_mixed_dilation<DIM, INF, false, T>), dim3(ma.ntiles_hbm), dim3(T), 0, c->side,
-                           c->ds, ma);
-      if (ma.ntiles_lds && ma.small)
-        hipLaunchKernelGGL((k_mixed_force<DIM, INF, true, T, LDS_SMALL>), dim3(ma.ntiles_lds), dim3(T), 0, c->side,
-                           c->ds, ma);
-      else if (ma.ntiles_lds)
-        hipLaunchKernelGGL((k_mixed_force<DIM, INF, true, T>), dim3(ma.ntiles_lds), dim3(T), 0, c->side, c->ds, ma);
-      if (ma.ntiles_hbm)
-        hipLaunchKernelGGL((k_mixed_force<DIM, INF, false, T>), dim3(ma.ntiles_hbm), dim3(T), 0, c->side, c->ds,
-                           ma);
+      open_first<T, GEOM>(c, c->side);
+      hbm_first(c, c->side);
+      open_second<T, GEOM>(c, c->side);
+      hbm_second(c, c->side);
       ev_end(c, es, c->side, grp);
       HIPCHK(hipEventRecord(c->ev_join, c->side));
       HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
@@ -347,10 +354,11 @@ struct Launch {
       if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(nb), dim3(TPB), 0, st, c->ds);
       if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(nb), dim3(TPB), 0, st, c->ds);
       // timed inside: both state-based passes (dilation and force), all tiles
+      const bool geom = c->mixed.geom != 0;
       if (c->mixed_tpb == 256)
-        mixed_state<INF, 256>(c);
+        geom ? mixed_state<256, true>(c) : mixed_state<256, false>(c);
       else
-        mixed_state<INF, 1024>(c);
+        geom ? mixed_state<1024, true>(c) : mixed_state<1024, false>(c);
       return;
     }
     const unsigned pb = (unsigned)c->pd_tpb, pnb = blocks(c->N, c->pd_tpb);
@@ -735,6 +743,106 @@ void build_rnp_tiles(pdem_ctx* c) {
   c->rnp_tile = true;
 }
 
+// Lists of the mixed tiles (DevTile).  Tiles with equal lists (the copies of
+// one mesh) share one: tiles are grouped by a hash of their degrees and
+// entries, the first of a group gives its list, and every tile's own list is
+// compared with the one it is given; a tile that differs gets its own.
+void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
+  const size_t nt = tiles.size();
+  if (nt == 0) return;
+  DS& s = c->ds;
+  HIPCHK(hipStreamSynchronize(c->stream));
+  auto put_tiles = [&] {
+    HIPCHK(hipMemcpy(c->d_tiles, tiles.data(), nt * sizeof(DevTile), hipMemcpyHostToDevice));
+  };
+  put_tiles();
+  std::vector<unsigned long long> hash(nt);
+  std::vector<int> diff(nt, 0), which;
+  unsigned long long* d_hash = c->dalloc<unsigned long long>(nt, false);
+  int* d_int = c->dalloc<int>(nt, false);
+  const dim3 gt((unsigned)nt), tb(256);
+  hipLaunchKernelGGL(k_list_hash, gt, tb, 0, c->stream, s, (const DevTile*)c->d_tiles, d_hash);
+  check_launch(c);
+  HIPCHK(hipMemcpyAsync(hash.data(), d_hash, nt * 8, hipMemcpyDeviceToHost, c->stream));
+  HIPCHK(hipStreamSynchronize(c->stream));
+  for (int round = 0; round < 2; round++) {
+    std::map<std::array<int64_t, 6>, size_t> first;
+    std::vector<uint32_t> lnode;
+    std::vector<int> lslice, order;
+    which.clear();
+    int64_t data = 0, lds_data = 0;  // entries, of all lists and of the LDS tiles'
+    for (size_t k = 0; k < nt; k++) {
+      DevTile& t = tiles[k];
+      const int n = t.te - t.ts, gs = (int)c->hp[t.pid].glob_start;
+      const auto at = first.emplace(
+          std::array<int64_t, 6>{(int64_t)hash[k], n, t.we - t.ws, t.lds ? t.ts - t.ws : t.ts - gs, t.lds ? 1 : 0,
+                                 diff[k] ? (int64_t)k : -1},
+          k);
+      if (!at.second) {
+        const DevTile& o = tiles[at.first->second];
+        t.node = o.node;
+        t.slice = o.slice;
+        t.data = o.data;
+        continue;
+      }
+      which.push_back((int)k);
+      t.node = (int)lnode.size();
+      t.slice = (int)lslice.size();
+      t.data = data;
+      // slots: nodes by their count of half blocks (most first), then by id
+      const int* deg = c->h_deg.data() + t.ts;
+      order.resize(n);
+      for (int q = 0; q < n; q++) order[q] = q;
+      std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+        return (deg[a] + KB / 2 - 1) / (KB / 2) > (deg[b] + KB / 2 - 1) / (KB / 2);
+      });
+      int64_t len = 0;
+      for (int q = 0; q < n; q += WAVE) {
+        lslice.push_back((int)len);
+        int w = 0;
+        for (int l = q; l < std::min(n, q + WAVE); l++) w = std::max(w, deg[order[l]]);
+        if (w > 0xffff) throw HipError{"mixed precision needs nodes of at most 65535 neighbors"};
+        len += (int64_t)((w + KB - 1) / KB) * KB * WAVE;
+      }
+      data += len;
+      if (t.lds) lds_data += len;
+      for (int q = 0; q < n; q++) lnode.push_back((uint32_t)order[q] | ((uint32_t)deg[order[q]] << 16));
+    }
+    c->grow(c->d_col16, c->col16_cap, (size_t)data + 8);
+    c->grow(c->d_wgt, c->wgt_cap, (size_t)data + 8);
+    c->grow(c->d_lnode, c->lnode_cap, lnode.size());
+    c->grow(c->d_lslice, c->lslice_cap, lslice.size());
+    HIPCHK(hipMemcpy(c->d_lnode, lnode.data(), lnode.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpy(c->d_lslice, lslice.data(), lslice.size() * sizeof(int), hipMemcpyHostToDevice));
+    put_tiles();
+    HIPCHK(hipMemcpy(d_int, which.data(), which.size() * sizeof(int), hipMemcpyHostToDevice));
+    c->mixed.lnode = c->d_lnode;
+    c->mixed.lslice = c->d_lslice;
+    c->mixed.col16 = c->d_col16;
+    c->mixed.wgt = c->d_wgt;
+    c->mixed.geom = lds_data > GEOM_MIN_ENTRIES && s.inf_type != 2 ? 1 : 0;
+    const dim3 gw((unsigned)which.size());
+    dispatch(
+        c,
+        [&] { hipLaunchKernelGGL(k_list_fill<2>, gw, tb, 0, c->stream, s, c->mixed, (const int*)d_int, c->d_col16, c->d_wgt); },
+        [&] { hipLaunchKernelGGL(k_list_fill<3>, gw, tb, 0, c->stream, s, c->mixed, (const int*)d_int, c->d_col16, c->d_wgt); });
+    check_launch(c);
+    if (round == 1 || which.size() == nt) break;
+    HIPCHK(hipStreamSynchronize(c->stream));
+    HIPCHK(hipMemcpy(d_int, diff.data(), nt * sizeof(int), hipMemcpyHostToDevice));
+    dispatch(
+        c, [&] { hipLaunchKernelGGL(k_list_check<2>, gt, tb, 0, c->stream, s, c->mixed, d_int); },
+        [&] { hipLaunchKernelGGL(k_list_check<3>, gt, tb, 0, c->stream, s, c->mixed, d_int); });
+    check_launch(c);
+    HIPCHK(hipMemcpyAsync(diff.data(), d_int, nt * sizeof(int), hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(hipStreamSynchronize(c->stream));
+    if (std::find(diff.begin(), diff.end(), 1) == diff.end()) break;
+  }
+  HIPCHK(hipStreamSynchronize(c->stream));
+  c->dfree(d_hash);
+  c->dfree(d_int);
+}
+
 // Tiles of the mixed kernels: for every state-based particle, the largest
 // tile size (power of two, 64..tile_max) whose neighbor windows all fit in
 // LDS, else tiles of tile_max nodes that gather from HBM; LDS tiles first.
@@ -776,36 +884,6 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
       tiles.push_back(DevTile{(int)ts, (int)te, ws, we, p, closed ? 2 : lds ? 1 : 0});
     }
   }
-  // thread slots: inside every tile, nodes by 8-bond block count (most
-  // first), then by id; the 16-bit id lists follow the slot order
-  const int64_t N = c->ds.N;
-  std::vector<int> slot(N);
-  for (int64_t q = 0; q < N; q++) slot[q] = (int)q;
-  for (const auto& t : tiles)
-    std::stable_sort(slot.begin() + t.ts, slot.begin() + t.te, [&](int a, int b) {
-      return (c->h_deg[a] + KB - 1) / KB > (c->h_deg[b] + KB - 1) / KB;
-    });
-  std::vector<int64_t> sp16(c->nslices + 1, 0);
-  for (int64_t sl = 0; sl < c->nslices; sl++) {
-    int w = 0;
-    for (int64_t q = sl * WAVE; q < std::min<int64_t>(N, (sl + 1) * WAVE); q++) w = std::max(w, c->h_deg[slot[q]]);
-    sp16[sl + 1] = sp16[sl] + (int64_t)((w + KB - 1) / KB) * KB * WAVE;
-  }
-  const size_t need = (size_t)sp16[c->nslices] + 8;
-  HIPCHK(hipStreamSynchronize(c->stream));
-  if (need > c->col16_cap) {
-    if (c->d_col16) c->dfree(c->d_col16);
-    c->d_col16 = c->dalloc<uint16_t>(need);
-    c->col16_cap = need;
-  }
-  HIPCHK(hipMemcpy(c->d_slot, slot.data(), N * sizeof(int), hipMemcpyHostToDevice));
-  HIPCHK(hipMemcpy(c->d_sp16, sp16.data(), sp16.size() * sizeof(int64_t), hipMemcpyHostToDevice));
-  hipLaunchKernelGGL(k_col16, dim3(blocks(N)), dim3(TPB), 0, c->stream, c->ds, c->d_col16, c->d_sp16,
-                     (const int*)c->d_slot);
-  check_launch(c);
-  c->mixed.slot = c->d_slot;
-  c->mixed.col16 = c->d_col16;
-  c->mixed.sptr16 = c->d_sp16;
   // closed tiles (fused kernel), then open LDS tiles, then HBM tiles
   std::stable_sort(tiles.begin(), tiles.end(), [](const DevTile& a, const DevTile& b) { return a.lds > b.lds; });
   if (tiles.size() > c->d_tiles_cap) throw HipError{"tile buffer too small"};
@@ -840,11 +918,12 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
   for (auto& t : tiles)
     if (t.lds) maxw = std::max(maxw, t.we - t.ws);
   c->mixed.small = maxw <= LDS_SMALL ? 1 : 0;
+  c->mixed.mid = maxw <= LDS_MID ? 1 : 0;
   c->mixed.ntiles_hbm = c->ntiles_global;
+  c->mixed.hbm_split = std::max(1, (int)(tile_max * HBM_LPN / HBM_TPB));
   c->tile_nodes = (int)tile_max;
-  if (!tiles.empty())
-    HIPCHK(hipMemcpy(c->d_tiles, tiles.data(), tiles.size() * sizeof(DevTile), hipMemcpyHostToDevice));
   c->mixed.tiles = c->d_tiles;
+  build_lists(c, tiles);
 }
 
 void build(pdem_ctx* c, const pdem_desc* d) {
@@ -1045,8 +1124,6 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     HIPCHK(hipStreamCreateWithFlags(&c->side, hipStreamNonBlocking));
     HIPCHK(hipEventCreateWithFlags(&c->ev_fork, hipEventDisableTiming));
     HIPCHK(hipEventCreateWithFlags(&c->ev_join, hipEventDisableTiming));
-    c->d_slot = c->dalloc<int>(N, false);
-    c->d_sp16 = c->dalloc<int64_t>(c->nslices + 1, false);
     int* dlo = c->dalloc<int>(N);
     int* dhi = c->dalloc<int>(N);
     hipLaunchKernelGGL(k_nbr_range, dim3(blocks(N)), dim3(TPB), 0, c->stream, s, dlo, dhi);
@@ -1063,7 +1140,11 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     c->d_tiles = c->dalloc<DevTile>(maxt);
     c->d_tiles_cap = maxt;
     build_tiles(c, TILE_NODES);
-    c->mixed.fa = c->dalloc<float>(N);
+    // windows of at most LDS_SMALL nodes: eight workgroups of 256 threads fit
+    // a CU, while most threads of larger workgroups would find no node
+    // (512-instance ensemble, particles of 127 to 367 nodes: 0.71 ms per step
+    // with 1024 threads, 0.49 ms with 256)
+    if (c->mixed.small) c->mixed_tpb = 256;
     c->mixed.fb = c->dalloc<float>(N);
   }
 
@@ -1245,6 +1326,12 @@ void build(pdem_ctx* c, const pdem_desc* d) {
       [&] { hipLaunchKernelGGL(k_mx<3>, dim3(blocks(N)), dim3(TPB), 0, c->stream, s); });
   // nodes that never search keep an empty candidate list
   check_launch(c);
+  if (c->precision == PDEM_PREC_MIXED && c->state_any) {
+    float* fa = c->dalloc<float>(N);
+    hipLaunchKernelGGL(k_mixed_alpha, dim3(blocks(N)), dim3(TPB), 0, c->stream, s, fa);
+    check_launch(c);
+    c->mixed.fa = fa;
+  }
   if (c->multi) {
     Ctrl h2 = h;
     h2.interval = d->neigh_update_interval;

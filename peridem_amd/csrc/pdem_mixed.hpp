@@ -7,24 +7,35 @@
 // Work unit: a tile = up to TILE_NODES consecutive nodes of one particle.
 // Horizons never cross particles, so a tile's neighbors lie in a window of
 // node ids [ws, we) inside its particle.  LDS tiles (the window fits) stage
-// the window once per workgroup (48 B per node: a float4 of the FP32
-// position offset from the particle's first reference node (independent of
-// the tile shape) and the volume, the FP64 displacement as a double2 and a
-// double, a float2 of the dilation terms) and every bond reads LDS; the remaining
+// the window once per workgroup (three records of 16 bytes per node, see
+// Win) and every bond reads LDS; the remaining
 // tiles (particles whose numbering spreads neighbors over more ids than the
 // window holds) gather from HBM through the caches: a separate
 // instantiation, launched on a second stream beside the LDS tiles.
 //
-// Neighbor ids are 16-bit offsets from the particle's first node, stored in
-// blocks of KB = 8 per lane: one 16-byte load yields a lane's next 8 ids and
-// the block loop is unrolled so each id is a compile-time lane of the block.
+// Neighbor ids are 16-bit, stored in blocks of KB = 8 per lane: one 16-byte
+// load yields a lane's next 8 ids and the block loop is unrolled so each id is
+// a compile-time lane of the block.  Beside each id lies the bond's constant
+// weight (its reference geometry: r J(r) V_j^c), so the loops evaluate only
+// what moves.
+//
+// (Models of many different meshes evaluate the weights instead, see
+// GEOM_MIN_ENTRIES.)
+//
+// Lists are shared: the particles of a model are mostly scaled and turned
+// copies of a few meshes, whose tiles then have the same relative ids and,
+// up to the particle's scale h V, the same weights.  Set-up finds such tiles
+// (by hash, then by comparing every entry) and stores one list for all of
+// them, which stays in L2: on the packing of 2000 spheres the lists of 1.4e8
+// bonds (0.9 GB) shrink to a few of 0.4 MB.  A tile whose list matches no
+// other keeps its own.
 //
 // Threads take nodes in slot order: inside every tile the nodes are ordered
-// by their number of 8-bond blocks (most first, node id second), so the 64
-// lanes of a wavefront run lists of about the same length (a wavefront runs
-// as long as its longest list; surface nodes have far fewer bonds than
-// interior ones).  The 16-bit id lists are laid out by slot; node data,
-// bond bits and results stay indexed by node.
+// by their number of 4-bond half blocks (most first, node id second), so the
+// 64 lanes of a wavefront run lists of about the same length (a wavefront
+// runs as long as its longest list; surface nodes have far fewer bonds than
+// interior ones).  The lists are laid out by slot; node data, bond bits and
+// results stay indexed by node.
 //
 // FMA contraction is allowed inside these kernels only (the FP64 parity
 // kernels are built without it).
@@ -33,6 +44,8 @@
 //   |xi + eta| - |xi| = (2 xi.eta + eta.eta) / (|xi + eta| + |xi|)
 // so FP32 keeps ~1e-7 relative accuracy at small strains.
 #pragma once
+#include <type_traits>
+
 #include "pdem_kernels.hpp"
 
 namespace pdem {
@@ -43,8 +56,18 @@ constexpr int LDS_NODES = 1280;   // window of up to 1280 nodes, ~61 KB of LDS p
 // uses the small instantiation (~19 KB of LDS per workgroup, so small particles
 // do not hold LDS sized for the largest window and more workgroups fit a CU).
 constexpr int LDS_SMALL = 384;
-constexpr int MIXED_TPB = 1024;   // default workgroup size (the autotuner may pick 256)
+// Windows of up to LDS_MID nodes leave room for three workgroups on a CU:
+// there the fused kernel runs 512 threads where 1024 are asked for, two nodes
+// a thread (24 wavefronts and up to 85 VGPRs instead of 32 and 64, no spills;
+// 2000 spheres of 1021 nodes: 0.541 to 0.516 ms per step).
+constexpr int LDS_MID = 1120;
 constexpr int KB = 8;             // neighbor ids per 16-byte block
+// HBM tiles: workgroup size and lanes per node.  They are few (a meshed wall)
+// and wait on gathers, so a node's list is dealt to 8 lanes and a tile to
+// several workgroups (top wall of the packing, 17 tiles: 273 us for both
+// passes with a lane per node and a workgroup per tile, 114 us now, beside
+// the fused kernel's 325 us).
+constexpr int HBM_TPB = 256, HBM_LPN = 8;
 // waves per SIMD the bond kernels are compiled for (at most 64 VGPRs): two
 // 1024-thread workgroups per CU, so one stages its window while the other computes
 constexpr int MIXED_WAVES_PER_SIMD = 8;
@@ -54,19 +77,34 @@ struct DevTile {
   int ws, we;     // neighbor window [ws, we)
   int pid;
   int lds;        // window staged in LDS; 2: also closed (the tile is its whole particle)
+  // the tile's list: thread slot q runs node ts + (lnode[node + q] & 0xffff)
+  // with lnode[node + q] >> 16 bonds, named by col16 from element
+  // data + lslice[slice + q / 64] + (q % 64) * KB on: entry k at
+  // (k / KB) * 64 * KB + k % KB beyond it.  An entry is the byte offset
+  // 16 (j - ws) of the neighbor's LDS records (LDS tiles, padded to whole
+  // blocks with 16 (we - ws)) or j - glob_start (HBM tiles, padded with 0).
+  // The weights 2 r J(r) V_j^c / particle_scale (0 in the padding) lie in
+  // half blocks: wgt[data + lslice + (k / 4) * 64 * 4 + (q % 64) * 4 + k % 4].
+  int node, slice;
+  int64_t data;
 };
 
 struct MixedArgs {
   const DevTile* tiles;   // closed LDS tiles, then open LDS tiles, then HBM tiles
   int ntiles_closed, ntiles_lds, ntiles_hbm;
+  int hbm_split;          // workgroups per HBM tile
   int small;              // every LDS window holds at most LDS_SMALL nodes
-  // thread slot q runs node slot[q]; its k-th neighbor id is
-  // col16[sptr16[q / 64] + (k / KB) * 64 * KB + (q % 64) * KB + k % KB]
-  const int* slot;
+  int mid;                // every LDS window holds at most LDS_MID nodes
+  // the lists (see DevTile)
+  const uint32_t* lnode;
+  const int* lslice;
   const uint16_t* col16;
-  const int64_t* sptr16;
-  float* fa;              // per node alpha = 15 G / m           (force pass)
-  float* fb;              // per node theta ((3K/m) - alpha / 3)  (force pass)
+  const float* wgt;
+  // LDS tiles evaluate the weights from the reference positions instead of
+  // reading them (lists too many to stay in cache)
+  int geom;
+  const float* fa;        // per node 2 alpha particle_scale, alpha = 15 G / m (constant, from set-up)
+  float* fb;              // per node b particle_scale, b = theta ((3K/m) - alpha / 3), of the open tiles
   // particles with open LDS tiles: max |u - u(first node)| over the particle
   // (rounded up to float), for the fixed-point step of their windows
   const int* open_pids;
@@ -74,6 +112,35 @@ struct MixedArgs {
   float* pumax;           // [np]
 };
 
+// The bond weights are read from the lists while the lists of the LDS tiles
+// hold at most this many entries (6 bytes each; an XCD's L2 holds 4 MB) and
+// evaluated from the reference positions beyond it, where their lists would
+// come from HBM in both passes (constant and linear influence functions; the
+// Gaussian one costs an exponential, so its weights are always read).
+// Measured with the particles' lists shared by 1 / 16 / 64 / 256 / no others,
+// step in us, read and evaluated: packing of 2000 spheres of 1021 nodes (76k
+// entries each) 478, 499, 521, 562, 645 against 486, 488, 490, 499, 518;
+// 512-instance ensemble of particles of up to 367 nodes (12k entries)
+// 493, 494, 504, 522, 574 against 510, 508, 513, 513, 520.
+constexpr int64_t GEOM_MIN_ENTRIES = 1 << 21;
+
+// the particle's scale h V(first node), by which the weights are divided: the
+// copies of one mesh then have equal weights, and weights times alpha or b
+// are of moderate size in any unit
+__device__ __forceinline__ double particle_scale(const DS& s, const DevParticle& p) {
+  const double c = p.h * s.vol[p.glob_start];
+  return c > 1e-300 ? c : 1.;
+}
+
+// keeps the work of one group of bonds apart from the next: without it the
+// compiler gathers the loads of a whole block first and runs out of registers
+__device__ __forceinline__ void pin(float (&f)[3], float& z) {
+  asm volatile("" : "+v"(f[0]), "+v"(f[1]), "+v"(f[2]), "+v"(z)::"memory");
+}
+// a value that is the same in every lane, kept in a scalar register
+__device__ __forceinline__ float uniform(float x) {
+  return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
+}
 __device__ __forceinline__ float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
 // hardware square root and reciprocal square root (1 ulp, no denormal
 // rescaling): bond lengths squared are far from the FP32 denormal range.
@@ -86,105 +153,98 @@ __device__ __forceinline__ float rsqf_hw(float x) { return __builtin_amdgcn_rsqf
 // threshold scaled once per particle.
 constexpr float REL_KEEP = 1.f - 1e-5f;
 
-// Influence function J(r) in FP32 (util::ConstInfluenceFn, LinearInfluenceFn,
-// GaussianInfluenceFn of influenceFn.h, argument r / delta) with its
-// constants folded once per particle: J = a, a + b r (b = p1 / delta) or
-// a exp(-b |xi|^2) (b = 1 / (p1 delta^2)).
-template <int INF>
-struct InfF {
-  float a, b;
-  __device__ InfF(const DS& s, float inv_delta)
-      : a((float)s.inf_p0),
-        b(INF == 1 ? (float)s.inf_p1 * inv_delta
-                   : INF == 2 ? inv_delta * inv_delta / (float)s.inf_p1 : 0.f) {}
-  __device__ __forceinline__ float operator()(float r, float xx) const {
-    if (INF == 0) return a;
-    if (INF == 1) return fmaf(b, r, a);
-    return a * __expf(-b * xx);
-  }
-};
-
+// entry t of a block; in LDS tiles the first entry's top bit is a mark of the block
+template <bool LDS>
 __device__ __forceinline__ int block_id(const uint4& b, int t) {
   const unsigned w = t < 2 ? b.x : t < 4 ? b.y : t < 6 ? b.z : b.w;
-  return (int)((w >> ((t & 1) * 16)) & 0xffffu);
+  return (int)((w >> ((t & 1) * 16)) & (LDS ? 0x7fffu : 0xffffu));
 }
 
-// Node data by particle-relative id jp (node gs + jp): the LDS window or HBM.
+// Node data of the bond loops: the LDS window (LDS) or HBM.
 //
-// LDS window records, per window node: a float4 of the FP32 position offset
-// from the particle's first reference node and the volume; an int4 of the
-// displacement relative to the window's first node in fixed point (three
-// int32 in units of a power-of-two step `us` chosen per window so that every
-// value stays below 2^29 in magnitude) and, in the force pass, the node's
-// b term; the node's alpha term as a float.  A bond's relative displacement
-// is the exact integer difference of two records, rounded once to FP32 and
-// scaled by us (exact): as accurate as rounding the FP64 difference to FP32,
-// plus a quantisation of 2^-29 of the window's largest relative
-// displacement.  32 bytes per bond in the dilation pass, 36 in the force pass.
-// HBM tiles read the FP64 displacements (us = 1).
+// A neighbor is named by the 16-bit entry of the id list: the byte offset of
+// its 16-byte LDS records (LDS tiles) or its id relative to the particle's
+// first node (HBM tiles).
+//
+// LDS records, 16 bytes each, per window node:
+//   lx  twice the FP32 position offset from the particle's first reference
+//       node, and the volume            (first pass; with GEOM both passes)
+//   lq  the displacement relative to the particle's first node in fixed
+//       point (three int32 in units of a power-of-two step `us` chosen per
+//       particle so that every value stays below 2^29 in magnitude), and the
+//       node's alpha term (MixedArgs::fa)                     (first pass)
+//   ly  the FP32 current position relative to that of the particle's first
+//       node, and the node's b term                           (second pass)
+// A bond's relative displacement is the exact integer difference of two lq
+// records, rounded once to FP32 and scaled by us (exact): as accurate as
+// rounding the FP64 difference to FP32, plus a quantisation of 2^-29 of the
+// particle's largest relative displacement.  HBM tiles read the FP64 arrays
+// (us = 1).
+//
+// The record after the window's last node (offset 16 (we - ws)) stands for
+// the list padding: a position so far off that its bond has no stretch, and
+// weight 0, so the entries that fill up a lane's last block add nothing and
+// the block loops need no test per bond.
+constexpr float PAD_POS = 1.0e18f;
+
 template <int DIM, bool LDS>
 struct Win {
-  const float4* lxv;
-  const int4* lq;
-  const float* la;
+  const char* lx;
+  const char* lq;
+  const char* ly;
   const DS* s;
   const MixedArgs* m;
   int gs;    // particle's first node
-  int off;   // gs - window start: LDS index of jp
+  int ws;    // window start
   float us;  // fixed-point step of the displacement records (1 for HBM tiles)
   double org[3];
-  __device__ __forceinline__ float4 xv(int jp) const {
-    if (LDS) return lxv[jp + off];
-    const int64_t j = gs + jp;
-    return make_float4((float)(s->xr[0][j] - org[0]), (float)(s->xr[1][j] - org[1]),
-                       DIM == 3 ? (float)(s->xr[2][j] - org[2]) : 0.f, (float)s->vol[j]);
+  __device__ __forceinline__ int entry(int i) const { return LDS ? (i - ws) * 16 : i - gs; }
+  __device__ __forceinline__ float4 x2(int e) const {
+    if (LDS) return *(const float4*)(lx + e);
+    const int64_t j = gs + e;
+    return make_float4(2.f * (float)(s->xr[0][j] - org[0]), 2.f * (float)(s->xr[1][j] - org[1]),
+                       DIM == 3 ? 2.f * (float)(s->xr[2][j] - org[2]) : 0.f, (float)s->vol[j]);
   }
   // the node's own displacement record (fixed point) or displacement (FP64)
   struct Own {
     int q[3];
     double u[3];
-    float b;  // the node's b term (force pass)
+    float a;
   };
-  __device__ __forceinline__ Own own(int jp) const {
+  __device__ __forceinline__ Own own(int e) const {
     Own o{};
     if (LDS) {
-      const int4 r = lq[jp + off];
+      const int4 r = *(const int4*)(lq + e);
       o.q[0] = r.x;
       o.q[1] = r.y;
       o.q[2] = r.z;
-      o.b = __int_as_float(r.w);
+      o.a = __int_as_float(r.w);
     } else {
-      for (int d = 0; d < DIM; d++) o.u[d] = s->u[d][gs + jp];
+      for (int d = 0; d < DIM; d++) o.u[d] = s->u[d][gs + e];
+      o.a = m->fa[gs + e];
     }
     return o;
   }
-  // relative displacement of neighbor jp in units of us (FP32); with B, bj
-  // gets the neighbor's b term from the same LDS record (the dilation pass
-  // reads only the displacement words: in the fused kernel it runs while b
-  // terms are being written)
-  template <bool B>
-  __device__ __forceinline__ void du(int jp, const Own& o, float* out, float& bj) const {
+  // relative displacement of neighbor e in units of us (FP32) and its alpha term
+  __device__ __forceinline__ void du(int e, const Own& o, float* out, float& aj) const {
     if (LDS) {
-      if (B) {
-        const int4 r = lq[jp + off];
-        out[0] = (float)(r.x - o.q[0]);
-        out[1] = (float)(r.y - o.q[1]);
-        if (DIM == 3) out[2] = (float)(r.z - o.q[2]);
-        bj = __int_as_float(r.w);
-      } else {
-        const int* r = (const int*)(lq + jp + off);
-        out[0] = (float)(r[0] - o.q[0]);
-        out[1] = (float)(r[1] - o.q[1]);
-        if (DIM == 3) out[2] = (float)(r[2] - o.q[2]);
-        bj = 0.f;
-      }
+      const int4 r = *(const int4*)(lq + e);
+      out[0] = (float)(r.x - o.q[0]);
+      out[1] = (float)(r.y - o.q[1]);
+      if (DIM == 3) out[2] = (float)(r.z - o.q[2]);
+      aj = __int_as_float(r.w);
     } else {
-      for (int d = 0; d < DIM; d++) out[d] = (float)(s->u[d][gs + jp] - o.u[d]);
-      bj = 0.f;
+      for (int d = 0; d < DIM; d++) out[d] = (float)(s->u[d][gs + e] - o.u[d]);
+      aj = m->fa[gs + e];
     }
   }
-  __device__ __forceinline__ float2 ab(int jp, float bj) const {
-    return LDS ? make_float2(la[jp + off], bj) : make_float2(m->fa[gs + jp], m->fb[gs + jp]);
+  // current position relative to the particle's first node, and the b term
+  __device__ __forceinline__ float4 yb(int e) const {
+    if (LDS) return *(const float4*)(ly + e);
+    const int64_t j = gs + e;
+    float y[3] = {0.f, 0.f, 0.f};
+    for (int d = 0; d < DIM; d++) y[d] = (float)((s->xr[d][j] - org[d]) + (s->u[d][j] - s->u[d][gs]));
+    return make_float4(y[0], y[1], y[2], m->fb[j]);
   }
 };
 
@@ -219,302 +279,523 @@ __global__ void __launch_bounds__(256) k_mixed_umax(DS s, MixedArgs m) {
   if (threadIdx.x == 0) m.pumax[pid] = mf;
 }
 
-// Stage a tile's window in LDS: positions and volumes, fixed-point
-// displacements relative to the particle's first node (the step us: the
-// smallest power of two with max |u - u_first| / us < 2^29 over the whole
-// particle, so that the records, and the results, do not depend on the tile
-// shape) and, for the force pass of an open tile, the dilation terms of
-// every window node.  A closed tile (the whole particle) takes the maximum
-// over its window; an open tile reads it from k_mixed_umax.  Returns us.
-template <int DIM, bool FORCE>
-__device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, const DevTile& t, float4* lxv,
-                                              int4* lq, float* la, const double* org, float* red) {
+// Stage a tile's window in LDS: the records that the pass (or, FIRST and
+// SECOND, both passes) reads.  The fixed-point step us is the smallest power
+// of two with max |u - u_first| / us < 2^29 over the whole particle, so that
+// the records, and the results, do not depend on the tile shape; a closed
+// tile (the whole particle) takes the maximum over its window, an open tile
+// reads it from k_mixed_umax.  The b terms of the fused kernel are written by
+// its first pass; those of an open tile come from the other kernel.
+// Returns us.
+template <int DIM, bool FIRST, bool SECOND, bool GEOM>
+__device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, const DevTile& t, float4* lx,
+                                              int4* lq, float4* ly, const double* org, float* red) {
   const int nw = t.we - t.ws;
   const int gs = (int)s.P[t.pid].glob_start;
   double u0[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) u0[d] = s.u[d][gs];
   for (int q = threadIdx.x; q < nw; q += blockDim.x) {
     const int j = t.ws + q;
-    lxv[q] = make_float4((float)(s.xr[0][j] - org[0]), (float)(s.xr[1][j] - org[1]),
-                         DIM == 3 ? (float)(s.xr[2][j] - org[2]) : 0.f, (float)s.vol[j]);
+    double xd[3] = {0., 0., 0.};
+    for (int d = 0; d < DIM; d++) xd[d] = s.xr[d][j] - org[d];
+    if (FIRST || GEOM) lx[q] = make_float4(2.f * (float)xd[0], 2.f * (float)xd[1], 2.f * (float)xd[2], (float)s.vol[j]);
+    if (SECOND) {
+      float y[3] = {0.f, 0.f, 0.f};
+      for (int d = 0; d < DIM; d++) y[d] = (float)(xd[d] + (s.u[d][j] - u0[d]));
+      ly[q] = make_float4(y[0], y[1], y[2], FIRST ? 0.f : m.fb[j]);
+    }
   }
-  const float mf = t.lds == 2 ? particle_umax<DIM>(s, gs, t.ws, t.we, red) : m.pumax[t.pid];
-  // us = 2^e with mf / us < 2^29 (e >= -126: a window at rest keeps all zeros)
-  int e = -126;
-  if (mf > 0.f) {
-    int ex;
-    frexpf(mf, &ex);  // mf < 2^ex
-    e = ex - 29 > -126 ? ex - 29 : -126;
+  float us = 1.f;
+  if (FIRST) {
+    const float mf = t.lds == 2 ? particle_umax<DIM>(s, gs, t.ws, t.we, red) : m.pumax[t.pid];
+    // us = 2^e with mf / us < 2^29 (e >= -126: a window at rest keeps all zeros)
+    int e = -126;
+    if (mf > 0.f) {
+      int ex;
+      frexpf(mf, &ex);  // mf < 2^ex
+      e = ex - 29 > -126 ? ex - 29 : -126;
+    }
+    us = ldexpf(1.f, e);
+    const double inv_us = ldexp(1., -e);
+    for (int q = threadIdx.x; q < nw; q += blockDim.x) {
+      const int j = t.ws + q;
+      int qq[3] = {0, 0, 0};
+      for (int d = 0; d < DIM; d++) qq[d] = (int)rint((s.u[d][j] - u0[d]) * inv_us);
+      lq[q] = make_int4(qq[0], qq[1], qq[2], __float_as_int(m.fa[j]));
+    }
   }
-  const float us = ldexpf(1.f, e);
-  const double inv_us = ldexp(1., -e);
-  for (int q = threadIdx.x; q < nw; q += blockDim.x) {
-    const int j = t.ws + q;
-    int qq[3] = {0, 0, 0};
-    for (int d = 0; d < DIM; d++) qq[d] = (int)rint((s.u[d][j] - u0[d]) * inv_us);
-    lq[q] = make_int4(qq[0], qq[1], qq[2], FORCE ? __float_as_int(m.fb[j]) : 0);
-    if (FORCE) la[q] = m.fa[j];
+  if (threadIdx.x == 0) {  // the padding's record
+    if (FIRST || GEOM) lx[nw] = make_float4(PAD_POS, PAD_POS, DIM == 3 ? PAD_POS : 0.f, 0.f);
+    if (FIRST) lq[nw] = make_int4(0, 0, 0, 0);
+    if (SECOND) ly[nw] = make_float4(PAD_POS, PAD_POS, DIM == 3 ? PAD_POS : 0.f, 0.f);
   }
   __syncthreads();
   return us;
 }
 
-// Per-particle constants of the mixed bond loops (FP32, folded once per
-// workgroup).
-template <int INF>
+// Per-particle constants of the mixed bond loops (those of every bond in
+// scalar registers)
 struct StateConsts {
-  float low_rel;   // r > low_rel: isGreater(r, horizon - h/2), the volume correction applies
-  float thr_rel;   // |S| > thr_rel: the bond breaks (isGreater(|S|, s0 + 1e-10))
-  float inv_h, up_h, inv_s0, Kn, Rc;
-  double K, G;
-  InfF<INF> J;
-  __device__ StateConsts(const DS& s, const DevParticle& p)
-      : J(s, rcpf((float)p.horizon)) {
-    const float horizon = (float)p.horizon, h = (float)p.h;
-    const float check_up = horizon + 0.5f * h, check_low = horizon - 0.5f * h;
-    low_rel = check_low / REL_KEEP;
-    thr_rel = (float)(p.mat[2] + 1.0e-10) / REL_KEEP;
-    inv_h = rcpf(h);
-    up_h = check_up * inv_h;
+  float thr4;      // |S| / 4 > thr4: the bond breaks (isGreater(|S|, s0 + 1e-10))
+  float inv_s0, Kn, Rc;
+  double K, G, scale;
+  // GEOM: J / scale = ja + jb r2 (constant and linear influence functions),
+  // volume correction up_h - r2 inv_h2 where r2 > low2
+  float ja, jb, low2, inv_h2, up_h;
+  __device__ StateConsts(const DS& s, const DevParticle& p) {
+    thr4 = uniform(0.25f * ((float)(p.mat[2] + 1.0e-10) / REL_KEEP));
     inv_s0 = (float)(1.0 / p.mat[2]);
     Kn = (float)p.Kn;
     Rc = (float)p.Rc;
     K = p.mat[0];
     G = p.mat[1];
+    scale = particle_scale(s, p);
+    const double inv = 1. / scale;
+    ja = uniform((float)(s.inf_p0 * inv));
+    jb = uniform(s.inf_type == 1 ? (float)(0.5 * s.inf_p1 / p.horizon * inv) : 0.f);
+    low2 = uniform(2.f * ((float)(p.horizon - 0.5 * p.h) / REL_KEEP));
+    inv_h2 = uniform((float)(0.5 / p.h));
+    up_h = uniform((float)((p.horizon + 0.5 * p.h) / p.h));
+  }
+  // GEOM: the weight 2 r J V^c / scale of a bond of length r2 / 2 whose
+  // neighbor has volume v.  The correction is 1 at the distance horizon - h/2
+  // from which it applies, so clamping it to [0, 1], which the multiply-add
+  // does for nothing, saves the compare and the select (EXACT) for every bond
+  // but those in the slack of the reference's compare (see slack_bond).
+  template <bool EXACT>
+  __device__ __forceinline__ float weight(float r2, float v) const {
+#pragma clang fp contract(fast)
+    const float c = up_h - r2 * inv_h2;
+    const float k = EXACT ? (r2 > low2 ? c : 1.f) : __builtin_amdgcn_fmed3f(c, 0.f, 1.f);
+    return r2 * ((ja + jb * r2) * (v * k));
   }
 };
 
-// Dilation of the node in thread slot q (demModel.cpp:610-679) in mixed
-// precision: breaks bonds, writes theta and the damage Z and returns the
-// node's force-pass terms (alpha, theta (3K/m - alpha/3)) as FP32.  The
-// damage Z_i (demModel.cpp:770-773) is the plain maximum of |S| / s0 over
-// the list, broken bonds included: |S| is the break test's value, taken
-// here rather than in the force pass (the reference's running compare with
-// a 1e-5 relative slack keeps a value at most 1e-5 below it; FP32 bond
-// arithmetic is the larger difference).
-template <int DIM, int INF, bool LDS>
-__device__ __forceinline__ float2 dilation_node(const DS& s, const MixedArgs& m, const Win<DIM, LDS>& w,
-                                                const StateConsts<INF>& c, int q, int& node) {
-#pragma clang fp contract(fast)
-  const int i = m.slot[q];
-  node = i;
-  const int ip = i - w.gs;
-  const uint4* cb = (const uint4*)(m.col16 + m.sptr16[q / WAVE] + (q % WAVE) * KB);
-  unsigned* bw = s.bits + s.bptr[i / WAVE] + i % WAVE;
-  const int n = s.deg[i];
-  const float4 xvi = w.xv(ip);
-  const float xi[3] = {xvi.x, xvi.y, xvi.z};
-  const auto own = w.own(ip);
-  const float us = w.us;
-  // |xi + eta|^2 - |xi|^2 = us^2 ee + 2 us xe in one multiply and one FMA
-  // (us is a power of two: the same value as us (us ee + 2 xe) while us^2
-  // is a normal float, i.e. for displacements above ~1e-14 of the unit)
-  const float us2 = us * us, us2x = 2.f * us;
-  double theta = 0.;
-  float Zs = 0.f;  // maximum of |S| over all bonds, broken ones included; Z = Zs / s0
-  unsigned word = 0, wnew = 0;
-  uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
-  for (int kb = 0; kb < n; kb += KB) {
-    if ((kb & 31) == 0) {
-      if (kb > 0 && wnew != word) bw[(int64_t)((kb >> 5) - 1) * WAVE] = wnew;
-      word = bw[(int64_t)(kb >> 5) * WAVE];
-      wnew = word;
-    }
-    const unsigned wblk = word >> (kb & 31);  // this block's 8 bond bits from bit 0
-    unsigned brk = 0;                         // bonds of the block that break now
-    const uint4 cur = blk;
-    if (kb + KB < n) blk = cb[(int64_t)(kb / KB + 1) * WAVE];
-    auto bond = [&](const int tt) {
-      if (kb + tt < n) {
-        const int jp = block_id(cur, tt);
-        const float4 xvj = w.xv(jp);
-        const float xj[3] = {xvj.x, xvj.y, xvj.z};
-        float dx[3], du[3], bj;
-        w.template du<false>(jp, own, du, bj);  // in units of us
-        for (int d = 0; d < DIM; d++) dx[d] = xj[d] - xi[d];
-        float volj = xvj.w;
-        float xx = dx[0] * dx[0], xe = dx[0] * du[0], ee = du[0] * du[0];
-        for (int d = 1; d < DIM; d++) {
-          xx += dx[d] * dx[d];
-          xe += dx[d] * du[d];
-          ee += du[d] * du[d];
-        }
-        const float t2 = fmaf(us2, ee, us2x * xe);  // |xi + eta|^2 - |xi|^2
-        const float inv_r = rsqf_hw(xx);
-        const float r = xx * inv_r;
-        const float cl = t2 * rcpf(sqrtf_hw(xx + t2) + r);
-        bool fs = ((wblk >> tt) & 1u) != 0u;
-        const float sa = fabsf(cl) * inv_r;  // |S|
-        // maximum of non-negative floats: their bit patterns order alike
-        Zs = __uint_as_float(max(__float_as_uint(Zs), __float_as_uint(sa)));
-        if (!fs && sa > c.thr_rel) {
-          fs = true;
-          brk |= 1u << tt;
-        }
-        if (!fs) {
-          if (r > c.low_rel) volj *= c.up_h - r * c.inv_h;
-          theta += (double)(r * cl * c.J(r, xx) * volj);
-        }
-      }
-    };
-#pragma unroll
-    for (int tt = 0; tt < KB; tt++) bond(tt);
-    wnew |= brk << (kb & 31);
-  }
-  if (n > 0 && wnew != word) bw[(int64_t)((n - 1) >> 5) * WAVE] = wnew;
-  const double mi = s.mx[i];
-  const double th = 3. * theta / mi;
-  s.theta[i] = th;
-  s.Z[i] = Zs * c.inv_s0;
-  const double alpha = 15. * c.G / mi;
-  return make_float2((float)alpha, (float)(th * ((3. * c.K / mi) - alpha / 3.)));
+// A bond whose length r is above low = horizon - h/2 by less than the slack
+// 1e-5 r of the reference's compare keeps its full volume, where the formula
+// gives up to 1e-5 low / h less.  Its 8-bond block is marked in the LDS tiles'
+// lists (SLACK_BLOCK in the block's first entry, whose value stays below it)
+// and takes the exact form.  (Within 2^-24 of low the two agree to rounding;
+// the upper end is taken with a margin.)
+constexpr unsigned SLACK_BLOCK = 0x8000u;
+__device__ __forceinline__ bool slack_bond(double r, double low) {
+  return r > low * (1. + 0x1p-24) && r < low * (1. + 1.2 * COMPARE_EPS);
 }
 
-// Force of the node in thread slot q (demModel.cpp:682-788,
-// PdState::getBondEF material.h:1415-1429) in mixed precision:
-// ef_i + ef_j = J (r (b_i + b_j) + cl (a_i + a_j)).
-template <int DIM, int INF, bool LDS>
-__device__ __forceinline__ void force_node(const DS& s, const MixedArgs& m, const Win<DIM, LDS>& w,
-                                           const StateConsts<INF>& c, int q) {
+// The two passes of a node (dilation, demModel.cpp:610-679; force, :682-788
+// with PdState::getBondEF, material.h:1415-1429) in mixed precision.
+//
+// With ef_i + ef_j = J (r (b_i + b_j) + c (alpha_i + alpha_j)), c = |y| - |xi|
+// the change of length, y = xi + eta and b = theta (3K/m - alpha / 3), only
+// the b terms of the force need the dilation of the neighbors; alpha is
+// constant.  So the first pass, which has the accurate change of length
+//   c = (2 xi.eta + eta.eta) / (|y| + |xi|)
+// at hand, also sums the alpha part of the force and the repulsion of broken
+// bonds (into f), and the second pass only adds
+//   sum_j r J V_j^c (b_i + b_j) y / |y|
+// from the bond's weight and one record of current positions per neighbor.
+//
+// The loops are bound by FP32 instruction issue and the latency of the list
+// reads.  Per bond in 3D they take 42 instructions in the first pass and 14 in
+// the second (of which 3 and 1 are half-rate transcendentals); with the
+// reference geometry evaluated in both passes and the alpha part in the second
+// they took 57 each.  Packing of 2000 spheres, both passes of a step: 409 us
+// before, 325 us now (kernel trace), 412 MB against 179 MB fetched.
+//
+// The loops take 4 bonds at a time without any test per bond: the lists are
+// padded to whole blocks (see Win), and a block with a bond that is broken, or
+// whose largest stretch says that one breaks now, is done again bond by bond.
+// Every sum is taken per block (theta in FP64, forces in FP32) and the blocks
+// are added in list order in FP64, so the results do not depend on how blocks
+// are dealt to lanes.
+
+// one bond of the first pass: doubled lengths, the quarter stretch and the
+// doubled current bond vector
+template <int DIM>
+struct Stretch {
+  float xx4, r2, inv_r2, l2, inv_l2, c2, y2[3];
+  // d2: twice the reference bond vector; q: relative displacement in units of us
+  __device__ __forceinline__ Stretch(const float* d2, const float* q, float us) {
 #pragma clang fp contract(fast)
-  const int i = m.slot[q];
-  const int ip = i - w.gs;
-  const uint4* cb = (const uint4*)(m.col16 + m.sptr16[q / WAVE] + (q % WAVE) * KB);
-  const unsigned* bw = s.bits + s.bptr[i / WAVE] + i % WAVE;
-  const int n = s.deg[i];
-  const float4 xvi = w.xv(ip);
-  const float xi[3] = {xvi.x, xvi.y, xvi.z};
-  const auto own = w.own(ip);
-  const float us = w.us;
-  const float2 abi = w.ab(ip, own.b);
-  const float ai = abi.x, bi = abi.y;
-  const float us2 = us * us, us2x = 2.f * us;
-  double force[3] = {0., 0., 0.};
-  unsigned word = 0;
-  uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
-  for (int kb = 0; kb < n; kb += KB) {
-    if ((kb & 31) == 0) word = bw[(int64_t)(kb >> 5) * WAVE];
-    const unsigned wblk = word >> (kb & 31);  // this block's 8 bond bits from bit 0
-    const uint4 cur = blk;
-    if (kb + KB < n) blk = cb[(int64_t)(kb / KB + 1) * WAVE];
-    float fblk[3] = {0.f, 0.f, 0.f};
-    auto bond = [&](const int tt) {
-      if (kb + tt < n) {
-        const int jp = block_id(cur, tt);
-        const float4 xvj = w.xv(jp);
-        const float xj[3] = {xvj.x, xvj.y, xvj.z};
-        float dx[3], du[3], y[3], bj;
-        w.template du<true>(jp, own, du, bj);  // in units of us
-        for (int d = 0; d < DIM; d++) {
-          dx[d] = xj[d] - xi[d];
-          y[d] = fmaf(us, du[d], dx[d]);
-        }
-        float volj = xvj.w;
-        float xx = dx[0] * dx[0], xe = dx[0] * du[0], ee = du[0] * du[0];
-        for (int d = 1; d < DIM; d++) {
-          xx += dx[d] * dx[d];
-          xe += dx[d] * du[d];
-          ee += du[d] * du[d];
-        }
-        const float t2 = fmaf(us2, ee, us2x * xe);  // |y|^2 - |xi|^2
-        const float yy = xx + t2;
-        const float inv_r = rsqf_hw(xx), inv_ly = rsqf_hw(yy);
-        const float r = xx * inv_r, ly = yy * inv_ly;
-        const float cl = t2 * rcpf(ly + r);
-        const bool fs = (wblk & (1u << tt)) != 0u;
-        float sf;
-        if (!fs) {
-          if (r > c.low_rel) volj *= c.up_h - r * c.inv_h;
-          const float Jr = c.J(r, xx);
-          const float2 abj = w.ab(jp, bj);
-          sf = Jr * (r * (bi + abj.y) + cl * (ai + abj.x)) * volj * inv_ly;
-        } else {
-          sf = c.Kn * volj * (ly - c.Rc) * inv_ly;
-          if (sf > 0.f) sf = 0.f;
-        }
-        for (int d = 0; d < DIM; d++) fblk[d] += sf * y[d];
-      }
-    };
-#pragma unroll
-    for (int tt = 0; tt < KB; tt++) bond(tt);
-    for (int d = 0; d < DIM; d++) force[d] += (double)fblk[d];
+    float t = q[0] * (d2[0] + us * q[0]);
+    xx4 = d2[0] * d2[0];
+    for (int d = 1; d < DIM; d++) {
+      xx4 += d2[d] * d2[d];
+      t += q[d] * (d2[d] + us * q[d]);
+    }
+    for (int d = 0; d < DIM; d++) y2[d] = d2[d] + 2.f * us * q[d];
+    t *= us;                      // |y|^2 - |xi|^2
+    const float yy4 = xx4 + 4.f * t;
+    inv_r2 = rsqf_hw(xx4);
+    inv_l2 = rsqf_hw(yy4);
+    r2 = xx4 * inv_r2;            // 2 |xi|
+    l2 = yy4 * inv_l2;            // 2 |y|
+    c2 = t * rcpf(l2 + r2);       // (|y| - |xi|) / 2
   }
-  for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
+  __device__ __forceinline__ float s4() const { return fabsf(c2) * inv_r2; }  // |S| / 4
+};
+
+// the sums of one 8-bond block in the first pass
+struct Block1 {
+  double theta;  // sum r c J V^c / particle_scale
+  float f[3];
+  float z;       // largest |S| / 4
+};
+
+// First pass of one block of a node's list: entries `cur`, weights at wg,
+// `left` bonds to the list's end, broken bits wblk; brk gets the bonds that
+// break now.
+template <int DIM, bool LDS, bool GEOM>
+__device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const StateConsts& c, const uint4& cur,
+                                              const float4* wg, int left, unsigned wblk, const float* xi,
+                                              const typename Win<DIM, LDS>::Own& own, float us, unsigned& brk) {
+#pragma clang fp contract(fast)
+  Block1 o{0., {0.f, 0.f, 0.f}, 0.f};
+  auto load = [&](int e, float* d2, float* du, float& vj, float& aj) {
+    const float4 xvj = w.x2(e);
+    const float xj[3] = {xvj.x, xvj.y, xvj.z};
+    w.du(e, own, du, aj);
+    for (int d = 0; d < DIM; d++) d2[d] = xj[d] - xi[d];
+    vj = xvj.w;
+  };
+  if (LDS) {
+    auto bond = [&](const int tt, const float wt) {
+      float d2[3], du[3], vj, aj;
+      load(block_id<LDS>(cur, tt), d2, du, vj, aj);
+      const Stretch<DIM> b(d2, du, us);
+      const float wj = GEOM ? c.weight<false>(b.r2, vj) : wt;
+      const float p = b.c2 * b.inv_r2;  // S / 4
+      o.z = fmaxf(o.z, fabsf(p));
+      o.theta += (double)(b.c2 * wj);
+      const float sf = p * wj * (own.a + aj) * b.inv_l2;
+      for (int d = 0; d < DIM; d++) o.f[d] += sf * b.y2[d];
+      if (tt % 2 == 1) pin(o.f, o.z);
+    };
+    const float4 wa = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[0];
+    const float4 wb = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[WAVE];
+    bond(0, wa.x);
+    bond(1, wa.y);
+    bond(2, wa.z);
+    bond(3, wa.w);
+    if (left > KB / 2) {
+      bond(4, wb.x);
+      bond(5, wb.y);
+      bond(6, wb.z);
+      bond(7, wb.w);
+    }
+    if (wblk == 0u && o.z <= c.thr4 && !(GEOM && (cur.x & SLACK_BLOCK))) return o;
+    o = Block1{0., {0.f, 0.f, 0.f}, o.z};
+  }
+  // bond by bond: a bond of the block is broken, breaks now or (GEOM) is in
+  // the slack, and every block of an HBM tile
+  const int nb = left < KB ? left : KB;
+#pragma unroll 1
+  for (int tt = 0; tt < nb; tt++) {
+    float d2[3], du[3], vj, aj;
+    load(block_id<LDS>(cur, tt), d2, du, vj, aj);
+    const Stretch<DIM> b(d2, du, us);
+    const float wj = GEOM ? c.weight<true>(b.r2, vj) : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4];
+    const float p = b.c2 * b.inv_r2;
+    o.z = fmaxf(o.z, fabsf(p));
+    bool fs = ((wblk >> tt) & 1u) != 0u;
+    if (!fs && fabsf(p) > c.thr4) {
+      fs = true;
+      brk |= 1u << tt;
+    }
+    float sf;
+    if (!fs) {
+      o.theta += (double)(b.c2 * wj);
+      sf = p * wj * (own.a + aj) * b.inv_l2;
+    } else {
+      // Kn V (|y| - Rc) y / |y| where it repels
+      sf = c.Kn * vj * (0.5f * b.l2 - c.Rc) * b.inv_l2;
+      if (sf > 0.f) sf = 0.f;
+    }
+    for (int d = 0; d < DIM; d++) o.f[d] += sf * b.y2[d];
+  }
+  return o;
+}
+
+// A node's list may be dealt to LPN neighboring lanes (LPN 1, 4 or 8: a
+// 32-bit bond word's four blocks are then taken at once): lane `sub` takes
+// blocks sub, sub + LPN, ...; the group's lanes then all add the blocks' sums
+// in list order, so every lane holds the node's sums.  (value of group lane k)
+template <int LPN, class T>
+__device__ __forceinline__ T group_lane(T v, int k) {
+  return LPN == 1 ? v : __shfl(v, k, LPN);
+}
+
+// First pass of the node in thread slot q: breaks bonds, writes theta, the
+// damage Z and the first part of the force, and returns the node's b term.
+// The damage Z_i (demModel.cpp:770-773) is the plain maximum of |S| / s0 over
+// the list, broken bonds included (the reference's running compare with a
+// 1e-5 relative slack keeps a value at most 1e-5 below it; FP32 bond
+// arithmetic is the larger difference).
+template <int DIM, bool LDS, bool GEOM, int LPN>
+__device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m, const DevTile& t,
+                                                 const Win<DIM, LDS>& w, const StateConsts& c, int q, int& node) {
+  const uint32_t ln = m.lnode[t.node + q];
+  const int i = t.ts + (int)(ln & 0xffffu), n = (int)(ln >> 16);
+  node = i;
+  const int sub = LPN == 1 ? 0 : (int)(threadIdx.x % LPN);
+  const int ei = w.entry(i);
+  const int64_t at = t.data + m.lslice[t.slice + q / WAVE];
+  const uint4* cb = (const uint4*)(m.col16 + at) + q % WAVE;
+  const float4* wb = (const float4*)(m.wgt + at) + q % WAVE;
+  unsigned* bw = s.bits + s.bptr[i / WAVE] + i % WAVE;
+  const float4 xvi = w.x2(ei);
+  const float xi[3] = {xvi.x, xvi.y, xvi.z};
+  const auto own = w.own(ei);
+  const float us = uniform(w.us);
+  double theta = 0., force[3] = {0., 0., 0.};
+  float Zs = 0.f;  // maximum of |S| / 4 over all bonds, broken ones included
+  auto add = [&](const Block1& o, int k) {
+    theta += group_lane<LPN>(o.theta, k);
+    Zs = fmaxf(Zs, group_lane<LPN>(o.z, k));
+    for (int d = 0; d < DIM; d++) force[d] += (double)group_lane<LPN>(o.f[d], k);
+  };
+  if (LPN == 1) {
+    unsigned word = 0, wnew = 0;
+    uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
+    for (int kb = 0; kb < n; kb += KB) {
+      if ((kb & 31) == 0) {
+        if (kb > 0 && wnew != word) bw[(int64_t)((kb >> 5) - 1) * WAVE] = wnew;
+        word = bw[(int64_t)(kb >> 5) * WAVE];
+        wnew = word;
+      }
+      const uint4 cur = blk;
+      if (kb + KB < n) blk = cb[(kb / KB + 1) * WAVE];
+      unsigned brk = 0;
+      const Block1 o = first_block<DIM, LDS, GEOM>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb,
+                                             (word >> (kb & 31)) & 0xffu, xi, own, us, brk);
+      wnew |= brk << (kb & 31);
+      add(o, 0);
+    }
+    if (n > 0 && wnew != word) bw[(int64_t)((n - 1) >> 5) * WAVE] = wnew;
+  } else {
+    for (int k0 = 0; k0 < n; k0 += KB * LPN) {
+      const int kb = k0 + KB * sub;
+      Block1 o{0., {0.f, 0.f, 0.f}, 0.f};
+      unsigned word = 0, brk = 0;
+      if (kb < n) {
+        word = bw[(int64_t)(kb >> 5) * WAVE];
+        o = first_block<DIM, LDS, GEOM>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
+                                  (word >> (kb & 31)) & 0xffu, xi, own, us, brk);
+      }
+      for (int k = 0; k < LPN; k++)
+        if (k0 + KB * k < n) add(o, k);
+      // the breaks of a word's four blocks joined, written by their first lane
+      unsigned b = brk << (kb & 31);
+      b |= (unsigned)__shfl_xor((int)b, 1, LPN);
+      b |= (unsigned)__shfl_xor((int)b, 2, LPN);
+      if (kb < n && b != 0u && (sub & 3) == 0) bw[(int64_t)(kb >> 5) * WAVE] = word | b;
+    }
+  }
+  const double mi = s.mx[i];
+  const double th = 3. * (c.scale * theta) / mi;
+  if (sub == 0) {
+    s.theta[i] = th;
+    s.Z[i] = 4.f * Zs * c.inv_s0;
+    for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
+  }
+  const double alpha = 15. * c.G / mi;
+  return (float)(c.scale * (th * ((3. * c.K / mi) - alpha / 3.)));
+}
+
+// Second pass of one block: sum of 2 r J V^c (b_i + b_j) y / |y| into f
+template <int DIM, bool LDS, bool GEOM>
+__device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const StateConsts& c, const uint4& cur,
+                                             const float4* wg, int left, unsigned wblk, const float* xi,
+                                             const float* yi, float bi, float (&f)[3]) {
+#pragma clang fp contract(fast)
+  auto bond = [&](const int tt, const float wt, auto exact) {
+    const int e = block_id<LDS>(cur, tt);
+    float wj = wt;
+    if (GEOM) {
+      const float4 xvj = w.x2(e);
+      const float xj[3] = {xvj.x, xvj.y, xvj.z};
+      float d2 = xj[0] - xi[0], xx4 = d2 * d2;
+      for (int d = 1; d < DIM; d++) {
+        d2 = xj[d] - xi[d];
+        xx4 += d2 * d2;
+      }
+      wj = c.weight<decltype(exact)::value>(xx4 * rsqf_hw(xx4), xvj.w);
+    }
+    const float4 ybj = w.yb(e);
+    const float yj[3] = {ybj.x, ybj.y, ybj.z};
+    float y[3];
+    for (int d = 0; d < DIM; d++) y[d] = yj[d] - yi[d];
+    float yy = y[0] * y[0];
+    for (int d = 1; d < DIM; d++) yy += y[d] * y[d];
+    const float sf = wj * (bi + ybj.w) * rsqf_hw(yy);
+    for (int d = 0; d < DIM; d++) f[d] += sf * y[d];
+  };
+  const std::false_type fast{};
+  if (LDS && wblk == 0u && !(GEOM && (cur.x & SLACK_BLOCK))) {
+    const float4 wa = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[0];
+    const float4 wb = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[WAVE];
+    bond(0, wa.x, fast);
+    bond(1, wa.y, fast);
+    if (GEOM) pin(f, f[0]);
+    bond(2, wa.z, fast);
+    bond(3, wa.w, fast);
+    pin(f, f[0]);
+    if (left > KB / 2) {
+      bond(4, wb.x, fast);
+      bond(5, wb.y, fast);
+      if (GEOM) pin(f, f[0]);
+      bond(6, wb.z, fast);
+      bond(7, wb.w, fast);
+    }
+    return;
+  }
+  const int nb = left < KB ? left : KB;
+#pragma unroll 1
+  for (int tt = 0; tt < nb; tt++)  // broken bonds: in the first pass
+    if (!((wblk >> tt) & 1u))
+      bond(tt, GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], std::true_type{});
+}
+
+// Second pass of the node in thread slot q: adds the b terms to f.
+template <int DIM, bool LDS, bool GEOM, int LPN>
+__device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m, const DevTile& t,
+                                                 const Win<DIM, LDS>& w, const StateConsts& c, int q) {
+  const uint32_t ln = m.lnode[t.node + q];
+  const int i = t.ts + (int)(ln & 0xffffu), n = (int)(ln >> 16);
+  const int sub = LPN == 1 ? 0 : (int)(threadIdx.x % LPN);
+  const int64_t at = t.data + m.lslice[t.slice + q / WAVE];
+  const uint4* cb = (const uint4*)(m.col16 + at) + q % WAVE;
+  const float4* wb = (const float4*)(m.wgt + at) + q % WAVE;
+  const unsigned* bw = s.bits + s.bptr[i / WAVE] + i % WAVE;
+  const float4 ybi = w.yb(w.entry(i)), xvi = GEOM ? w.x2(w.entry(i)) : ybi;
+  const float yi[3] = {ybi.x, ybi.y, ybi.z}, xi[3] = {xvi.x, xvi.y, xvi.z};
+  double force[3] = {0., 0., 0.};
+  for (int d = 0; d < DIM; d++) force[d] = s.f[d][i];
+  if (LPN == 1) {
+    unsigned word = 0;
+    uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
+    for (int kb = 0; kb < n; kb += KB) {
+      if ((kb & 31) == 0) word = bw[(int64_t)(kb >> 5) * WAVE];
+      const uint4 cur = blk;
+      if (kb + KB < n) blk = cb[(kb / KB + 1) * WAVE];
+      float fb[3] = {0.f, 0.f, 0.f};
+      second_block<DIM, LDS, GEOM>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb, (word >> (kb & 31)) & 0xffu, xi, yi,
+                                   ybi.w, fb);
+      for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)fb[d];
+    }
+  } else {
+    for (int k0 = 0; k0 < n; k0 += KB * LPN) {
+      const int kb = k0 + KB * sub;
+      float fb[3] = {0.f, 0.f, 0.f};
+      if (kb < n)
+        second_block<DIM, LDS, GEOM>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
+                                     (bw[(int64_t)(kb >> 5) * WAVE] >> (kb & 31)) & 0xffu, xi, yi, ybi.w, fb);
+      for (int k = 0; k < LPN; k++)
+        if (k0 + KB * k < n)
+          for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)group_lane<LPN>(fb[d], k);
+    }
+  }
+  if (sub == 0)
+    for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
 }
 
 // Tile ranges of MixedArgs::tiles: closed LDS tiles (whole particles, fused
-// kernel), open LDS tiles, HBM tiles.
-__device__ __forceinline__ const DevTile& tile_of(const MixedArgs& m, bool lds) {
-  return m.tiles[(lds ? m.ntiles_closed : m.ntiles_closed + m.ntiles_lds) + blockIdx.x];
+// kernel), open LDS tiles, HBM tiles.  An HBM tile is shared by hbm_split
+// workgroups of HBM_TPB threads (there is no window to stage).
+template <bool LDS>
+__device__ __forceinline__ const DevTile& tile_of(const MixedArgs& m) {
+  return m.tiles[LDS ? m.ntiles_closed + (int)blockIdx.x
+                     : m.ntiles_closed + m.ntiles_lds + (int)blockIdx.x / m.hbm_split];
+}
+// thread slot of the workgroup's round `it` over the tile's slots (LPN lanes per slot)
+template <bool LDS, int LPN>
+__device__ __forceinline__ int slot_of(const MixedArgs& m, int it) {
+  return ((LDS ? it : it * m.hbm_split + (int)blockIdx.x % m.hbm_split) * (int)blockDim.x + (int)threadIdx.x) / LPN;
+}
+template <bool LDS, int LPN>
+__device__ __forceinline__ int slot_rounds(const MixedArgs& m, const DevTile& t) {
+  const int per = (int)blockDim.x / LPN * (LDS ? 1 : m.hbm_split);
+  return (t.te - t.ts + per - 1) / per;
 }
 
-// LDS of the window records (LDS tiles) or a dummy (HBM tiles)
-#define PDEM_WINDOW_LDS(LDS_ON, NODES)                 \
-  __shared__ float4 lxv[(LDS_ON) ? (NODES) : 1];       \
-  __shared__ int4 lq[(LDS_ON) ? (NODES) : 1];          \
-  __shared__ float la[(LDS_ON) ? (NODES) : 1];         \
+// LDS of the window records, one more than the window for the list padding
+// (LDS tiles), or a dummy (HBM tiles)
+#define PDEM_WINDOW_LDS(LDS_ON, NODES, FIRST, SECOND, GEOM)    \
+  __shared__ float4 lx[(LDS_ON) && ((FIRST) || (GEOM)) ? (NODES) + 1 : 1]; \
+  __shared__ int4 lq[(LDS_ON) && (FIRST) ? (NODES) + 1 : 1];   \
+  __shared__ float4 ly[(LDS_ON) && (SECOND) ? (NODES) + 1 : 1]; \
   __shared__ float red[1024 / WAVE];
+#define PDEM_WINDOW(DIM, LDS_ON, t, gs) \
+  Win<DIM, LDS_ON> w{(const char*)lx, (const char*)lq, (const char*)ly, &s, &m, gs, t.ws, 1.f, {0., 0., 0.}}; \
+  for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
 
-// Dilation pass of the open tiles (tiles that do not hold a whole particle:
-// the force pass of a tile reads the dilation terms of nodes of other tiles).
-template <int DIM, int INF, bool LDS, int TPB, int NODES = LDS_NODES>
+// First pass of the open tiles (tiles that do not hold a whole particle:
+// the second pass of a tile reads the b terms of nodes of other tiles).
+template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = LDS ? 1 : HBM_LPN>
 __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_dilation(DS s, MixedArgs m) {
-  PDEM_WINDOW_LDS(LDS, NODES)
-  const DevTile t = tile_of(m, LDS);
+  PDEM_WINDOW_LDS(LDS, NODES, true, false, GEOM)
+  const DevTile t = tile_of<LDS>(m);
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
-  Win<DIM, LDS> w{lxv, lq, la, &s, &m, gs, gs - t.ws, 1.f, {0., 0., 0.}};
-  for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
-  if (LDS) w.us = stage_window<DIM, false>(s, m, t, lxv, lq, la, w.org, red);
-  const StateConsts<INF> c(s, p);
-  for (int q = t.ts + threadIdx.x; q < t.te; q += blockDim.x) {
+  PDEM_WINDOW(DIM, LDS, t, gs)
+  if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  const StateConsts c(s, p);
+  const int nr = slot_rounds<LDS, LPN>(m, t);
+  for (int it = 0; it < nr; it++) {
+    const int q = slot_of<LDS, LPN>(m, it);
+    if (q >= t.te - t.ts) continue;
     int i;
-    const float2 ab = dilation_node<DIM, INF, LDS>(s, m, w, c, q, i);
-    m.fa[i] = ab.x;
-    m.fb[i] = ab.y;
+    const float b = first_pass_node<DIM, LDS, GEOM, LPN>(s, m, t, w, c, q, i);
+    if (LPN == 1 || threadIdx.x % LPN == 0) m.fb[i] = b;
   }
 }
 
-// Force pass of the open tiles.
-template <int DIM, int INF, bool LDS, int TPB, int NODES = LDS_NODES>
+// Second pass of the open tiles.
+template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = LDS ? 1 : HBM_LPN>
 __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_force(DS s, MixedArgs m) {
-  PDEM_WINDOW_LDS(LDS, NODES)
-  const DevTile t = tile_of(m, LDS);
+  PDEM_WINDOW_LDS(LDS, NODES, false, true, GEOM)
+  const DevTile t = tile_of<LDS>(m);
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
-  Win<DIM, LDS> w{lxv, lq, la, &s, &m, gs, gs - t.ws, 1.f, {0., 0., 0.}};
-  for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
-  if (LDS) w.us = stage_window<DIM, true>(s, m, t, lxv, lq, la, w.org, red);
-  const StateConsts<INF> c(s, p);
-  for (int q = t.ts + threadIdx.x; q < t.te; q += blockDim.x) force_node<DIM, INF, LDS>(s, m, w, c, q);
+  PDEM_WINDOW(DIM, LDS, t, gs)
+  if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  const StateConsts c(s, p);
+  const int nr = slot_rounds<LDS, LPN>(m, t);
+  for (int it = 0; it < nr; it++) {
+    const int q = slot_of<LDS, LPN>(m, it);
+    if (q < t.te - t.ts) second_pass_node<DIM, LDS, GEOM, LPN>(s, m, t, w, c, q);
+  }
 }
 
-// Both passes (demModel.cpp:610-679 and :682-788) of a closed tile, a whole
-// particle, so that every neighbor of its nodes is one of its nodes, in one
-// workgroup: the window is staged in LDS once, the dilation pass leaves each
-// node's force-pass terms in its LDS record, and after a barrier the force
-// pass reads them there.  Nothing of the dilation pass goes through HBM but
-// theta.
-template <int DIM, int INF, int TPB, int NODES = LDS_NODES>
-__global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_state(DS s, MixedArgs m) {
-  PDEM_WINDOW_LDS(true, NODES)
+// Both passes of a closed tile, a whole particle, so that every neighbor of
+// its nodes is one of its nodes, in one workgroup: the window is staged in
+// LDS once, the first pass leaves each node's b term in its LDS record, and
+// after a barrier the second pass reads them there.
+template <int DIM, bool GEOM, int TPB, int NODES = LDS_NODES>
+__global__ void __launch_bounds__(TPB, TPB == 512 ? 6 : MIXED_WAVES_PER_SIMD) k_mixed_state(DS s, MixedArgs m) {
+  PDEM_WINDOW_LDS(true, NODES, true, true, GEOM)
   const DevTile t = m.tiles[blockIdx.x];
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
-  Win<DIM, true> w{lxv, lq, la, &s, &m, gs, gs - t.ws, 1.f, {0., 0., 0.}};
-  for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
-  w.us = stage_window<DIM, false>(s, m, t, lxv, lq, la, w.org, red);
-  const StateConsts<INF> c(s, p);
-  for (int q = t.ts + threadIdx.x; q < t.te; q += blockDim.x) {
+  PDEM_WINDOW(DIM, true, t, gs)
+  w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  const StateConsts c(s, p);
+  const int nr = slot_rounds<true, 1>(m, t);
+  for (int it = 0; it < nr; it++) {
+    const int q = slot_of<true, 1>(m, it);
+    if (q >= t.te - t.ts) continue;
     int i;
-    const float2 ab = dilation_node<DIM, INF, true>(s, m, w, c, q, i);
-    la[i - t.ws] = ab.x;
-    lq[i - t.ws].w = __float_as_int(ab.y);
+    const float b = first_pass_node<DIM, true, GEOM, 1>(s, m, t, w, c, q, i);
+    ly[i - t.ws].w = b;
   }
   __syncthreads();
-  for (int q = t.ts + threadIdx.x; q < t.te; q += blockDim.x) force_node<DIM, INF, true>(s, m, w, c, q);
+  for (int it = 0; it < nr; it++) {
+    const int q = slot_of<true, 1>(m, it);
+    if (q < t.te - t.ts) second_pass_node<DIM, true, GEOM, 1>(s, m, t, w, c, q);
+  }
 }
 
+#undef PDEM_WINDOW
 #undef PDEM_WINDOW_LDS
 
 // the force reset of nodes that take no PD force (a list built at set-up);
@@ -527,6 +808,119 @@ __global__ void k_zero_noforce(DS s) {
     const int64_t i = s.noforce_nodes[k];
     for (int d = 0; d < DIM; d++) s.f[d][i] = 0.;
   }
+}
+
+// Set-up of the lists (see DevTile).
+
+// weight 2 r J(r) V_j^c / particle_scale of a bond (materialUtil.cpp:21-73, m_x's terms)
+template <int DIM>
+__device__ __forceinline__ double bond_weight(const DS& s, const DevParticle& p, double inv_scale, int i, int j,
+                                              bool& slack) {
+  double dx[3];
+  for (int d = 0; d < DIM; d++) dx[d] = s.xr[d][j] - s.xr[d][i];
+  const double r = len3<DIM>(dx);
+  double v = s.vol[j];
+  slack |= slack_bond(r, p.horizon - 0.5 * p.h);
+  if (isGreater(r, p.horizon - 0.5 * p.h)) v *= (p.horizon + 0.5 * p.h - r) / p.h;
+  return 2. * r * infFn(s, r / p.horizon) * v * inv_scale;
+}
+__device__ __forceinline__ int list_entry(const DevTile& t, int gs, int j) {
+  return t.lds ? (j - t.ws) * 16 : j - gs;
+}
+__device__ __forceinline__ uint64_t list_mix(uint64_t x) {  // splitmix64's finaliser
+  x = (x ^ (x >> 30)) * 0xbf58476d1ce4e5b9ull;
+  x = (x ^ (x >> 27)) * 0x94d049bb133111ebull;
+  return x ^ (x >> 31);
+}
+
+// hash of a tile's lists: degrees and entries of its nodes; a workgroup per tile
+__global__ void __launch_bounds__(256) k_list_hash(DS s, const DevTile* tiles, unsigned long long* out) {
+  __shared__ unsigned long long red[256 / WAVE];
+  const DevTile t = tiles[blockIdx.x];
+  const int gs = (int)s.P[t.pid].glob_start;
+  unsigned long long h = 0;
+  for (int l = threadIdx.x; l < t.te - t.ts; l += blockDim.x) {
+    const int i = t.ts + l, n = s.deg[i];
+    const int* c = s.col + s.sptr[i / WAVE] + i % WAVE;
+    h += list_mix(((uint64_t)l << 34) + (uint64_t)n + 0x9e3779b97f4a7c15ull);
+    for (int k = 0; k < n; k++)
+      h += list_mix(((uint64_t)l << 34) ^ ((uint64_t)k << 17) ^ (uint64_t)list_entry(t, gs, c[(int64_t)k * WAVE]));
+  }
+  for (int o = WAVE / 2; o > 0; o >>= 1) h += __shfl_xor(h, o);
+  if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = h;
+  __syncthreads();
+  if (threadIdx.x == 0) out[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
+}
+
+// the lists of tiles[which[block]] from the PD neighbor lists
+template <int DIM>
+__global__ void __launch_bounds__(256) k_list_fill(DS s, MixedArgs m, const int* which, uint16_t* col16, float* wgt) {
+  const DevTile t = m.tiles[which[blockIdx.x]];
+  const DevParticle& p = s.P[t.pid];
+  const int gs = (int)p.glob_start;
+  const double inv_scale = 1. / particle_scale(s, p);
+  for (int q = threadIdx.x; q < t.te - t.ts; q += blockDim.x) {
+    const uint32_t ln = m.lnode[t.node + q];
+    const int i = t.ts + (int)(ln & 0xffffu), n = (int)(ln >> 16);
+    const int* c = s.col + s.sptr[i / WAVE] + i % WAVE;
+    const int64_t at = t.data + m.lslice[t.slice + q / WAVE];
+    for (int kb = 0; kb < n; kb += KB) {
+      uint16_t* id = col16 + at + (int64_t)kb * WAVE + (q % WAVE) * KB;
+      bool slack = false;
+      unsigned id0 = 0;
+      for (int k = kb; k < kb + KB; k++) {
+        const int j = k < n ? c[(int64_t)k * WAVE] : -1;
+        const unsigned e = k < n ? (unsigned)list_entry(t, gs, j) : t.lds ? (unsigned)(t.we - t.ws) * 16u : 0u;
+        if (k == kb) id0 = e;
+        id[k - kb] = (uint16_t)e;
+        wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] =
+            k < n ? (float)bond_weight<DIM>(s, p, inv_scale, i, j, slack) : 0.f;
+      }
+      if (slack && t.lds) id[0] = (uint16_t)(id0 | SLACK_BLOCK);
+    }
+  }
+}
+
+// whether the tiles' own lists equal the ones they are given (degrees and
+// entries the same, weights within an ulp): diff[tile] is set where not
+template <int DIM>
+__global__ void __launch_bounds__(256) k_list_check(DS s, MixedArgs m, int* diff) {
+  const DevTile t = m.tiles[blockIdx.x];
+  const DevParticle& p = s.P[t.pid];
+  const int gs = (int)p.glob_start;
+  const double inv_scale = 1. / particle_scale(s, p);
+  bool bad = false;
+  for (int q = threadIdx.x; q < t.te - t.ts; q += blockDim.x) {
+    const uint32_t ln = m.lnode[t.node + q];
+    const int i = t.ts + (int)(ln & 0xffffu), n = (int)(ln >> 16);
+    if (s.deg[i] != n) {
+      bad = true;
+      continue;
+    }
+    const int* c = s.col + s.sptr[i / WAVE] + i % WAVE;
+    const int64_t at = t.data + m.lslice[t.slice + q / WAVE];
+    const unsigned mask = t.lds ? SLACK_BLOCK - 1 : 0xffffu;
+    for (int kb = 0; kb < n; kb += KB) {
+      const uint16_t* id = m.col16 + at + (int64_t)kb * WAVE + (q % WAVE) * KB;
+      bool slack = false;
+      for (int k = kb; k < n && k < kb + KB; k++) {
+        const int j = c[(int64_t)k * WAVE];
+        const double w = bond_weight<DIM>(s, p, inv_scale, i, j, slack);
+        bad |= (id[k - kb] & mask) != (unsigned)list_entry(t, gs, j);
+        bad |= !(fabs((double)m.wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] - w) <= 0x1p-23 * fabs(w));
+      }
+      bad |= t.lds && ((id[0] & SLACK_BLOCK) != 0) != slack;
+    }
+  }
+  if (bad) diff[blockIdx.x] = 1;
+}
+
+// the nodes' constant alpha terms (set-up)
+__global__ void k_mixed_alpha(DS s, float* fa) {
+  const int64_t i = gid();
+  if (i >= s.N) return;
+  const DevParticle& p = s.P[s.ptid[i]];
+  fa[i] = (float)(2. * (15. * p.mat[1] / s.mx[i]) * particle_scale(s, p));
 }
 
 // copy of f of the nodes that take no PD force (save != 0: into buf, else
