@@ -21,22 +21,30 @@ namespace mlp {
 // Gradient of loss = (1/B) sum_rows sum_o tw[o] (y_o - t_o)^2 over a batch of
 // B rows.  Rows: sample index = rows in order (shuffle == 0, rows >= n
 // inactive) or drawn with replacement by a hash of (shuffle, row).
-// partial: per workgroup NPARAM gradient entries + 1 loss entry.
-__global__ void __launch_bounds__(256) k_mlp_grad(Net n, const float* X, const float* T, const float* tw,
-                                                  int64_t nsamp, int64_t batch, uint64_t shuffle,
-                                                  float inv_batch, float* partial) {
-  __shared__ short XT[NIN * ROWS_WG];
-  __shared__ short HT[3][NH * ROWS_WG];
-  __shared__ short DYT[NOP * ROWS_WG];
+// partial: per 64 rows NPARAM gradient entries + 1 loss entry.
+// Workgroups: blockIdx.x takes the 64 rows, blockIdx.y one of gridDim.y shares
+// of the weight-gradient blocks; every share repeats the forward and backward
+// passes, which wait on their chains of loads and products, not on the matrix
+// cores.  At a batch of 1024 (16 times 64 rows) one workgroup each left 240
+// of 256 CUs idle.  With that, the weight copies in fragment order, the loads
+// of a layer in flight together (unrolled loops) and the padded LDS rows the
+// launch takes 18.7 us at a batch of 1024 (80 us before), a training iteration
+// 23.5 us (89 us); 32.5 us at 4096 (101 us).  Results are the same bit for bit.
+__global__ void __launch_bounds__(256, 1) k_mlp_grad(Net n, const float* X, const float* T, const float* tw,
+                                                     int64_t nsamp, int64_t batch, uint64_t shuffle,
+                                                     float inv_batch, float* partial) {
+  __shared__ __align__(16) short XT[NIN * ROWS_LD];
+  __shared__ __align__(16) short HT[3][NH * ROWS_LD];
+  __shared__ __align__(16) short DYT[NOP * ROWS_LD];
   __shared__ float lsum[4];
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, q = lane >> 4, j = lane & 15;
+  const int part = (int)blockIdx.y, parts = (int)gridDim.y;
   const int64_t brow = (int64_t)blockIdx.x * ROWS_WG + wave * 16 + j;
   const bool active = brow < batch;
   int64_t srow = 0;
   if (active) srow = shuffle ? (int64_t)(splitmix(shuffle * 0x100000001b3ull + (uint64_t)brow) % (uint64_t)nsamp) : brow;
-  float x16[NIN];
-  for (int f = 0; f < NIN; f++) x16[f] = active ? X[srow * NIN + f] : n.in_mean[f];
-  const s4 xb = input_frag(n, x16, lane);
+  const f4 x = *(const f4*)((active ? X + srow * NIN : n.in_mean) + 4 * q);
+  const s4 xb = input_frag(n, x, lane);
   s4 h1[8], h2[8], h3[8];
   const f4 y = forward(n, xb, h1, h2, h3, lane);
   // output gradient (lanes q == 0 hold the 4 outputs)
@@ -60,14 +68,15 @@ __global__ void __launch_bounds__(256) k_mlp_grad(Net n, const float* X, const f
   store_fm(DYT, &dy, 1, wave, lane);
   __syncthreads();
   float* g = partial + (size_t)blockIdx.x * (NPARAM + 1);
-  if (threadIdx.x == 0) g[NPARAM] = (lsum[0] + lsum[1] + lsum[2] + lsum[3]) * inv_batch;
-  weight_grad(HT[2], DYT, NH, NOP, NOUT, g + OW4, wave, lane);
-  bias_grad(DYT, NOUT, g + OB4);
+  if (threadIdx.x == 0 && part == 0) g[NPARAM] = (lsum[0] + lsum[1] + lsum[2] + lsum[3]) * inv_batch;
+  weight_grad(HT[2], DYT, NH, NOP, NOUT, g + OW4, wave, lane, part, parts);
+  if (part == 0) bias_grad(DYT, NOUT, g + OB4);
   // dz3 = mask(h3) * W4 dy
   s4 dz[8], dzn[8];
+#pragma unroll
   for (int ib = 0; ib < 8; ib++) {
     f4 acc = {0.f, 0.f, 0.f, 0.f};
-    acc = mfma(frag(n.w + BW4, NOP, ib * 16, 0, lane), dy, acc);
+    acc = mfma(wfrag(n.w + BW4, NOP, ib, 0, lane), dy, acc);
     s4 o;
     for (int r = 0; r < 4; r++) o[r] = bf16_f(h3[ib][r]) > 0.f ? bf16_rne(acc[r]) : (short)0;
     dz[ib] = o;
@@ -75,20 +84,20 @@ __global__ void __launch_bounds__(256) k_mlp_grad(Net n, const float* X, const f
   __syncthreads();  // H3 consumed: its LDS now holds dZ3
   store_fm(HT[2], dz, 8, wave, lane);
   __syncthreads();
-  weight_grad(HT[1], HT[2], NH, NH, NH, g + OW3, wave, lane);
-  bias_grad(HT[2], NH, g + OB3);
+  weight_grad(HT[1], HT[2], NH, NH, NH, g + OW3, wave, lane, part, parts);
+  if (part == 1 % parts) bias_grad(HT[2], NH, g + OB3);
   back_hidden(n, BW3, dz, h2, dzn, lane);
   __syncthreads();
   store_fm(HT[1], dzn, 8, wave, lane);
   __syncthreads();
-  weight_grad(HT[0], HT[1], NH, NH, NH, g + OW2, wave, lane);
-  bias_grad(HT[1], NH, g + OB2);
+  weight_grad(HT[0], HT[1], NH, NH, NH, g + OW2, wave, lane, part, parts);
+  if (part == 2 % parts) bias_grad(HT[1], NH, g + OB2);
   back_hidden(n, BW2, dzn, h1, dz, lane);
   __syncthreads();
   store_fm(HT[0], dz, 8, wave, lane);
   __syncthreads();
-  weight_grad(XT, HT[0], NIN, NH, NH, g + OW1, wave, lane);
-  bias_grad(HT[0], NH, g + OB1);
+  weight_grad(XT, HT[0], NIN, NH, NH, g + OW1, wave, lane, part, parts);
+  if (part == 3 % parts) bias_grad(HT[0], NH, g + OB1);
 }
 
 // bf16 copies of one master parameter
@@ -101,8 +110,8 @@ __device__ __forceinline__ void pack_one(int i, float w, short* wb, short* wtb) 
   else return;  // biases stay FP32
   const int a = k / nout, b = k % nout;
   const short h = bf16_rne(w);
-  wb[bw + a * nout_p + b] = h;
-  wtb[bw + b * nin + a] = h;
+  wb[bw + wpos(nout_p, a, b)] = h;
+  wtb[bw + wpos(nin, b, a)] = h;
 }
 
 __global__ void k_mlp_pack(const float* p, short* wb, short* wtb) {
@@ -116,7 +125,15 @@ __global__ void k_mlp_adam(float* p, float* m, float* v, short* wb, short* wtb, 
                            float* loss_out) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
   if (i > NPARAM) return;
+  // (moments and parameter are read before the sum: one round of loads)
+  float mo = 0.f, vo = 0.f, po = 0.f;
+  if (i < NPARAM && lr != 0.f) {
+    mo = m[i];
+    vo = v[i];
+    po = p[i];
+  }
   float g = 0.f;
+#pragma unroll 16
   for (int w = 0; w < nwg; w++) g += partial[(size_t)w * (NPARAM + 1) + i];
   if (i == NPARAM) {
     if (loss_out) *loss_out = g;
@@ -124,11 +141,11 @@ __global__ void k_mlp_adam(float* p, float* m, float* v, short* wb, short* wtb, 
   }
   if (grad_out) grad_out[i] = g;
   if (lr == 0.f) return;
-  const float mi = b1 * m[i] + (1.f - b1) * g;
-  const float vi = b2 * v[i] + (1.f - b2) * g * g;
+  const float mi = b1 * mo + (1.f - b1) * g;
+  const float vi = b2 * vo + (1.f - b2) * g * g;
   m[i] = mi;
   v[i] = vi;
-  const float w = p[i] - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
+  const float w = po - lr * (mi * c1) / (sqrtf(vi * c2) + eps);
   p[i] = w;
   pack_one(i, w, wb, wtb);
 }
@@ -138,10 +155,9 @@ __global__ void __launch_bounds__(256) k_mlp_infer(Net n, const float* X, int64_
   const int lane = threadIdx.x & 63, q = lane >> 4, j = lane & 15;
   const int64_t row = ((int64_t)blockIdx.x * 4 + (threadIdx.x >> 6)) * 16 + j;
   const bool active = row < nrows;
-  float x16[NIN];
-  for (int f = 0; f < NIN; f++) x16[f] = active ? X[row * NIN + f] : n.in_mean[f];
+  const f4 x = *(const f4*)((active ? X + row * NIN : n.in_mean) + 4 * q);
   s4 h1[8], h2[8], h3[8];
-  const f4 y = forward(n, input_frag(n, x16, lane), h1, h2, h3, lane);
+  const f4 y = forward(n, input_frag(n, x, lane), h1, h2, h3, lane);
   if (q == 0 && active)
     for (int r = 0; r < 4; r++) Y[row * NOUT + r] = y[r] / n.out_scale[r];
 }
@@ -166,6 +182,17 @@ int mguard(pdem_mlp* m, F f) {
     m->err = e.what();
   }
   return -1;
+}
+
+// grid of k_mlp_grad: shares of the weight-gradient blocks (at most 16: one
+// 16 x 16 block a wavefront and layer) until about GRAD_WGS workgroups run
+// (batch 4096: 44 us an iteration at 128, 47 at 256, 54 at 64; 1024 and below
+// do not care)
+constexpr int64_t GRAD_WGS = 128;
+dim3 grad_grid(int64_t nwg) {
+  int64_t parts = 1;
+  while (parts < 16 && 2 * parts * nwg <= GRAD_WGS) parts *= 2;
+  return dim3((unsigned)nwg, (unsigned)parts);
 }
 
 mlp::Net net_of(const pdem_mlp* m) { return mlp::make_net(m->wb, m->wtb, m->p, m->norm); }
@@ -333,7 +360,7 @@ int pdem_mlp_gradient(pdem_mlp* m, const float* x, const float* t, int64_t n, fl
     HIPCHK(hipMemcpyAsync(dx.p, x, n * mlp::NIN * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipMemcpyAsync(dt.p, t, n * mlp::NOUT * sizeof(float), hipMemcpyHostToDevice, m->stream));
     const mlp::Net net = net_of(m);
-    hipLaunchKernelGGL(mlp::k_mlp_grad, dim3((unsigned)nwg), dim3(256), 0, m->stream, net, dx.as<float>(),
+    hipLaunchKernelGGL(mlp::k_mlp_grad, grad_grid(nwg), dim3(256), 0, m->stream, net, dx.as<float>(),
                        dt.as<float>(), m->norm + 2 * mlp::NIN + mlp::NOUT, n, n, (uint64_t)0,
                        1.f / (float)n, m->partial);
     HIPCHK(hipGetLastError());
@@ -367,7 +394,7 @@ int pdem_mlp_train(pdem_mlp* m, const float* x, const float* t, int64_t n, int32
       const float c1 = 1.f / (1.f - std::pow(b1, (float)m->adam_step));
       const float c2 = 1.f / (1.f - std::pow(b2, (float)m->adam_step));
       const uint64_t sh = (seed * 0x2545f4914f6cdd1dull) ^ (uint64_t)(it + 1);
-      hipLaunchKernelGGL(mlp::k_mlp_grad, dim3((unsigned)nwg), dim3(256), 0, m->stream, net, dx.as<float>(),
+      hipLaunchKernelGGL(mlp::k_mlp_grad, grad_grid(nwg), dim3(256), 0, m->stream, net, dx.as<float>(),
                          dt.as<float>(), m->norm + 2 * mlp::NIN + mlp::NOUT, n, (int64_t)batch, sh ? sh : 1,
                          1.f / (float)batch, m->partial);
       hipLaunchKernelGGL(mlp::k_mlp_adam, dim3(blocks(mlp::NPARAM + 1)), dim3(TPB), 0, m->stream, m->p, m->m,
