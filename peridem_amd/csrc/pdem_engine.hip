@@ -362,7 +362,8 @@ struct Launch {
       return;
     }
     const unsigned pb = (unsigned)c->pd_tpb, pnb = blocks(c->N, c->pd_tpb);
-    if (c->ds.state_global) hipLaunchKernelGGL((k_pd_dilation<DIM, INF>), dim3(pnb), dim3(pb), 0, st, c->ds);
+    const unsigned qnb = blocks(c->N * PD_LPN, c->pd_tpb);
+    if (c->ds.state_global) hipLaunchKernelGGL((k_pd_dilation<DIM, INF>), dim3(qnb), dim3(pb), 0, st, c->ds);
     auto ev = ev_begin(c, st);
     if (c->rnp_tile)
       hipLaunchKernelGGL((k_pd_rnp_tile<DIM, INF>), dim3(c->rt.ntiles), dim3(RT_THREADS), c->rt.lds_bytes, st,
@@ -371,7 +372,7 @@ struct Launch {
       hipLaunchKernelGGL((k_pd_rnp<DIM, INF>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(pnb), dim3(pb), 0, st, c->ds);
-    if (c->state_any) hipLaunchKernelGGL((k_pd_state<DIM, INF>), dim3(pnb), dim3(pb), 0, st, c->ds);
+    if (c->state_any) hipLaunchKernelGGL((k_pd_state<DIM, INF>), dim3(qnb), dim3(pb), 0, st, c->ds);
     ev_end(c, ev, st, c->ev_next_group++);
   }
   static void pd_forces(pdem_ctx* c) {
@@ -1326,6 +1327,14 @@ void build(pdem_ctx* c, const pdem_desc* d) {
       [&] { hipLaunchKernelGGL(k_mx<3>, dim3(blocks(N)), dim3(TPB), 0, c->stream, s); });
   // nodes that never search keep an empty candidate list
   check_launch(c);
+  if (c->state_any && !(c->precision == PDEM_PREC_MIXED && c->ntiles > 0)) {
+    double* alpha = c->dalloc<double>(N);
+    double* factor = c->dalloc<double>(N);
+    hipLaunchKernelGGL(k_pd_factors, dim3(blocks(N)), dim3(TPB), 0, c->stream, s, alpha, factor);
+    check_launch(c);
+    s.alpha = alpha;
+    s.factor = factor;
+  }
   if (c->precision == PDEM_PREC_MIXED && c->state_any) {
     float* fa = c->dalloc<float>(N);
     hipLaunchKernelGGL(k_mixed_alpha, dim3(blocks(N)), dim3(TPB), 0, c->stream, s, fa);

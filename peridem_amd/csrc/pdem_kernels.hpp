@@ -113,6 +113,7 @@ struct DS {
   double* v[3];
   double* f[3];
   double *vol, *mx, *theta, *vmag;
+  const double *alpha, *factor;  // FP64 state-based passes: k_pd_factors
   float* Z;
   uint8_t* fix;
   int* ptid;
@@ -235,12 +236,10 @@ struct DS {
 
 // --------------------------------------------------------------- helpers
 __device__ __forceinline__ bool isGreater(double a, double b) {
-  double fa = fabs(a), fb = fabs(b);
-  return (a - b) > ((fa < fb ? fb : fa) * COMPARE_EPS);
+  return (a - b) > (fmax(fabs(a), fabs(b)) * COMPARE_EPS);
 }
 __device__ __forceinline__ bool isLess(double a, double b) {
-  double fa = fabs(a), fb = fabs(b);
-  return (b - a) > ((fa < fb ? fb : fa) * COMPARE_EPS);
+  return (b - a) > (fmax(fabs(a), fabs(b)) * COMPARE_EPS);
 }
 __device__ __forceinline__ double infFn(const DS& s, double r) {
   if (s.inf_type == 0) return s.inf_p0;
@@ -837,6 +836,16 @@ __device__ __forceinline__ double infJ(const DS& s, double r_over_delta, double 
   return s.inf_p0 * exp(-r * r / s.inf_p1);
 }
 
+// the same with the horizon's reciprocal at hand
+__device__ __forceinline__ double div_by(double a, double b, double y);
+template <int INF>
+__device__ __forceinline__ double infJr(const DS& s, double rji, double horizon, double yho) {
+  if (INF == 0) return s.inf_p0;
+  const double r = div_by(rji, horizon, yho);
+  if (INF == 1) return s.inf_p0 + s.inf_p1 * r;
+  return s.inf_p0 * exp(-r * r / s.inf_p1);
+}
+
 // Bond-based RNP: computePeridynamicForces force pass (demModel.cpp:682-788)
 // with RnpMaterial::getBondEF (material.h:342-368).  One lane per node; the
 // force sum runs over the neighbor list in order, as the reference's does.
@@ -1005,16 +1014,62 @@ __global__ void __launch_bounds__(256) k_pd_bond(DS s) {
   s.Z[i] = Zi;
 }
 
+// ------------------------------------------- FP64 helpers of the bond loops
+// a / b rounded correctly from y = 1 / b rounded correctly: two corrections of
+// a y by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990: the first
+// leaves the quotient within an ulp, the second rounds it), 5 instructions
+// where a division of its own takes about 15.  For divisors that several
+// quotients share.
+__device__ __forceinline__ double div_by(double a, double b, double y) {
+  double q = a * y;
+  q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// value of lane R of the own group of four lanes (no LDS access)
+template <int R>
+__device__ __forceinline__ int quad_lane(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, R * 0x55, 0xf, 0xf, true);
+}
+template <int R>
+__device__ __forceinline__ double quad_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)quad_lane<R>((int)b), hi = (unsigned)quad_lane<R>((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// acc + the group's four terms in lane order (bonds in list order; lanes
+// without a term give 0, which adds nothing)
+__device__ __forceinline__ double quad_add(double acc, double t) {
+  acc += quad_lane<0>(t);
+  acc += quad_lane<1>(t);
+  acc += quad_lane<2>(t);
+  return acc + quad_lane<3>(t);
+}
+
+// The state-based FP64 passes deal a node's bonds to four neighboring lanes:
+// lane `sub` evaluates bonds sub, sub + 4, ..., and the group adds the terms
+// in list order (the reference's order, so the sums are the same bit for bit).
+// With a lane per node the passes waited on each bond's gathers and its chain
+// of roots and divisions: the 60-sphere packing (67k nodes) is one wavefront
+// per SIMD.  Measured there: dilation 86 us and force 103 us with a lane per
+// node, 38 and 52 us now; a step of 400 spheres 1096 us, 495 us now (the lanes
+// also even out the lists' lengths).  What is left is FP64 issue: two roots,
+// three divisions and the ordered sums' lane moves per bond.  Divisions by the particle's h and horizon and by a
+// bond's length use the divisor's reciprocal (div_by); alpha and the dilation
+// factor of a node are constant and come from set-up.
+constexpr int PD_LPN = 4;
+
 // State-based dilation pass (demModel.cpp:610-679): bond breaking on the
 // actual stretch, theta_i = 3 sum r (|y|-r) J V^c / m_i.
 template <int DIM, int INF>
 __global__ void __launch_bounds__(256) k_pd_dilation(DS s) {
-  int64_t i = gid();
+  const int64_t i = gid() / PD_LPN;
   if (i >= s.N) return;
+  const int sub = (int)threadIdx.x & (PD_LPN - 1);
   const DevParticle& p = s.P[s.ptid[i]];
   if (!p.compute_force || p.material_type != 1) return;
   const double horizon = p.horizon, h = p.h;
   const double check_up = horizon + 0.5 * h, check_low = horizon - 0.5 * h;
+  const double yh = 1. / h, yho = 1. / horizon;
   const double sc = p.mat[2];
   const int64_t sl = i / WAVE, lane = i % WAVE;
   const int* c = s.col + s.sptr[sl] + lane;
@@ -1025,53 +1080,78 @@ __global__ void __launch_bounds__(256) k_pd_dilation(DS s) {
     xi[d] = s.xr[d][i];
     ui[d] = s.u[d][i];
   }
-  const double m = s.mx[i];
   double theta = 0.;
   unsigned word = 0, wnew = 0;
-  for (int k = 0; k < n; k++) {
-    if ((k & 31) == 0) {
-      if (k > 0 && wnew != word) bw[(int64_t)((k >> 5) - 1) * WAVE] = wnew;
-      word = bw[(int64_t)(k >> 5) * WAVE];
+  int jn = sub < n ? c[(int64_t)sub * WAVE] : (int)i;
+  for (int k0 = 0; k0 < n; k0 += PD_LPN) {
+    if ((k0 & 31) == 0) {
+      if (k0 > 0 && wnew != word && sub == 0) bw[(int64_t)((k0 >> 5) - 1) * WAVE] = wnew;
+      word = bw[(int64_t)(k0 >> 5) * WAVE];
       wnew = word;
     }
-    const int j = c[(int64_t)k * WAVE];
-    double dx[3], dy[3];
-    for (int d = 0; d < DIM; d++) {
-      dx[d] = s.xr[d][j] - xi[d];
-      dy[d] = (dx[d] + s.u[d][j]) - ui[d];
+    const int k = k0 + sub, j = jn;
+    if (k + PD_LPN < n) jn = c[(int64_t)(k + PD_LPN) * WAVE];
+    double term = 0.;
+    int brk = 0;  // breaks now
+    if (k < n) {
+      double dx[3], dy[3];
+      for (int d = 0; d < DIM; d++) {
+        dx[d] = s.xr[d][j] - xi[d];
+        dy[d] = (dx[d] + s.u[d][j]) - ui[d];
+      }
+      const double rji = len3<DIM>(dx);
+      const double change_length = len3<DIM>(dy) - rji;
+      const double st = change_length / rji;
+      bool fs = (word >> (k & 31)) & 1u;
+      if (!fs && isGreater(fabs(st), sc + 1.0e-10)) {
+        fs = true;
+        brk = 1;
+      }
+      if (!fs) {
+        double volj = s.vol[j];
+        if (isGreater(rji, check_low)) volj *= div_by(check_up - rji, h, yh);
+        term = rji * change_length * infJr<INF>(s, rji, horizon, yho) * volj;
+      }
     }
-    const double rji = len3<DIM>(dx);
-    const double change_length = len3<DIM>(dy) - rji;
-    const double st = change_length / rji;
-    bool fs = (word >> (k & 31)) & 1u;
-    if (!fs && isGreater(fabs(st), sc + 1.0e-10)) {
-      fs = true;
-      wnew |= 1u << (k & 31);
-    }
-    if (!fs) {
-      double volj = s.vol[j];
-      if (isGreater(rji, check_low)) volj *= (check_up - rji) / h;
-      theta += rji * change_length * infJ<INF>(s, 0., rji, horizon) * volj;
-    }
+    theta = quad_add(theta, term);
+    // (bonds rarely break)
+    if (quad_lane<0>(brk) | quad_lane<1>(brk) | quad_lane<2>(brk) | quad_lane<3>(brk))
+      wnew |= (unsigned)(quad_lane<0>(brk) | quad_lane<1>(brk) << 1 | quad_lane<2>(brk) << 2 | quad_lane<3>(brk) << 3)
+              << (k0 & 31);
   }
+  if (sub != 0) return;
   if (n > 0 && wnew != word) bw[(int64_t)((n - 1) >> 5) * WAVE] = wnew;
-  s.theta[i] = 3. * theta / m;
+  s.theta[i] = 3. * theta / s.mx[i];
+}
+
+// alpha and the dilation factor of the state-based law (constant per node)
+__global__ void k_pd_factors(DS s, double* alpha, double* factor) {
+  const int64_t i = gid();
+  if (i >= s.N) return;
+  const DevParticle& p = s.P[s.ptid[i]];
+  const double K = p.mat[0], G = p.mat[1], m = s.mx[i];
+  const double a = 15. * G / m;
+  alpha[i] = a;
+  factor[i] = (3. * K / m) - a / 3.;
 }
 
 // State-based force pass with PdState::getBondEF for both ends (material.h:1415-1429).
 template <int DIM, int INF>
 __global__ void __launch_bounds__(256) k_pd_state(DS s) {
-  int64_t i = gid();
+  const int64_t i = gid() / PD_LPN;
   if (i >= s.N) return;
+  const int sub = (int)threadIdx.x & (PD_LPN - 1);
   const DevParticle& p = s.P[s.ptid[i]];
   if (!p.compute_force) {
-    for (int d = 0; d < DIM; d++) s.f[d][i] = 0.;
+    if (sub == 0)
+      for (int d = 0; d < DIM; d++) s.f[d][i] = 0.;
     return;
   }
   if (p.material_type != 1) return;
   const double horizon = p.horizon, h = p.h;
   const double check_up = horizon + 0.5 * h, check_low = horizon - 0.5 * h;
-  const double K = p.mat[0], G = p.mat[1], s0 = p.mat[2];
+  const double s0 = p.mat[2];
+  const double yh = 1. / h, yho = 1. / horizon, ys0 = 1. / s0;
   const double Kn = p.Kn, Rc = p.Rc;
   const int64_t sl = i / WAVE, lane = i % WAVE;
   const int* c = s.col + s.sptr[sl] + lane;
@@ -1082,47 +1162,61 @@ __global__ void __launch_bounds__(256) k_pd_state(DS s) {
     xi[d] = s.xr[d][i];
     ui[d] = s.u[d][i];
   }
-  const double mi = s.mx[i], thetai = s.theta[i];
-  const double alpha_i = 15. * G / mi;
-  const double factor_i = (3. * K / mi) - alpha_i / 3.;
+  const double thetai = s.theta[i];
+  const double alpha_i = s.alpha[i], factor_i = s.factor[i];
   double force[3] = {0., 0., 0.};
   float Zi = 0.f;
   unsigned word = 0;
-  for (int k = 0; k < n; k++) {
-    if ((k & 31) == 0) word = bw[(int64_t)(k >> 5) * WAVE];
-    const int j = c[(int64_t)k * WAVE];
-    const bool fs = (word >> (k & 31)) & 1u;
-    double dx[3], du[3], dy[3];
-    for (int d = 0; d < DIM; d++) {
-      dx[d] = s.xr[d][j] - xi[d];
-      du[d] = s.u[d][j] - ui[d];
-      dy[d] = dx[d] + du[d];
+  int jn = sub < n ? c[(int64_t)sub * WAVE] : (int)i;
+  for (int k0 = 0; k0 < n; k0 += PD_LPN) {
+    if ((k0 & 31) == 0) word = bw[(int64_t)(k0 >> 5) * WAVE];
+    const int k = k0 + sub, j = jn;
+    if (k + PD_LPN < n) jn = c[(int64_t)(k + PD_LPN) * WAVE];
+    double term[3] = {0., 0., 0.}, z = 0.;
+    if (k < n) {
+      const bool fs = (word >> (k & 31)) & 1u;
+      double dx[3], dy[3];
+      for (int d = 0; d < DIM; d++) {
+        dx[d] = s.xr[d][j] - xi[d];
+        dy[d] = dx[d] + (s.u[d][j] - ui[d]);
+      }
+      double volj = s.vol[j];
+      const double rji = len3<DIM>(dx);
+      const double ly = len3<DIM>(dy);
+      const double Sji = (ly - rji) / rji;
+      if (!fs) {
+        if (isGreater(rji, check_low)) volj *= div_by(check_up - rji, h, yh);
+        const double J = infJr<INF>(s, rji, horizon, yho);
+        const double thetaj = s.theta[j];
+        const double cl = Sji * rji;
+        const double ef_i = J * (rji * thetai * factor_i + cl * alpha_i);
+        const double ef_j = J * (rji * thetaj * s.factor[j] + cl * s.alpha[j]);
+        const double scalar_f = (ef_i + ef_j) * volj;
+        const double yly = 1. / ly;
+        for (int d = 0; d < DIM; d++) term[d] = scalar_f * div_by(dy[d], ly, yly);
+      } else {
+        double y[3];
+        for (int d = 0; d < DIM; d++) y[d] = (s.xr[d][j] + s.u[d][j]) - (xi[d] + ui[d]);
+        const double R = len3<DIM>(y);
+        double scalar_f = Kn * volj * (R - Rc) / R;
+        if (scalar_f > 0.) scalar_f = 0.;
+        for (int d = 0; d < DIM; d++) term[d] = scalar_f * y[d];
+      }
+      z = fabs(div_by(Sji, s0, ys0));
     }
-    double volj = s.vol[j];
-    const double rji = len3<DIM>(dx);
-    const double ly = len3<DIM>(dy);
-    const double Sji = (ly - len3<DIM>(dx)) / len3<DIM>(dx);
-    if (!fs) {
-      if (isGreater(rji, check_low)) volj *= (check_up - rji) / h;
-      const double J = infJ<INF>(s, 0., rji, horizon);
-      const double mj = s.mx[j], thetaj = s.theta[j];
-      const double cl = Sji * rji;
-      const double ef_i = J * (rji * thetai * factor_i + cl * alpha_i);
-      const double alpha_j = 15. * G / mj;
-      const double factor_j = (3. * K / mj) - alpha_j / 3.;
-      const double ef_j = J * (rji * thetaj * factor_j + cl * alpha_j);
-      const double scalar_f = (ef_i + ef_j) * volj;
-      for (int d = 0; d < DIM; d++) force[d] += scalar_f * (dy[d] / ly);
-    } else {
-      double y[3];
-      for (int d = 0; d < DIM; d++) y[d] = (s.xr[d][j] + s.u[d][j]) - (xi[d] + ui[d]);
-      const double R = len3<DIM>(y);
-      double scalar_f = Kn * volj * (R - Rc) / R;
-      if (scalar_f > 0.) scalar_f = 0.;
-      for (int d = 0; d < DIM; d++) force[d] += scalar_f * y[d];
+    for (int d = 0; d < DIM; d++) force[d] = quad_add(force[d], term[d]);
+    // running damage maximum (relative compare, list order): looked at in
+    // order only where one of the group's four values would be stored
+    const int up = isGreater(z, (double)Zi) ? 1 : 0;
+    if (quad_lane<0>(up) | quad_lane<1>(up) | quad_lane<2>(up) | quad_lane<3>(up)) {
+      const double z0 = quad_lane<0>(z), z1 = quad_lane<1>(z), z2 = quad_lane<2>(z), z3 = quad_lane<3>(z);
+      if (isGreater(z0, (double)Zi)) Zi = (float)z0;
+      if (isGreater(z1, (double)Zi)) Zi = (float)z1;
+      if (isGreater(z2, (double)Zi)) Zi = (float)z2;
+      if (isGreater(z3, (double)Zi)) Zi = (float)z3;
     }
-    if (isGreater(fabs(Sji / s0), (double)Zi)) Zi = (float)fabs(Sji / s0);
   }
+  if (sub != 0) return;
   for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
   s.Z[i] = Zi;
 }
