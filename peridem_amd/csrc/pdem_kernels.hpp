@@ -1232,19 +1232,34 @@ __global__ void __launch_bounds__(256) k_pd_state(DS s) {
 // sets and contact sums run in ascending node id.
 constexpr int CELL_BLOCK = 4096;  // cells per scan block (1024 threads x 4)
 constexpr int CELL_TPB = 1024;
+constexpr int COUNT_GROUPS = 8;
 constexpr int CELL_MAX_BLOCKS = (1 << 25) / CELL_BLOCK;
 
-__device__ __forceinline__ int cellc(double a, double lo, double cell, int n) {
-  double k = floor((a - lo) / cell);
-  int ki = k < 0. ? 0 : (k > (double)(n - 1) ? n - 1 : (int)k);
-  return ki;
+// Cell coordinates wrap around: the cell a position falls in, counted from
+// glo in steps of `cell`, is taken modulo the grid's size, so nodes that leave
+// the grid spread over its cells like the others (the grid has at least
+// 2 csub + 1 cells a side, so a query's cells are distinct; the FP64 distance
+// test drops nodes that only share a cell).  Clamped to the edge cells
+// instead, the fragments of a bed that breaks up would all meet in a few
+// cells: 100 particles, 32k nodes, 5890 us per step, 150 wrapped.  Positions
+// CELL_FAR cells out and more (or not a number) are clamped there.
+constexpr int CELL_FAR = 1 << 26;
+__device__ __forceinline__ int cell_coord(double a, double lo, double cell) {
+  return (int)fmin(fmax(floor((a - lo) / cell), -(double)CELL_FAR), (double)CELL_FAR);
+}
+__device__ __forceinline__ int cell_wrap(int k, int n) {
+  if ((unsigned)k >= (unsigned)n) {
+    k %= n;
+    if (k < 0) k += n;
+  }
+  return k;
 }
 
 template <int DIM>
 __device__ __forceinline__ void count_node(const DS& s, int64_t i) {
-  int cx = cellc(s.x[0][i], s.glo[0], s.cell, s.gn[0]);
-  int cy = cellc(s.x[1][i], s.glo[1], s.cell, s.gn[1]);
-  int cz = DIM == 3 ? cellc(s.x[2][i], s.glo[2], s.cell, s.gn[2]) : 0;
+  int cx = cell_wrap(cell_coord(s.x[0][i], s.glo[0], s.cell), s.gn[0]);
+  int cy = cell_wrap(cell_coord(s.x[1][i], s.glo[1], s.cell), s.gn[1]);
+  int cz = DIM == 3 ? cell_wrap(cell_coord(s.x[2][i], s.glo[2], s.cell), s.gn[2]) : 0;
   int c = (cz * s.gn[1] + cy) * s.gn[0] + cx;
   const int pid = s.ptid[i];
   // the owner only moves -2 (empty) -> a particle id -> -1 (several): a cell
@@ -1255,20 +1270,25 @@ __device__ __forceinline__ void count_node(const DS& s, int64_t i) {
     if (old != -2 && old != pid) s.cell_owner[c] = -1;
   }
   // ranks: one atomic per distinct cell among the wavefront's active lanes
-  // (the lanes of a wavefront bin neighboring nodes, mostly into a few cells)
+  // (the lanes of a wavefront bin neighboring nodes, mostly into a few cells;
+  // lanes left after COUNT_GROUPS cells take one each).  The lanes agree on
+  // leaders first, so all atomics are in flight together: one after the
+  // other, scattered nodes waited for up to 64
   const int lane = (int)(threadIdx.x & (WAVE - 1));
-  unsigned long long todo = __ballot(1);
-  int slot = 0;
-  while (todo) {
+  unsigned long long todo = __ballot(1), mine = 1ull << lane;
+  int lead = lane;
+  for (int g = 0; g < COUNT_GROUPS && todo; g++) {
     const int leader = __ffsll((long long)todo) - 1;
-    const int cl = __shfl(c, leader);
-    const unsigned long long same = __ballot(c == cl);
-    int base = 0;
-    if (lane == leader) base = atomicAdd(&s.cell_count[cl], (int)__popcll(same));
-    base = __shfl(base, leader);
-    if (c == cl) slot = base + (int)__popcll(same & ((1ull << lane) - 1ull));
+    const unsigned long long same = __ballot(c == __shfl(c, leader));
+    if ((same >> lane) & 1ull) {
+      lead = leader;
+      mine = same;
+    }
     todo &= ~same;
   }
+  int slot = 0;
+  if (lane == lead) slot = atomicAdd(&s.cell_count[c], (int)__popcll(mine));
+  slot = __shfl(slot, lead) + (int)__popcll(mine & ((1ull << lane) - 1ull));
   s.node_cell[i] = c;
   s.node_slot[i] = slot;
 }
@@ -1379,31 +1399,29 @@ __device__ int query_node(const DS& s, int64_t i, int pi) {
   const float rf = (float)r;
   const float Rf = rf + 0x1p-19f * (amax + rf);
   const float R2f = Rf * Rf;
-  int cc0[3] = {0, 0, 0}, lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
-  for (int d = 0; d < DIM; d++) {
-    cc0[d] = cellc(xi[d], s.glo[d], s.cell, s.gn[d]);
-    lo[d] = cc0[d] - s.csub > 0 ? cc0[d] - s.csub : 0;
-    hi[d] = cc0[d] + s.csub < s.gn[d] - 1 ? cc0[d] + s.csub : s.gn[d] - 1;
-  }
+  int k0[3] = {0, 0, 0};
+  for (int d = 0; d < DIM; d++) k0[d] = cell_coord(xi[d], s.glo[d], s.cell);
+  const int cz = DIM == 3 ? s.csub : 0;
   int cnt = 0;
   double near2 = r2;  // nearest candidate (squared distance)
   const int cap = s.cap;
-  for (int z = lo[2]; z <= hi[2]; z++)
-    for (int y = lo[1]; y <= hi[1]; y++)
-      for (int x = lo[0]; x <= hi[0]; x++) {
-        // skip cells whose box lies beyond the search radius (clamped edge
-        // cells hold nodes outside the grid: never skipped)
-        const int c3[3] = {x, y, z};
+  for (int z = -cz; z <= cz; z++)
+    for (int y = -s.csub; y <= s.csub; y++)
+      for (int x = -s.csub; x <= s.csub; x++) {
+        // skip cells whose box lies beyond the search radius (clamped cells
+        // hold all nodes farther out: never skipped)
+        const int c3[3] = {k0[0] + x, k0[1] + y, k0[2] + z};
         double dmin2 = 0.;
         bool edge = false;
         for (int d = 0; d < DIM; d++) {
-          if (c3[d] == 0 || c3[d] == s.gn[d] - 1) edge = true;
+          if (abs(c3[d]) >= CELL_FAR) edge = true;
           const double b0 = s.glo[d] + c3[d] * s.cell, b1 = b0 + s.cell;
           const double t = xi[d] < b0 ? b0 - xi[d] : (xi[d] > b1 ? xi[d] - b1 : 0.);
           dmin2 += t * t;
         }
         if (!edge && dmin2 > r2 * 1.0000001) continue;
-        const int cc = (z * s.gn[1] + y) * s.gn[0] + x;
+        const int cc = ((DIM == 3 ? cell_wrap(c3[2], s.gn[2]) : 0) * s.gn[1] + cell_wrap(c3[1], s.gn[1])) * s.gn[0] +
+                       cell_wrap(c3[0], s.gn[0]);
         if (s.cell_owner[cc] == pi) continue;  // only the node's own particle
         const int m = s.cell_count[cc];
         const int64_t e0 = (int64_t)s.cell_boff[cc / CELL_BLOCK] + s.cell_start[cc];
