@@ -398,7 +398,7 @@ struct Launch {
   // the same dependencies, and a captured graph keeps the PD chain on the
   // engine's queue.
   static void pd_forces_and_cells(pdem_ctx* c) {
-    if (!c->multi) {
+    if (!c->multi || c->ds.cells_in_ctrl) {
       pd_forces(c);
       return;
     }
@@ -412,8 +412,8 @@ struct Launch {
   // standalone search: controller, cell list, candidate query
   static void contact_search(pdem_ctx* c) {
     hipStream_t st = c->stream;
-    hipLaunchKernelGGL(k_ctrl, dim3(CTRL_BLOCKS), dim3(1024), 0, st, c->ds, 0);
-    cells_build(c, st);
+    hipLaunchKernelGGL(k_ctrl<DIM>, dim3(CTRL_BLOCKS), dim3(1024), 0, st, c->ds, 0);
+    if (!c->ds.cells_in_ctrl) cells_build(c, st);
     rebuild_lists(c);
     hipLaunchKernelGGL(k_cells_init, dim3((unsigned)std::min<int64_t>(blocks(c->ds.ncells), 4096)), dim3(TPB), 0,
                        st, c->ds);
@@ -522,7 +522,7 @@ struct Launch {
     external_forces(c, c->multi != 0, fin || defer);
   }
   static void compute_forces(pdem_ctx* c) {
-    if (c->multi) hipLaunchKernelGGL(k_ctrl, dim3(CTRL_BLOCKS), dim3(1024), 0, c->stream, c->ds, 0);
+    if (c->multi) hipLaunchKernelGGL(k_ctrl<DIM>, dim3(CTRL_BLOCKS), dim3(1024), 0, c->stream, c->ds, 0);
     forces_after_ctrl(c);
   }
   // forces left pending by a deferred step, finalised in place
@@ -545,10 +545,10 @@ struct Launch {
       hipLaunchKernelGGL((k_integrate<DIM, false>), dim3(blocks(c->N)), dim3(TPB), 0, c->stream, c->ds, c->multi,
                          verlet ? 1 : 0);
     if (fused) {
-      hipLaunchKernelGGL(k_ctrl, dim3(1), dim3(1024), 0, c->stream, c->ds, 1);
+      hipLaunchKernelGGL(k_ctrl<DIM>, dim3(1), dim3(1024), 0, c->stream, c->ds, 1);
     } else {
       displacement_bc(c);
-      if (c->multi) hipLaunchKernelGGL(k_ctrl, dim3(CTRL_BLOCKS), dim3(1024), 0, c->stream, c->ds, 0);
+      if (c->multi) hipLaunchKernelGGL(k_ctrl<DIM>, dim3(CTRL_BLOCKS), dim3(1024), 0, c->stream, c->ds, 0);
     }
     c->nf_zeroed = c->ds.nf_zero != 0;  // the node update above zeroed f of the non-force nodes
     forces_after_ctrl(c, verlet);
@@ -1186,6 +1186,7 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     s.cell = cell;
     s.ncells = ncells;
     s.ncell_blocks = (ncells + CELL_BLOCK - 1) / CELL_BLOCK;
+    s.cells_in_ctrl = N <= CTRL_CELLS_NODES && ncells <= CTRL_CELLS ? 1 : 0;
     s.cell_count = c->dalloc<int>(ncells + 1);
     s.cell_owner = c->dalloc<int>(ncells + 1);
     hipLaunchKernelGGL(k_cells_init, dim3((unsigned)std::min<int64_t>(blocks(ncells), 4096)), dim3(TPB), 0,

@@ -149,6 +149,7 @@ struct DS {
   int* cell_btot;   // [nblocks] count total of each block of cells
   int* cell_boff;   // [nblocks] exclusive prefix of the block totals
   int64_t ncell_blocks;
+  int cells_in_ctrl;  // the controller builds the cell list (small models)
   int* node_cell;   // [N] cell of each node (this rebuild)
   int* node_slot;   // [N] rank of the node inside its cell
   int* cell_nodes;  // [N] node ids by cell
@@ -423,10 +424,25 @@ __device__ void ctrl_decide(Ctrl* cg) {
 // and runs the controller; all workgroups pack the non-wall particles' centre
 // data (and clear the closure's per-step flags).  The cell table is cleared
 // after each rebuild's query (k_contact_force), so no step clears it here.
+// For models of at most CTRL_CELLS_NODES nodes and CTRL_CELLS cells, workgroup 0
+// also builds the cell list on a rebuild step (cells_build_one): three launches
+// and a side stream less in every step, of which most find nothing to do.  With
+// them a small model's step waits for the side stream's fork, three kernels
+// that return at once and the join, about 26 us, whatever the bond kernel
+// takes (two-particle collision of 734 nodes: 56 us per step with the side
+// stream, 49 without; 3D packing of 10.4k nodes: 70 and 62).  The one workgroup
+// takes about 4 us per 1024 nodes, so at 16384 nodes it breaks even when every
+// third step rebuilds the list (11k nodes: 37 us per step against 54 with
+// rebuilds every 40 steps, 164 against 119 with one in every step).
 constexpr int CTRL_BLOCKS = 64;
+constexpr int64_t CTRL_CELLS_NODES = 16384, CTRL_CELLS = 65536;
+template <int DIM>
+__device__ void cells_build_one(const DS& s, int* lds);
 
+template <int DIM>
 __global__ void __launch_bounds__(1024) k_ctrl(DS s, int advance) {
   __shared__ unsigned long long red[1024 / WAVE], redm[1024 / WAVE];
+  __shared__ int scan_lds[1024 / WAVE];
   Ctrl* c = s.ctrl;
   const int t = threadIdx.x;
   // the node update before this kernel consumed any pending forces, and the
@@ -493,6 +509,10 @@ __global__ void __launch_bounds__(1024) k_ctrl(DS s, int advance) {
       if (moved) step += sqrt(__longlong_as_double((long long)mvb));
       c->dsum = c->rebuild ? 0. : c->dsum + step * (1. + 1e-9);
       c->mv_bc_acc = 0ull;
+    }
+    if (s.cells_in_ctrl) {
+      __syncthreads();
+      if (c->rebuild) cells_build_one<DIM>(s, scan_lds);
     }
   }
   if (advance) return;  // centre data packed by the fused node update
@@ -1344,6 +1364,14 @@ __global__ void __launch_bounds__(CELL_TPB) k_cells_scan(DS s) {
   if (threadIdx.x == 0) s.cell_btot[blockIdx.x] = tot;
 }
 
+// node i to its place e in the sorted list
+template <int DIM>
+__device__ __forceinline__ void cells_place(const DS& s, int64_t i, int64_t e) {
+  s.cell_nodes[e] = (int)i;
+  s.cell_xf[e] = make_float4((float)(s.x[0][i] - s.glo[0]), (float)(s.x[1][i] - s.glo[1]),
+                             DIM == 3 ? (float)(s.x[2][i] - s.glo[2]) : 0.f, __int_as_float(s.ptid[i]));
+}
+
 // block offsets (every workgroup scans the block totals; workgroup 0 stores
 // them for the query), then each node to its place in the sorted list
 template <int DIM>
@@ -1368,10 +1396,41 @@ __global__ void __launch_bounds__(CELL_TPB) k_cells_scatter(DS s) {
   const int64_t stride = (int64_t)gridDim.x * blockDim.x;
   for (int64_t i = gid(); i < s.N; i += stride) {
     const int c = s.node_cell[i];
-    const int64_t e = (int64_t)boff[c / CELL_BLOCK] + s.cell_start[c] + s.node_slot[i];
-    s.cell_nodes[e] = (int)i;
-    s.cell_xf[e] = make_float4((float)(s.x[0][i] - s.glo[0]), (float)(s.x[1][i] - s.glo[1]),
-                               DIM == 3 ? (float)(s.x[2][i] - s.glo[2]) : 0.f, __int_as_float(s.ptid[i]));
+    cells_place<DIM>(s, i, (int64_t)boff[c / CELL_BLOCK] + s.cell_start[c] + s.node_slot[i]);
+  }
+}
+
+// the whole cell list by one workgroup of CELL_TPB threads (see k_ctrl)
+template <int DIM>
+__device__ void cells_build_one(const DS& s, int* lds) {
+  for (int64_t i = threadIdx.x; i < s.N; i += CELL_TPB) count_node<DIM>(s, i);
+  __threadfence();
+  __syncthreads();
+  const auto load4 = [&](int64_t b, int* v) {
+    const int64_t c0 = b * CELL_BLOCK + 4 * threadIdx.x;
+    for (int k = 0; k < 4; k++) v[k] = c0 + k < s.ncells ? s.cell_count[c0 + k] : 0;
+  };
+  int carry = 0, nx[4];
+  load4(0, nx);
+  for (int64_t b = 0; b < s.ncell_blocks; b++) {
+    const int64_t c0 = b * CELL_BLOCK + 4 * threadIdx.x;
+    const int v[4] = {nx[0], nx[1], nx[2], nx[3]};
+    load4(b + 1, nx);  // (zero past the last block)
+    const int mine = v[0] + v[1] + v[2] + v[3];
+    int tot;
+    int run = block_scan_incl(mine, lds, tot) - mine;
+    for (int k = 0; k < 4; k++) {
+      if (c0 + k < s.ncells) s.cell_start[c0 + k] = run;
+      run += v[k];
+    }
+    if (threadIdx.x == 0) s.cell_boff[b] = carry;
+    carry += tot;
+  }
+  __threadfence();
+  __syncthreads();
+  for (int64_t i = threadIdx.x; i < s.N; i += CELL_TPB) {
+    const int c = s.node_cell[i];
+    cells_place<DIM>(s, i, s.cell_boff[c / CELL_BLOCK] + s.cell_start[c] + s.node_slot[i]);
   }
 }
 
