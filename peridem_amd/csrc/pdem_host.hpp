@@ -5,6 +5,7 @@
 
 #include <stdint.h>
 #include <atomic>
+#include <mutex>
 #include <string>
 
 struct HipError {
@@ -36,6 +37,10 @@ struct pdem_mlp {
   float* norm = nullptr;     // in_mean[16] in_scale[16] out_scale[4] out_weight[4]
   float* partial = nullptr;  // per-workgroup gradient partials
   int64_t partial_wg = 0;
+  std::mutex io;             // held by the call that uses pin / dev
+  void* pin = nullptr;       // pinned rows of small inference calls
+  void* dev = nullptr;       // device rows of larger ones
+  int64_t pin_rows = 0, dev_rows = 0;
   int64_t adam_step = 0;
   // engine contexts whose closure reads this network (their captured steps
   // hold its buffers): pdem_mlp_destroy refuses while it is nonzero
