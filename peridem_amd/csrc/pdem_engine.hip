@@ -469,7 +469,7 @@ struct Launch {
   static void rebuild_lists(pdem_ctx* c) {
     const int qb = (int)blocks(c->N);
     const int db = (int)std::min<int64_t>((std::max(c->ds.n_nonwall, 1) + 3) / 4, 1024);
-    hipLaunchKernelGGL(k_rebuild_lists<DIM>, dim3((unsigned)(qb + db)), dim3(TPB), 0, c->stream, c->ds, qb);
+    hipLaunchKernelGGL(k_rebuild_lists<DIM>, dim3((unsigned)(qb + db)), dim3(TPB), 0, c->stream, c->ds, db);
   }
   // closure pairs: connections (rebuild steps), modes, network, patch
   // records (2D, closure mode only)
@@ -1151,10 +1151,9 @@ void build(pdem_ctx* c, const pdem_desc* d) {
 
   // ---- contact structures
   if (c->multi) {
-    // uniform grid: csub cells span the largest search radius the controller
-    // can pick; the query scans +-csub cells around a node
-    s.csub = dim == 3 ? 2 : 1;
-    double cell = std::max(1.0, d->search_factor) * maxR / s.csub;
+    // uniform grid: cell_sub cells span the largest search radius the
+    // controller can pick; the query scans +-cell_sub cells around a node
+    double cell = std::max(1.0, d->search_factor) * maxR / cell_sub(dim);
     if (!(cell > 0.)) cell = 1.;
     double lo[3], hi[3];
     for (int k = 0; k < 3; k++) {
@@ -1184,6 +1183,7 @@ void build(pdem_ctx* c, const pdem_desc* d) {
       s.gn[k] = 1;
     }
     s.cell = cell;
+    s.inv_cell = 1. / cell;
     s.ncells = ncells;
     s.ncell_blocks = (ncells + CELL_BLOCK - 1) / CELL_BLOCK;
     s.cells_in_ctrl = N <= CTRL_CELLS_NODES && ncells <= CTRL_CELLS ? 1 : 0;
@@ -1196,8 +1196,7 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     s.cell_boff = c->dalloc<int>(s.ncell_blocks, false);
     s.node_cell = c->dalloc<int>(N, false);
     s.node_slot = c->dalloc<int>(N, false);
-    s.cell_nodes = c->dalloc<int>(N, false);
-    s.cell_xf = c->dalloc<float4>(N, false);
+    s.cell_nodes = c->dalloc<double4>(N, false);
     s.xa = c->dalloc<double4>(N, false);
     s.xa_epoch = c->dalloc<uint8_t>(N);
     HIPCHK(hipStreamCreateWithFlags(&c->side2, hipStreamNonBlocking));

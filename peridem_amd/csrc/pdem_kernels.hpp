@@ -136,9 +136,8 @@ struct DS {
   int* light;   // [N] node ids with few candidates
   // cell grid
   double glo[3];
-  double cell;
+  double cell, inv_cell;
   int gn[3];
-  int csub;  // cells per largest search radius: the query scans +-csub cells
   int64_t ncells;
   // Cell list of the last rebuild: the nodes sorted by cell key (a counting
   // sort: per-cell counts, an exclusive scan over the cells in blocks of
@@ -152,8 +151,7 @@ struct DS {
   int cells_in_ctrl;  // the controller builds the cell list (small models)
   int* node_cell;   // [N] cell of each node (this rebuild)
   int* node_slot;   // [N] rank of the node inside its cell
-  int* cell_nodes;  // [N] node ids by cell
-  float4* cell_xf;  // [N] beside cell_nodes: position - glo in FP32, particle id (bits)
+  double4* cell_nodes;  // [N] nodes by cell: position, (particle << 32 | node id) as bits
   int* cell_owner;  // [ncells] particle id when one particle fills the cell, -1 mixed, -2 empty
   // Candidate positions for the contact loops of the steps between rebuilds:
   // one 32-byte record per node (x, y, z in FP64 and the particle id's bits
@@ -1242,7 +1240,7 @@ __global__ void __launch_bounds__(256) k_pd_state(DS s) {
 }
 
 // ---------------------------------------------------------- cell list
-// Uniform grid with cell >= the largest search radius / csub (at most 2^25
+// Uniform grid with cell >= the largest search radius / cell_sub (at most 2^25
 // cells: CELL_MAX_BLOCKS blocks of CELL_BLOCK).  At a rebuild
 // the nodes are sorted by cell key with a counting sort on the grid:
 // k_cells_count (per-cell counts and each node's rank in its cell),
@@ -1256,16 +1254,18 @@ constexpr int COUNT_GROUPS = 8;
 constexpr int CELL_MAX_BLOCKS = (1 << 25) / CELL_BLOCK;
 
 // Cell coordinates wrap around: the cell a position falls in, counted from
-// glo in steps of `cell`, is taken modulo the grid's size, so nodes that leave
+// glo in steps of the cell size, is taken modulo the grid's size, so nodes that leave
 // the grid spread over its cells like the others (the grid has at least
-// 2 csub + 1 cells a side, so a query's cells are distinct; the FP64 distance
+// 2 cell_sub + 1 cells a side, so a query's cells are distinct; the FP64 distance
 // test drops nodes that only share a cell).  Clamped to the edge cells
 // instead, the fragments of a bed that breaks up would all meet in a few
 // cells: 100 particles, 32k nodes, 5890 us per step, 150 wrapped.  Positions
 // CELL_FAR cells out and more (or not a number) are clamped there.
-constexpr int CELL_FAR = 1 << 26;
-__device__ __forceinline__ int cell_coord(double a, double lo, double cell) {
-  return (int)fmin(fmax(floor((a - lo) / cell), -(double)CELL_FAR), (double)CELL_FAR);
+constexpr int CELL_FAR = 1 << 22;
+// cells that span the largest search radius
+constexpr int cell_sub(int dim) { return dim == 3 ? 2 : 1; }
+__device__ __forceinline__ int cell_coord(double a, double lo, double inv_cell) {
+  return (int)fmin(fmax(floor((a - lo) * inv_cell), -(double)CELL_FAR), (double)CELL_FAR);
 }
 __device__ __forceinline__ int cell_wrap(int k, int n) {
   if ((unsigned)k >= (unsigned)n) {
@@ -1277,9 +1277,9 @@ __device__ __forceinline__ int cell_wrap(int k, int n) {
 
 template <int DIM>
 __device__ __forceinline__ void count_node(const DS& s, int64_t i) {
-  int cx = cell_wrap(cell_coord(s.x[0][i], s.glo[0], s.cell), s.gn[0]);
-  int cy = cell_wrap(cell_coord(s.x[1][i], s.glo[1], s.cell), s.gn[1]);
-  int cz = DIM == 3 ? cell_wrap(cell_coord(s.x[2][i], s.glo[2], s.cell), s.gn[2]) : 0;
+  int cx = cell_wrap(cell_coord(s.x[0][i], s.glo[0], s.inv_cell), s.gn[0]);
+  int cy = cell_wrap(cell_coord(s.x[1][i], s.glo[1], s.inv_cell), s.gn[1]);
+  int cz = DIM == 3 ? cell_wrap(cell_coord(s.x[2][i], s.glo[2], s.inv_cell), s.gn[2]) : 0;
   int c = (cz * s.gn[1] + cy) * s.gn[0] + cx;
   const int pid = s.ptid[i];
   // the owner only moves -2 (empty) -> a particle id -> -1 (several): a cell
@@ -1367,9 +1367,8 @@ __global__ void __launch_bounds__(CELL_TPB) k_cells_scan(DS s) {
 // node i to its place e in the sorted list
 template <int DIM>
 __device__ __forceinline__ void cells_place(const DS& s, int64_t i, int64_t e) {
-  s.cell_nodes[e] = (int)i;
-  s.cell_xf[e] = make_float4((float)(s.x[0][i] - s.glo[0]), (float)(s.x[1][i] - s.glo[1]),
-                             DIM == 3 ? (float)(s.x[2][i] - s.glo[2]) : 0.f, __int_as_float(s.ptid[i]));
+  s.cell_nodes[e] =
+      make_double4(s.x[0][i], s.x[1][i], DIM == 3 ? s.x[2][i] : 0., __hiloint2double(s.ptid[i], (int)i));
 }
 
 // block offsets (every workgroup scans the block totals; workgroup 0 stores
@@ -1436,75 +1435,85 @@ __device__ void cells_build_one(const DS& s, int* lds) {
 
 // radiusSearchExcludeTag for one searching node (demModel.cpp:1717-1756):
 // other particles, j != i, 0 + dx^2 + dy^2 + dz^2 < r^2.
-// Cell entries are first tested on their FP32 copy (one 16-byte load: the
-// position relative to the grid origin and the particle id): an entry is
-// dropped when its FP32 distance is at least Rf = r + 2^-19 (max|a| + r),
-// a = x_i - glo.  Rounding a and b = x_j - glo to FP32 moves each component
-// by at most 2^-24 |a| and 2^-24 (|a| + r) for |x_j - x_i| < r, and the FP32
-// difference and sum add a relative 2^-22 at most, so an entry within r of
-// node i always passes, with a factor of four to spare.  Entries that pass
-// take the FP64 test below, which alone decides the candidate set.
+// The query waits on loads, so they go out together: the owners of a plane of
+// (2 cell_sub + 1)^2 cells, the headers of a row of them where other
+// particles' nodes are, then QAHEAD list entries at a time.  An entry is
+// all that the test needs (position, particle, node id: 32 bytes).  With one
+// cell and one entry after the other, and FP32 copies of the positions that
+// led to the FP64 ones, a rebuild's launch took 290 us for 10k nodes in 3D
+// (170 now), 1120 us for 4.2M nodes of 512 2D instances (780), 98 us for 166k
+// nodes of a broken-up 2D ensemble (54).
+constexpr int QAHEAD = 4;
 template <int DIM>
 __device__ int query_node(const DS& s, int64_t i, int pi) {
+  constexpr int CS = cell_sub(DIM), NX = 2 * CS + 1;
   const double r = s.ctrl->radius, r2 = r * r;
   double xi[3] = {0., 0., 0.};
-  for (int d = 0; d < DIM; d++) xi[d] = s.x[d][i];
-  float af[3] = {0.f, 0.f, 0.f};
-  float amax = 0.f;
-  for (int d = 0; d < DIM; d++) {
-    af[d] = (float)(xi[d] - s.glo[d]);
-    amax = fmaxf(amax, fabsf(af[d]));
-  }
-  const float rf = (float)r;
-  const float Rf = rf + 0x1p-19f * (amax + rf);
-  const float R2f = Rf * Rf;
   int k0[3] = {0, 0, 0};
-  for (int d = 0; d < DIM; d++) k0[d] = cell_coord(xi[d], s.glo[d], s.cell);
-  const int cz = DIM == 3 ? s.csub : 0;
+  for (int d = 0; d < DIM; d++) {
+    xi[d] = s.x[d][i];
+    k0[d] = cell_coord(xi[d], s.glo[d], s.inv_cell);
+  }
+  // squared distance from the node to cell k of dimension d; clamped cells
+  // hold all nodes farther out (0)
+  const auto reach = [&](int d, int k) {
+    const double b0 = s.glo[d] + k * s.cell, b1 = b0 + s.cell;
+    const double t = xi[d] < b0 ? b0 - xi[d] : (xi[d] > b1 ? xi[d] - b1 : 0.);
+    return abs(k) >= CELL_FAR ? 0. : t * t;
+  };
   int cnt = 0;
   double near2 = r2;  // nearest candidate (squared distance)
   const int cap = s.cap;
-  for (int z = -cz; z <= cz; z++)
-    for (int y = -s.csub; y <= s.csub; y++)
-      for (int x = -s.csub; x <= s.csub; x++) {
-        // skip cells whose box lies beyond the search radius (clamped cells
-        // hold all nodes farther out: never skipped)
-        const int c3[3] = {k0[0] + x, k0[1] + y, k0[2] + z};
-        double dmin2 = 0.;
-        bool edge = false;
-        for (int d = 0; d < DIM; d++) {
-          if (abs(c3[d]) >= CELL_FAR) edge = true;
-          const double b0 = s.glo[d] + c3[d] * s.cell, b1 = b0 + s.cell;
-          const double t = xi[d] < b0 ? b0 - xi[d] : (xi[d] > b1 ? xi[d] - b1 : 0.);
-          dmin2 += t * t;
-        }
-        if (!edge && dmin2 > r2 * 1.0000001) continue;
-        const int cc = ((DIM == 3 ? cell_wrap(c3[2], s.gn[2]) : 0) * s.gn[1] + cell_wrap(c3[1], s.gn[1])) * s.gn[0] +
-                       cell_wrap(c3[0], s.gn[0]);
-        if (s.cell_owner[cc] == pi) continue;  // only the node's own particle
-        const int m = s.cell_count[cc];
-        const int64_t e0 = (int64_t)s.cell_boff[cc / CELL_BLOCK] + s.cell_start[cc];
-        const int* cn = s.cell_nodes + e0;
-        const float4* cx = s.cell_xf + e0;
-        for (int q = 0; q < m; q++) {
-          const float4 e = cx[q];
-          if (__float_as_int(e.w) == pi) continue;  // the node's own particle (and i itself)
-          const float t0 = af[0] - e.x, t1 = af[1] - e.y, t2 = DIM == 3 ? af[2] - e.z : 0.f;
-          const float d2f = t0 * t0 + t1 * t1 + t2 * t2;
-          if (!(d2f < R2f)) continue;
-          const int j = cn[q];
-          double d2 = 0.;
-          for (int d = 0; d < DIM; d++) {
-            double t = xi[d] - s.x[d][j];
-            d2 += t * t;
-          }
-          if (d2 < r2) {
-            if (cnt < cap) s.cand[cand_idx(s.N, i, cnt)] = j;
-            cnt++;
-            near2 = d2 < near2 ? d2 : near2;
+  for (int z = DIM == 3 ? -CS : 0; z <= (DIM == 3 ? CS : 0); z++) {
+    const double rz = DIM == 3 ? reach(2, k0[2] + z) : 0.;
+    if (rz > r2 * 1.0000001) continue;
+    const int plane = DIM == 3 ? cell_wrap(k0[2] + z, s.gn[2]) * s.gn[1] : 0;
+    int own[NX * NX];
+#pragma unroll
+    for (int q = 0; q < NX * NX; q++)
+      own[q] = s.cell_owner[(plane + cell_wrap(k0[1] + q / NX - CS, s.gn[1])) * s.gn[0] +
+                            cell_wrap(k0[0] + q % NX - CS, s.gn[0])];
+    // cells with other particles' nodes and within the search radius
+    unsigned todo = 0;
+#pragma unroll
+    for (int q = 0; q < NX * NX; q++)
+      if (own[q] != pi && own[q] != -2 &&
+          rz + reach(1, k0[1] + q / NX - CS) + reach(0, k0[0] + q % NX - CS) <= r2 * 1.0000001)
+        todo |= 1u << q;
+    for (int y = 0; todo; y++, todo >>= NX) {
+      if (!(todo & ((1u << NX) - 1u))) continue;
+      const int row = (plane + cell_wrap(k0[1] + y - CS, s.gn[1])) * s.gn[0];
+      int m[NX], e0[NX];
+#pragma unroll
+      for (int x = 0; x < NX; x++) {
+        const int cc = row + cell_wrap(k0[0] + x - CS, s.gn[0]);
+        m[x] = s.cell_count[cc];
+        e0[x] = s.cell_boff[cc / CELL_BLOCK] + s.cell_start[cc];
+      }
+#pragma unroll
+      for (int x = 0; x < NX; x++) {
+        if (!((todo >> x) & 1u)) continue;
+        const double4* ce = s.cell_nodes + e0[x];
+        for (int q0 = 0; q0 < m[x]; q0 += QAHEAD) {
+          double4 e[QAHEAD];
+          for (int q = 0; q < QAHEAD; q++) e[q] = ce[q0 + q < m[x] ? q0 + q : q0];
+          for (int q = 0; q < QAHEAD; q++) {
+            if (q0 + q >= m[x] || __double2hiint(e[q].w) == pi) continue;  // the node's own particle (and i itself)
+            const double t0 = xi[0] - e[q].x, t1 = xi[1] - e[q].y, t2 = xi[2] - e[q].z;
+            double d2 = 0.;
+            d2 += t0 * t0;
+            d2 += t1 * t1;
+            if (DIM == 3) d2 += t2 * t2;
+            if (d2 < r2) {
+              if (cnt < cap) s.cand[cand_idx(s.N, i, cnt)] = __double2loint(e[q].w);
+              cnt++;
+              near2 = d2 < near2 ? d2 : near2;
+            }
           }
         }
       }
+    }
+  }
   if (cnt > cap) {
     s.ctrl->overflow = 1;
     cnt = cap;
@@ -1898,22 +1907,25 @@ __device__ void damp_pairs_one(const DS& s, int q, int lane) {
   }
 }
 
-// Rebuild steps only: the candidate query (radiusSearchExcludeTag per
-// searching node, demModel.cpp:1717-1756) on workgroups [0, qblocks) and the
-// damping partner lists (a wavefront per particle) on the others; the two are
-// independent.  The cell table is emptied afterwards by the contact-force
-// kernel (or k_cells_init outside the step).
+// Rebuild steps only: the damping partner lists (a wavefront per particle) on
+// workgroups [0, dblocks) and the candidate query (radiusSearchExcludeTag per
+// searching node, demModel.cpp:1717-1756) on the others; the two are
+// independent.  (The long loops over the particles start first: after the
+// query they were a tail of a third of the launch for 17k particles.)  The
+// cell table is emptied afterwards by the contact-force kernel (or
+// k_cells_init outside the step).
 template <int DIM>
-__global__ void __launch_bounds__(256) k_rebuild_lists(DS s, int qblocks) {
+__global__ void __launch_bounds__(256, 4) k_rebuild_lists(DS s, int dblocks) {
   if (!s.ctrl->rebuild) return;
-  if ((int)blockIdx.x < qblocks) {
+  const int qblocks = (int)gridDim.x - dblocks, qb = (int)blockIdx.x - dblocks;
+  if (qb >= 0) {
     // the workgroup's nodes join the light and active lists with one atomic
     // per list and workgroup (ballot counts per wavefront, offsets in LDS)
     __shared__ unsigned wcnt[2][256 / WAVE];
     __shared__ unsigned wbase[2];
     const int lane = (int)(threadIdx.x & (WAVE - 1)), w = (int)(threadIdx.x / WAVE);
     const unsigned long long below = (1ull << lane) - 1ull;
-    for (int64_t b0 = (int64_t)blockIdx.x * blockDim.x; b0 < s.N; b0 += (int64_t)qblocks * blockDim.x) {
+    for (int64_t b0 = (int64_t)qb * blockDim.x; b0 < s.N; b0 += (int64_t)qblocks * blockDim.x) {
       const int64_t i = b0 + threadIdx.x;
       const int list = i < s.N ? query_one<DIM>(s, i) : 0;
       const unsigned long long ml = __ballot(list == 1), ma = __ballot(list == 2);
@@ -1940,8 +1952,8 @@ __global__ void __launch_bounds__(256) k_rebuild_lists(DS s, int qblocks) {
     return;
   }
   const int lane = threadIdx.x & (WAVE - 1);
-  const int nw = ((int)gridDim.x - qblocks) * (int)(blockDim.x / WAVE);
-  for (int q = ((int)blockIdx.x - qblocks) * (int)(blockDim.x / WAVE) + (int)(threadIdx.x / WAVE);
+  const int nw = dblocks * (int)(blockDim.x / WAVE);
+  for (int q = (int)blockIdx.x * (int)(blockDim.x / WAVE) + (int)(threadIdx.x / WAVE);
        q < s.n_nonwall; q += nw)
     damp_pairs_one<DIM>(s, q, lane);
 }
