@@ -121,7 +121,7 @@ struct pdem_ctx {
   bool graph_verlet = false;  // the captured step is integrateVerlet
   // bond-based RNP pair-tile kernel (FP64, all force-computing particles RNP)
   RnpTileArgs rt{};
-  bool rnp_tile = false;  // use it (set up by default, autotuned)
+  bool rnp_tile = false;  // use it (by size, RNP_TILE_NODES; autotuned)
   bool nf_zeroed = false;  // inside a step whose node update zeroed f of the non-force nodes
   int step_fusion = 1;  // fused step kernels: 0 never, 1 models up to FUSE_MAX_NODES, 2 any size
   bool state_fusion = true;  // closed state-based tiles run both passes in one kernel
@@ -343,6 +343,14 @@ struct Launch {
       HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
     }
   }
+  // lanes per node of the lane-group RNP kernel (RNP16_NODES)
+  template <int INF>
+  static void rnp(pdem_ctx* c, int tpb) {
+    if (c->N <= RNP16_NODES)
+      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 16>), dim3(blocks(c->N * 16, tpb)), dim3(tpb), 0, c->stream, c->ds);
+    else
+      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 4>), dim3(blocks(c->N * 4, tpb)), dim3(tpb), 0, c->stream, c->ds);
+  }
   template <int INF>
   static void pd_inf(pdem_ctx* c) {
     hipStream_t st = c->stream;
@@ -350,7 +358,7 @@ struct Launch {
     if (c->precision == PDEM_PREC_MIXED && c->ntiles > 0) {
       if (c->ds.n_noforce > 0 && !c->nf_zeroed)
         hipLaunchKernelGGL(k_zero_noforce<DIM>, dim3(std::min<unsigned>(nb, BZ_BLOCKS)), dim3(TPB), 0, st, c->ds);
-      if (c->rnp_any) hipLaunchKernelGGL((k_pd_rnp<DIM, INF>), dim3(nb), dim3(TPB), 0, st, c->ds);
+      if (c->rnp_any) rnp<INF>(c, TPB);
       if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(nb), dim3(TPB), 0, st, c->ds);
       if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(nb), dim3(TPB), 0, st, c->ds);
       // timed inside: both state-based passes (dilation and force), all tiles
@@ -369,7 +377,7 @@ struct Launch {
       hipLaunchKernelGGL((k_pd_rnp_tile<DIM, INF>), dim3(c->rt.ntiles), dim3(RT_THREADS), c->rt.lds_bytes, st,
                          c->ds, c->rt);
     else if (c->rnp_any || !(c->state_any || c->pmb_any || c->elastic_any))
-      hipLaunchKernelGGL((k_pd_rnp<DIM, INF>), dim3(pnb), dim3(pb), 0, st, c->ds);
+      rnp<INF>(c, c->pd_tpb);
     if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->state_any) hipLaunchKernelGGL((k_pd_state<DIM, INF>), dim3(qnb), dim3(pb), 0, st, c->ds);
@@ -741,7 +749,7 @@ void build_rnp_tiles(pdem_ctx* c) {
                        (const void*)k_pd_rnp_tile<3, 2>})
           HIPCHK(hipFuncSetAttribute(f, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
       });
-  c->rnp_tile = true;
+  c->rnp_tile = c->N > RNP_TILE_NODES;
 }
 
 // Lists of the mixed tiles (DevTile).  Tiles with equal lists (the copies of

@@ -845,6 +845,45 @@ __global__ void k_fbc(DS s, DevBc bc) {
   }
 }
 
+// ------------------------------------------- FP64 helpers of the bond loops
+// a / b rounded correctly from y = 1 / b rounded correctly: two corrections of
+// a y by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990: the first
+// leaves the quotient within an ulp, the second rounds it), 5 instructions
+// where a division of its own takes about 15.  For divisors that several
+// quotients share.
+__device__ __forceinline__ double div_by(double a, double b, double y) {
+  double q = a * y;
+  q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
+  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+}
+// value of lane R of the own group of four lanes (no LDS access)
+template <int R>
+__device__ __forceinline__ int quad_lane(int v) {
+  return __builtin_amdgcn_update_dpp(0, v, R * 0x55, 0xf, 0xf, true);
+}
+template <int R>
+__device__ __forceinline__ double quad_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)quad_lane<R>((int)b), hi = (unsigned)quad_lane<R>((int)(b >> 32));
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// value of lane R of the own group of 16 lanes
+template <int R>
+__device__ __forceinline__ double row_lane(double v) {
+  const long long b = __double_as_longlong(v);
+  const unsigned lo = (unsigned)__builtin_amdgcn_update_dpp(0, (int)b, 0x150 + R, 0xf, 0xf, true);
+  const unsigned hi = (unsigned)__builtin_amdgcn_update_dpp(0, (int)(b >> 32), 0x150 + R, 0xf, 0xf, true);
+  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
+}
+// acc + the group's four terms in lane order (bonds in list order; lanes
+// without a term give 0, which adds nothing)
+__device__ __forceinline__ double quad_add(double acc, double t) {
+  acc += quad_lane<0>(t);
+  acc += quad_lane<1>(t);
+  acc += quad_lane<2>(t);
+  return acc + quad_lane<3>(t);
+}
+
 // -------------------------------------------------------- PD bond forces
 template <int INF>
 __device__ __forceinline__ double infJ(const DS& s, double r_over_delta, double rji, double horizon) {
@@ -855,7 +894,6 @@ __device__ __forceinline__ double infJ(const DS& s, double r_over_delta, double 
 }
 
 // the same with the horizon's reciprocal at hand
-__device__ __forceinline__ double div_by(double a, double b, double y);
 template <int INF>
 __device__ __forceinline__ double infJr(const DS& s, double rji, double horizon, double yho) {
   if (INF == 0) return s.inf_p0;
@@ -864,23 +902,66 @@ __device__ __forceinline__ double infJr(const DS& s, double rji, double horizon,
   return s.inf_p0 * exp(-r * r / s.inf_p1);
 }
 
+// acc + the terms of the group's LPN lanes (4 or 16) in lane order
+template <int LPN>
+__device__ __forceinline__ double group_add(double acc, double t) {
+  if (LPN == 4) return quad_add(acc, t);
+  acc += row_lane<0>(t);
+  acc += row_lane<1>(t);
+  acc += row_lane<2>(t);
+  acc += row_lane<3>(t);
+  acc += row_lane<4>(t);
+  acc += row_lane<5>(t);
+  acc += row_lane<6>(t);
+  acc += row_lane<7>(t);
+  acc += row_lane<8>(t);
+  acc += row_lane<9>(t);
+  acc += row_lane<10>(t);
+  acc += row_lane<11>(t);
+  acc += row_lane<12>(t);
+  acc += row_lane<13>(t);
+  acc += row_lane<14>(t);
+  return acc + row_lane<15>(t);
+}
+// the own group's bits of a ballot
+template <int LPN>
+__device__ __forceinline__ unsigned group_bits(bool on) {
+  const unsigned long long m = __ballot(on);
+  return (unsigned)(m >> ((threadIdx.x & (WAVE - 1)) / LPN * LPN)) & ((1u << LPN) - 1u);
+}
+
 // Bond-based RNP: computePeridynamicForces force pass (demModel.cpp:682-788)
-// with RnpMaterial::getBondEF (material.h:342-368).  One lane per node; the
-// force sum runs over the neighbor list in order, as the reference's does.
-// The next neighbor's data is loaded while the current bond is evaluated.
-template <int DIM, int INF>
+// with RnpMaterial::getBondEF (material.h:342-368).  LPN lanes per node: the
+// group evaluates LPN bonds at a time and adds their terms in list order, as
+// the reference does.
+// A node's bonds one after the other are a chain of about 28 gathers, divides,
+// square roots and exponentials; with fewer nodes than the chip has lanes the
+// pass takes as long as one chain.  Dealt to 16 lanes a node has two rounds.
+// With more nodes the FP64 issue rate counts: 16 lanes then waste the last
+// round of each list, 4 lanes less, and the pair-tile kernel evaluates each
+// bond's law once for both ends.  Force pass of 2D beds, us, tile / 4 lanes /
+// 16 lanes (before, one lane per node was slower than the tile throughout):
+//     734 nodes   30 / 14 /  10        37k   27 / 21 / 25
+//    6926         25 / 14 /  11        59k   40 / 25 / 36
+//   14.6k         29 / 14 /  14        98k   34 / 36 / 58
+//     21k         28 / 18 /  19       191k   51 / 58 / 106
+constexpr int64_t RNP16_NODES = 16384, RNP_TILE_NODES = 81920;
+template <int DIM, int INF, int LPN>
 __global__ void __launch_bounds__(256) k_pd_rnp(DS s) {
-  int64_t i = gid();
+  const int64_t i = gid() / LPN;
   if (i >= s.N) return;
+  const int sub = (int)threadIdx.x & (LPN - 1);
   const DevParticle& p = s.P[s.ptid[i]];
   if (!p.compute_force) {
-    for (int d = 0; d < DIM; d++) s.f[d][i] = 0.;
+    if (sub == 0)
+      for (int d = 0; d < DIM; d++) s.f[d][i] = 0.;
     return;
   }
   if (p.material_type != 0) return;
   const double horizon = p.horizon, h = p.h;
   const double check_up = horizon + 0.5 * h, check_low = horizon - 0.5 * h;
   const double Cc = p.mat[0], beta = p.mat[1], rbar = p.mat[2], invF = p.mat[3], fsc = p.mat[4];
+  const double yh = 1. / h, yho = 1. / horizon, yF = 1. / invF;
   const bool irrev = p.irreversible != 0;
   const double Kn = p.Kn, Rc = p.Rc;
   const int64_t sl = i / WAVE, lane = i % WAVE;
@@ -895,63 +976,58 @@ __global__ void __launch_bounds__(256) k_pd_rnp(DS s) {
   double force[3] = {0., 0., 0.};
   float Zi = 0.f;
   unsigned word = 0, wnew = 0;
-  double xn[3], un[3], vn = 0.;
-  if (n > 0) {
-    const int j0 = c[0];
-    for (int d = 0; d < DIM; d++) {
-      xn[d] = s.xr[d][j0];
-      un[d] = s.u[d][j0];
-    }
-    vn = s.vol[j0];
-  }
-  for (int k = 0; k < n; k++) {
-    if ((k & 31) == 0) {
-      if (k > 0 && wnew != word) bw[(int64_t)((k >> 5) - 1) * WAVE] = wnew;
-      word = bw[(int64_t)(k >> 5) * WAVE];
+  int jn = sub < n ? c[(int64_t)sub * WAVE] : (int)i;
+  for (int k0 = 0; k0 < n; k0 += LPN) {
+    if ((k0 & 31) == 0) {
+      if (k0 > 0 && wnew != word && sub == 0) bw[(int64_t)((k0 >> 5) - 1) * WAVE] = wnew;
+      word = bw[(int64_t)(k0 >> 5) * WAVE];
       wnew = word;
     }
-    double xj[3], uj[3];
-    for (int d = 0; d < DIM; d++) {
-      xj[d] = xn[d];
-      uj[d] = un[d];
-    }
-    double volj = vn;
-    if (k + 1 < n) {
-      const int jn = c[(int64_t)(k + 1) * WAVE];
+    const int k = k0 + sub, j = jn;
+    if (k + LPN < n) jn = c[(int64_t)(k + LPN) * WAVE];
+    double term[3] = {0., 0., 0.}, z = 0.;
+    bool brk = false;
+    if (k < n) {
+      double xj[3], uj[3], dx[3], du[3];
       for (int d = 0; d < DIM; d++) {
-        xn[d] = s.xr[d][jn];
-        un[d] = s.u[d][jn];
+        xj[d] = s.xr[d][j];
+        uj[d] = s.u[d][j];
+        dx[d] = xj[d] - xi[d];
+        du[d] = uj[d] - ui[d];
       }
-      vn = s.vol[jn];
+      double volj = s.vol[j];
+      const double rji = len3<DIM>(dx);
+      const double Sji = dot3<DIM>(dx, du) / dot3<DIM>(dx, dx);
+      const double Sc = rbar / sqrt(rji);
+      if (!((word >> (k & 31)) & 1u)) {
+        if (isGreater(rji, check_low)) volj *= div_by(check_up - rji, h, yh);
+        const double J = infJr<INF>(s, rji, horizon, yho);
+        brk = irrev && isGreater(fabs(Sji), fsc * Sc);
+        double ef = 0.;
+        if (!brk) ef = div_by(J * 4. * Sji * Cc * beta * exp(-beta * rji * Sji * Sji), invF, yF);
+        const double scalar_f = ef * volj;
+        const double yr = 1. / rji;
+        for (int d = 0; d < DIM; d++) term[d] = scalar_f * div_by(dx[d], rji, yr);
+      } else {
+        double y[3];
+        for (int d = 0; d < DIM; d++) y[d] = (xj[d] + uj[d]) - (xi[d] + ui[d]);
+        const double R = len3<DIM>(y);
+        double scalar_f = Kn * volj * (R - Rc) / R;
+        if (scalar_f > 0.) scalar_f = 0.;
+        for (int d = 0; d < DIM; d++) term[d] = scalar_f * y[d];
+      }
+      z = fabs(Sji / Sc);
     }
-    bool fs = (word >> (k & 31)) & 1u;
-    double dx[3], du[3];
-    for (int d = 0; d < DIM; d++) {
-      dx[d] = xj[d] - xi[d];
-      du[d] = uj[d] - ui[d];
+    wnew |= group_bits<LPN>(brk) << (k0 & 31);
+    for (int d = 0; d < DIM; d++) force[d] = group_add<LPN>(force[d], term[d]);
+    // running damage maximum (relative compare, list order): only values that
+    // pass the compare now can be stored in this round
+    for (unsigned up = group_bits<LPN>(isGreater(z, (double)Zi)); up; up &= up - 1u) {
+      const double zr = __shfl(z, __ffs(up) - 1, LPN);
+      if (isGreater(zr, (double)Zi)) Zi = (float)zr;
     }
-    const double rji = len3<DIM>(dx);
-    const double Sji = dot3<DIM>(dx, du) / dot3<DIM>(dx, dx);
-    const double Sc = rbar / sqrt(rji);
-    if (!fs) {
-      if (isGreater(rji, check_low)) volj *= (check_up - rji) / h;
-      const double J = infJ<INF>(s, 0., rji, horizon);
-      if (irrev && isGreater(fabs(Sji), fsc * Sc)) fs = true;
-      double ef = 0.;
-      if (!fs) ef = J * 4. * Sji * Cc * beta * exp(-beta * rji * Sji * Sji) / invF;
-      if (fs) wnew |= 1u << (k & 31);
-      const double scalar_f = ef * volj;
-      for (int d = 0; d < DIM; d++) force[d] += scalar_f * (dx[d] / rji);
-    } else {
-      double y[3];
-      for (int d = 0; d < DIM; d++) y[d] = (xj[d] + uj[d]) - (xi[d] + ui[d]);
-      const double R = len3<DIM>(y);
-      double scalar_f = Kn * volj * (R - Rc) / R;
-      if (scalar_f > 0.) scalar_f = 0.;
-      for (int d = 0; d < DIM; d++) force[d] += scalar_f * y[d];
-    }
-    if (isGreater(fabs(Sji / Sc), (double)Zi)) Zi = (float)fabs(Sji / Sc);
   }
+  if (sub != 0) return;
   if (n > 0 && wnew != word) bw[(int64_t)((n - 1) >> 5) * WAVE] = wnew;
   for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
   s.Z[i] = Zi;
@@ -1030,37 +1106,6 @@ __global__ void __launch_bounds__(256) k_pd_bond(DS s) {
   if (n > 0 && wnew != word) bw[(int64_t)((n - 1) >> 5) * WAVE] = wnew;
   for (int d = 0; d < DIM; d++) s.f[d][i] = force[d];
   s.Z[i] = Zi;
-}
-
-// ------------------------------------------- FP64 helpers of the bond loops
-// a / b rounded correctly from y = 1 / b rounded correctly: two corrections of
-// a y by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990: the first
-// leaves the quotient within an ulp, the second rounds it), 5 instructions
-// where a division of its own takes about 15.  For divisors that several
-// quotients share.
-__device__ __forceinline__ double div_by(double a, double b, double y) {
-  double q = a * y;
-  q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
-  return __builtin_fma(__builtin_fma(-b, q, a), y, q);
-}
-// value of lane R of the own group of four lanes (no LDS access)
-template <int R>
-__device__ __forceinline__ int quad_lane(int v) {
-  return __builtin_amdgcn_update_dpp(0, v, R * 0x55, 0xf, 0xf, true);
-}
-template <int R>
-__device__ __forceinline__ double quad_lane(double v) {
-  const long long b = __double_as_longlong(v);
-  const unsigned lo = (unsigned)quad_lane<R>((int)b), hi = (unsigned)quad_lane<R>((int)(b >> 32));
-  return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
-}
-// acc + the group's four terms in lane order (bonds in list order; lanes
-// without a term give 0, which adds nothing)
-__device__ __forceinline__ double quad_add(double acc, double t) {
-  acc += quad_lane<0>(t);
-  acc += quad_lane<1>(t);
-  acc += quad_lane<2>(t);
-  return acc + quad_lane<3>(t);
 }
 
 // The state-based FP64 passes deal a node's bonds to four neighboring lanes:
