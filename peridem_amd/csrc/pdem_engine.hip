@@ -427,13 +427,11 @@ struct Launch {
                        st, c->ds);
   }
   static void contact_force_kernel(pdem_ctx* c) {
-    // lane-per-node list (grid-stride); empty unless a rebuild ran with light_max > 0
-    if (c->light_used)
-      hipLaunchKernelGGL(k_contact_light<DIM>, dim3((unsigned)std::min<int64_t>(blocks(c->N), 1024)), dim3(TPB), 0,
-                         c->stream, c->ds);
+    // workgroups of the lane-per-node list (empty unless a rebuild ran with light_max > 0)
+    const int lb = c->light_used ? (int)std::min<int64_t>(blocks(c->N, CWAVES * WAVE), 1024) : 0;
     const int64_t waves = std::min<int64_t>(c->N, 8192);
-    hipLaunchKernelGGL(k_contact_force<DIM>, dim3((unsigned)((waves + CWAVES - 1) / CWAVES)),
-                       dim3(CWAVES * WAVE), 0, c->stream, c->ds);
+    hipLaunchKernelGGL(k_contact_force<DIM>, dim3((unsigned)(lb + (waves + CWAVES - 1) / CWAVES)),
+                       dim3(CWAVES * WAVE), 0, c->stream, c->ds, lb);
   }
   // fin 1: the damping pass finalises the nodes; 2: it leaves the
   // finalisation to the next node update (f_pending)

@@ -1679,11 +1679,11 @@ __device__ __forceinline__ void cand_pos(const DS& s, bool rec, int j, const dou
 constexpr int NACT = LIGHT_MAX_C;  // every candidate of a light node fits
 
 template <int DIM>
-__global__ void __launch_bounds__(256) k_contact_light(DS s) {
+__device__ void contact_light(const DS& s, int a0, int stride) {
   const int nl = (int)s.ctrl->nlight;
   const bool rec = !s.ctrl->rebuild;
   const double two_dsum = 2. * s.ctrl->dsum;
-  for (int a = (int)gid(); a < nl; a += gridDim.x * blockDim.x) {
+  for (int a = a0; a < nl; a += stride) {
     const int i = s.light[a];
     if (skin_far(s, i, two_dsum)) continue;
     const int n = s.ccount[i];
@@ -1774,23 +1774,30 @@ __global__ void __launch_bounds__(256) k_contact_light(DS s) {
 constexpr int CWAVES = 4;      // wavefronts per workgroup
 constexpr int MAXACT = 64;     // active pairs per node held in LDS
 
+// The first lblocks workgroups take the light nodes (contact_light), the
+// others the active list: the two are independent, and a launch of its own
+// costs 4 us of every step.
 // (at most 128 VGPRs: 4 wavefronts per SIMD; the kernel waits on chains of
 // dependent gathers, and 3 wavefronts per SIMD took 28 % longer)
 template <int DIM>
-__global__ void __launch_bounds__(CWAVES * WAVE, 4) k_contact_force(DS s) {
+__global__ void __launch_bounds__(CWAVES * WAVE, 4) k_contact_force(DS s, int lblocks) {
   __shared__ int sj[CWAVES][MAXACT];
   __shared__ double st[CWAVES][MAXACT][6];
   // this rebuild's query is done: leave the cell table empty for the next
   if (s.ctrl->rebuild) clear_cells(s, gid(), (int64_t)gridDim.x * blockDim.x);
+  if ((int)blockIdx.x < lblocks) {
+    contact_light<DIM>(s, (int)gid(), lblocks * CWAVES * WAVE);
+    return;
+  }
   const int lane = threadIdx.x & (WAVE - 1);
   const int wv = threadIdx.x / WAVE;
-  const int nwaves = gridDim.x * CWAVES;
+  const int nwaves = ((int)gridDim.x - lblocks) * CWAVES;
   const int nact_nodes = (int)s.ctrl->nactive;
   const bool rec = !s.ctrl->rebuild;
   const double two_dsum = 2. * s.ctrl->dsum;
   // the skin test for the wavefront's next 64 nodes at once (a lane each),
   // then the nodes that pass it one after the other, in the same order
-  for (int a0 = blockIdx.x * CWAVES + wv; a0 < nact_nodes; a0 += WAVE * nwaves) {
+  for (int a0 = ((int)blockIdx.x - lblocks) * CWAVES + wv; a0 < nact_nodes; a0 += WAVE * nwaves) {
     const int al = a0 + lane * nwaves;
     int il = 0;
     bool near = false;
