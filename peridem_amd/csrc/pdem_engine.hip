@@ -67,7 +67,7 @@ __global__ void k_zero_u32(unsigned* p, int n) {
 }  // namespace
 
 // multi-particle models up to this many nodes use the fused step kernels
-constexpr int64_t LIGHT_2D_MIN_NODES = int64_t(1) << 20;  // 2D models from this size use the light-node contact kernel
+constexpr int64_t LIGHT_2D_MIN_NODES = int64_t(1) << 17;  // 2D models from this size use the light-node contact kernel
 constexpr int64_t FUSE_MAX_NODES = (int64_t)1 << 20;
 
 struct pdem_ctx {
@@ -1278,10 +1278,10 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     s.cdmin = c->dalloc<float>(N, false);
     s.n_ubc_sets = (int)c->ubc.size();
     // a lane per node for nodes with few candidates pays off where many nodes
-    // have candidates (3D, and large 2D models such as batched ensembles:
-    // 0.66 -> 0.60 ms per step for 512 instances); a small 2D model with few
-    // contacts does better with the wavefront-per-node kernel alone (one
-    // launch less per step: 87 -> 79 us for the 500-particle compressive test)
+    // have candidates: 3D, and 2D models from LIGHT_2D_MIN_NODES on (step of
+    // 4.2M nodes 660 -> 600 us, 412k 105 -> 102, 191k 85.7 -> 84.9, 166k 59 ->
+    // 58); in smaller 2D models a wavefront per node hides its loads better
+    // (51k nodes in violent motion: 130 us against 141 with lanes)
     s.light_max = (dim == 3 || N >= LIGHT_2D_MIN_NODES) ? LIGHT_MAX_C : 0;
     c->light_used = s.light_max > 0;
     s.nblockmax = (int)blocks(N);
