@@ -884,6 +884,16 @@ __device__ __forceinline__ double quad_add(double acc, double t) {
   return acc + quad_lane<3>(t);
 }
 
+// n nodes' components as x y z x y z ... (z 0 without a third component)
+constexpr int64_t PACK_NODES = int64_t(1) << 17;
+__global__ void k_pack3(const double* x, const double* y, const double* z, int64_t n, double* out) {
+  const int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (e >= 3 * n) return;
+  const int64_t i = e / 3;
+  const double* a = e % 3 == 0 ? x : (e % 3 == 1 ? y : z);
+  out[e] = a ? a[i] : 0.;
+}
+
 // -------------------------------------------------------- PD bond forces
 template <int INF>
 __device__ __forceinline__ double infJ(const DS& s, double r_over_delta, double rji, double horizon) {
