@@ -67,6 +67,14 @@ __global__ void k_zero_u32(unsigned* p, int n) {
 }  // namespace
 
 // multi-particle models up to this many nodes use the fused step kernels
+// Up to this size the cell list's kernels follow the bond forces on the
+// engine's queue.  Beside them on a side stream, the fork, the three kernels
+// and the join take about 36 us of a step, more than the bond forces of a
+// small model; in line they cost about 10 us on the steps that rebuild nothing
+// (2D bed of 37k nodes 56 -> 46 us per step, 59k 56 -> 50, 98k equal, 191k 84
+// -> 86; ensemble of 28k nodes 43 -> 38; 3D packing of 41k nodes 71 -> 68, 77k
+// 87 -> 91).
+constexpr int64_t CELLS_INLINE_NODES = int64_t(1) << 16;
 constexpr int64_t LIGHT_2D_MIN_NODES = int64_t(1) << 17;  // 2D models from this size use the light-node contact kernel
 constexpr int64_t FUSE_MAX_NODES = (int64_t)1 << 20;
 
@@ -401,20 +409,26 @@ struct Launch {
     hipLaunchKernelGGL(k_cells_scatter<DIM>, dim3((unsigned)std::min<int64_t>(blocks(c->N, CELL_TPB), 1024)),
                        dim3(CELL_TPB), 0, st, c->ds);
   }
-  // PD forces and, on a rebuild step, the cell list on the second side stream
-  // beside them (joined before the candidate query).  The fork point is
+  // PD forces and, on a rebuild step, the cell list and the candidate query;
+  // large models run these on the second side stream beside the PD kernels,
+  // which touch nothing of them (the query in line after the join: 2D bed of
+  // 191k nodes 84.6 us per step, beside 82.0; 3D packing of 77k 86 and 82;
+  // 48 ensemble instances 83 and 80).  The fork point is
   // recorded first and the PD kernels are enqueued before the cell kernels:
   // the same dependencies, and a captured graph keeps the PD chain on the
   // engine's queue.
   static void pd_forces_and_cells(pdem_ctx* c) {
-    if (!c->multi || c->ds.cells_in_ctrl) {
+    if (!c->multi || c->ds.cells_in_ctrl || c->N <= CELLS_INLINE_NODES) {
       pd_forces(c);
+      if (c->multi && !c->ds.cells_in_ctrl) cells_build(c, c->stream);
+      if (c->multi) rebuild_lists(c, c->stream);
       return;
     }
     HIPCHK(hipEventRecord(c->ev_fork2, c->stream));
     pd_forces(c);
     HIPCHK(hipStreamWaitEvent(c->side2, c->ev_fork2, 0));
     cells_build(c, c->side2);
+    rebuild_lists(c, c->side2);
     HIPCHK(hipEventRecord(c->ev_join2, c->side2));
     HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join2, 0));
   }
@@ -423,7 +437,7 @@ struct Launch {
     hipStream_t st = c->stream;
     hipLaunchKernelGGL(k_ctrl<DIM>, dim3(CTRL_BLOCKS), dim3(1024), 0, st, c->ds, 0);
     if (!c->ds.cells_in_ctrl) cells_build(c, st);
-    rebuild_lists(c);
+    rebuild_lists(c, st);
     hipLaunchKernelGGL(k_cells_init, dim3((unsigned)std::min<int64_t>(blocks(c->ds.ncells), 4096)), dim3(TPB), 0,
                        st, c->ds);
   }
@@ -473,10 +487,10 @@ struct Launch {
   // in length, and more wavefronts in flight hide their latency; the launch
   // of other steps, which returns at once, costs under 1 us more than a
   // capped grid) and damping partner lists in one launch
-  static void rebuild_lists(pdem_ctx* c) {
+  static void rebuild_lists(pdem_ctx* c, hipStream_t st) {
     const int qb = (int)blocks(c->N);
     const int db = (int)std::min<int64_t>((std::max(c->ds.n_nonwall, 1) + 3) / 4, 1024);
-    hipLaunchKernelGGL(k_rebuild_lists<DIM>, dim3((unsigned)(qb + db)), dim3(TPB), 0, c->stream, c->ds, db);
+    hipLaunchKernelGGL(k_rebuild_lists<DIM>, dim3((unsigned)(qb + db)), dim3(TPB), 0, st, c->ds, db);
   }
   // closure pairs: connections (rebuild steps), modes, network, patch
   // records (2D, closure mode only)
@@ -521,7 +535,6 @@ struct Launch {
     const bool fin = fuse_finalize(c);
     const bool defer = defer_finalize(c, verlet);
     if (c->multi) {
-      rebuild_lists(c);
       closure(c);
       contact_force_kernel(c);
       damping(c, fin ? 1 : (defer ? 2 : 0));
