@@ -130,6 +130,7 @@ struct pdem_ctx {
   bool graph_verlet = false;  // the captured step is integrateVerlet
   // bond-based RNP pair-tile kernel (FP64, all force-computing particles RNP)
   RnpTileArgs rt{};
+  bool lists_in_rnp = false;  // this RNP pass's launch also takes the candidate query (set around it)
   bool rnp_tile = false;  // use it (by size, RNP_TILE_NODES; autotuned)
   bool nf_zeroed = false;  // inside a step whose node update zeroed f of the non-force nodes
   int step_fusion = 1;  // fused step kernels: 0 never, 1 models up to FUSE_MAX_NODES, 2 any size
@@ -355,10 +356,19 @@ struct Launch {
   // lanes per node of the lane-group RNP kernel (RNP16_NODES)
   template <int INF>
   static void rnp(pdem_ctx* c, int tpb) {
-    if (c->N <= RNP16_NODES)
-      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 16>), dim3(blocks(c->N * 16, tpb)), dim3(tpb), 0, c->stream, c->ds);
-    else
-      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 4>), dim3(blocks(c->N * 4, tpb)), dim3(tpb), 0, c->stream, c->ds);
+    const int lpn = c->N <= RNP16_NODES ? 16 : 4;
+    const unsigned nb = blocks(c->N * lpn, tpb);
+    if (lpn == 16) {
+      const unsigned db = c->lists_in_rnp ? list_dblocks(c, tpb) : 0, qb = c->lists_in_rnp ? blocks(c->N, tpb) : 0;
+      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 16>), dim3(nb + db + qb), dim3(tpb), 0, c->stream, c->ds, (int)nb, (int)db);
+    } else {
+      hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 4>), dim3(nb), dim3(tpb), 0, c->stream, c->ds, (int)nb, 0);
+    }
+  }
+  // workgroups of the damping partner lists (a wavefront per particle)
+  static unsigned list_dblocks(pdem_ctx* c, int tpb) {
+    const int w = tpb / WAVE;
+    return (unsigned)std::min<int64_t>((std::max(c->ds.n_nonwall, 1) + w - 1) / w, 1024);
   }
   template <int INF>
   static void pd_inf(pdem_ctx* c) {
@@ -419,9 +429,14 @@ struct Launch {
   // engine's queue.
   static void pd_forces_and_cells(pdem_ctx* c) {
     if (!c->multi || c->ds.cells_in_ctrl || c->N <= CELLS_INLINE_NODES) {
+      // (FP64 RNP models whose cell list is there: the query rides in the bond pass's launch)
+      c->lists_in_rnp = c->multi && c->ds.cells_in_ctrl && c->N <= RNP16_NODES && c->rnp_any && !c->rnp_tile &&
+                        !(c->precision == PDEM_PREC_MIXED && c->ntiles > 0);
+      const bool done = c->lists_in_rnp;
       pd_forces(c);
+      c->lists_in_rnp = false;
       if (c->multi && !c->ds.cells_in_ctrl) cells_build(c, c->stream);
-      if (c->multi) rebuild_lists(c, c->stream);
+      if (c->multi && !done) rebuild_lists(c, c->stream);
       return;
     }
     HIPCHK(hipEventRecord(c->ev_fork2, c->stream));
@@ -489,7 +504,7 @@ struct Launch {
   // capped grid) and damping partner lists in one launch
   static void rebuild_lists(pdem_ctx* c, hipStream_t st) {
     const int qb = (int)blocks(c->N);
-    const int db = (int)std::min<int64_t>((std::max(c->ds.n_nonwall, 1) + 3) / 4, 1024);
+    const int db = (int)list_dblocks(c, TPB);
     hipLaunchKernelGGL(k_rebuild_lists<DIM>, dim3((unsigned)(qb + db)), dim3(TPB), 0, st, c->ds, db);
   }
   // closure pairs: connections (rebuild steps), modes, network, patch
