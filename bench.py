@@ -81,7 +81,8 @@ def pd_bytes_per_launch(spec, eng, precision):
                                                                    bond and the 4-byte pair entry)
         mixed state-based passes           24 d + 36 + 4.375 N_i (theta written, degree, thread slot;
                                                                    the 2-byte ids and the bond words
-                                                                   read by both passes)
+                                                                   read by both passes; particles of
+                                                                   one mesh share their ids in L2)
     Returns (bytes in this build's layout, canonical bytes, mean N_i)."""
     import numpy as np
     from peridem_amd import capi
@@ -122,7 +123,7 @@ def kernel_names(spec, eng, prec):
     state = any(p["material_type"] == capi.MAT_PDSTATE and p["compute_force"] for p in spec.particles)
     if prec == capi.PREC_MIXED and state:
         return ("k_mixed_state (+ k_mixed_dilation, k_mixed_force of open tiles)", "mixed_state",
-                "FP32 VALU issue (about one wave instruction per CU cycle, 57 per bond and pass)")
+                "FP32 VALU issue (about one wave instruction per CU cycle, about 42 per bond in the first pass, 14 in the second)")
     if state:
         return "k_pd_dilation + k_pd_state", "pd_state", "FP64 VALU"
     if eng.launch_config()[0] == 512:
