@@ -122,6 +122,7 @@ struct pdem_ctx {
   uint32_t* d_lnode = nullptr;
   int* d_lslice = nullptr;
   size_t col16_cap = 0, wgt_cap = 0, lnode_cap = 0, lslice_cap = 0;
+  int64_t n_lists = 0, n_list_entries = 0;
   // learned pair-contact closure
   bool cl_ready = false;        // closure data allocated (pdem_closure_setup)
   ClosureArgs ca{};
@@ -857,6 +858,8 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
     c->mixed.col16 = c->d_col16;
     c->mixed.wgt = c->d_wgt;
     c->mixed.geom = lds_data > GEOM_MIN_ENTRIES && s.inf_type != 2 ? 1 : 0;
+    c->n_lists = (int64_t)which.size();
+    c->n_list_entries = data;
     const dim3 gw((unsigned)which.size());
     dispatch(
         c,
@@ -2478,6 +2481,15 @@ int pdem_get_tile_counts(pdem_ctx* c, int32_t* lds_tiles, int32_t* hbm_tiles) {
     if (!lds_tiles || !hbm_tiles) throw HipError{"null output pointer"};
     *lds_tiles = c->mixed.ntiles_closed + c->mixed.ntiles_lds;
     *hbm_tiles = c->mixed.ntiles_hbm;
+  });
+}
+
+int pdem_get_list_info(pdem_ctx* c, int64_t* lists, int64_t* entries, int32_t* evaluated) {
+  return guarded(c, [&] {
+    if (!lists || !entries || !evaluated) throw HipError{"null output pointer"};
+    *lists = c->n_lists;
+    *entries = c->n_list_entries;
+    *evaluated = c->mixed.geom;
   });
 }
 

@@ -168,7 +168,8 @@ __device__ __forceinline__ int block_id(const uint4& b, int t) {
 //
 // LDS records, 16 bytes each, per window node:
 //   lx  twice the FP32 position offset from the particle's first reference
-//       node, and the volume            (first pass; with GEOM both passes)
+//       node, and the volume over particle_scale
+//                                       (first pass; with GEOM both passes)
 //   lq  the displacement relative to the particle's first node in fixed
 //       point (three int32 in units of a power-of-two step `us` chosen per
 //       particle so that every value stays below 2^29 in magnitude), and the
@@ -197,13 +198,14 @@ struct Win {
   int gs;    // particle's first node
   int ws;    // window start
   float us;  // fixed-point step of the displacement records (1 for HBM tiles)
+  double inv_scale;  // 1 / particle_scale
   double org[3];
   __device__ __forceinline__ int entry(int i) const { return LDS ? (i - ws) * 16 : i - gs; }
   __device__ __forceinline__ float4 x2(int e) const {
     if (LDS) return *(const float4*)(lx + e);
     const int64_t j = gs + e;
     return make_float4(2.f * (float)(s->xr[0][j] - org[0]), 2.f * (float)(s->xr[1][j] - org[1]),
-                       DIM == 3 ? 2.f * (float)(s->xr[2][j] - org[2]) : 0.f, (float)s->vol[j]);
+                       DIM == 3 ? 2.f * (float)(s->xr[2][j] - org[2]) : 0.f, (float)(s->vol[j] * inv_scale));
   }
   // the node's own displacement record (fixed point) or displacement (FP64)
   struct Own {
@@ -289,7 +291,8 @@ __global__ void __launch_bounds__(256) k_mixed_umax(DS s, MixedArgs m) {
 // Returns us.
 template <int DIM, bool FIRST, bool SECOND, bool GEOM>
 __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, const DevTile& t, float4* lx,
-                                              int4* lq, float4* ly, const double* org, float* red) {
+                                              int4* lq, float4* ly, const double* org, double inv_scale,
+                                              float* red) {
   const int nw = t.we - t.ws;
   const int gs = (int)s.P[t.pid].glob_start;
   double u0[3] = {0., 0., 0.};
@@ -298,7 +301,8 @@ __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, c
     const int j = t.ws + q;
     double xd[3] = {0., 0., 0.};
     for (int d = 0; d < DIM; d++) xd[d] = s.xr[d][j] - org[d];
-    if (FIRST || GEOM) lx[q] = make_float4(2.f * (float)xd[0], 2.f * (float)xd[1], 2.f * (float)xd[2], (float)s.vol[j]);
+    if (FIRST || GEOM)
+      lx[q] = make_float4(2.f * (float)xd[0], 2.f * (float)xd[1], 2.f * (float)xd[2], (float)(s.vol[j] * inv_scale));
     if (SECOND) {
       float y[3] = {0.f, 0.f, 0.f};
       for (int d = 0; d < DIM; d++) y[d] = (float)(xd[d] + (s.u[d][j] - u0[d]));
@@ -339,29 +343,31 @@ struct StateConsts {
   float thr4;      // |S| / 4 > thr4: the bond breaks (isGreater(|S|, s0 + 1e-10))
   float inv_s0, Kn, Rc;
   double K, G, scale;
-  // GEOM: J / scale = ja + jb r2 (constant and linear influence functions),
-  // volume correction up_h - r2 inv_h2 where r2 > low2
+  // GEOM: J = ja + jb r2 (constant and linear influence functions), volume
+  // correction up_h - r2 inv_h2 where r2 > low2
   float ja, jb, low2, inv_h2, up_h;
   __device__ StateConsts(const DS& s, const DevParticle& p) {
     thr4 = uniform(0.25f * ((float)(p.mat[2] + 1.0e-10) / REL_KEEP));
     inv_s0 = (float)(1.0 / p.mat[2]);
-    Kn = (float)p.Kn;
     Rc = (float)p.Rc;
     K = p.mat[0];
     G = p.mat[1];
     scale = particle_scale(s, p);
-    const double inv = 1. / scale;
-    ja = uniform((float)(s.inf_p0 * inv));
-    jb = uniform(s.inf_type == 1 ? (float)(0.5 * s.inf_p1 / p.horizon * inv) : 0.f);
+    Kn = (float)(p.Kn * scale);
+    ja = uniform((float)s.inf_p0);
+    jb = uniform(s.inf_type == 1 ? (float)(0.5 * s.inf_p1 / p.horizon) : 0.f);
     low2 = uniform(2.f * ((float)(p.horizon - 0.5 * p.h) / REL_KEEP));
     inv_h2 = uniform((float)(0.5 / p.h));
     up_h = uniform((float)((p.horizon + 0.5 * p.h) / p.h));
   }
   // GEOM: the weight 2 r J V^c / scale of a bond of length r2 / 2 whose
-  // neighbor has volume v.  The correction is 1 at the distance horizon - h/2
-  // from which it applies, so clamping it to [0, 1], which the multiply-add
-  // does for nothing, saves the compare and the select (EXACT) for every bond
-  // but those in the slack of the reference's compare (see slack_bond).
+  // neighbor has volume v scale.  The padding's length (Win) makes J a large
+  // number, but a finite one in any unit of length: the scale, which goes with
+  // the fourth power of the mesh size, is in v, which is 0 there.  The
+  // correction is 1 at the distance horizon - h/2 from which it applies, so
+  // clamping it to [0, 1], which the multiply-add does for nothing, saves the
+  // compare and the select (EXACT) for every bond but those in the slack of
+  // the reference's compare (see slack_bond).
   template <bool EXACT>
   __device__ __forceinline__ float weight(float r2, float v) const {
 #pragma clang fp contract(fast)
@@ -507,7 +513,7 @@ __device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const Stat
       o.theta += (double)(b.c2 * wj);
       sf = p * wj * (own.a + aj) * b.inv_l2;
     } else {
-      // Kn V (|y| - Rc) y / |y| where it repels
+      // Kn V (|y| - Rc) y / |y| where it repels (Kn with the scale of vj)
       sf = c.Kn * vj * (0.5f * b.l2 - c.Rc) * b.inv_l2;
       if (sf > 0.f) sf = 0.f;
     }
@@ -726,7 +732,8 @@ __device__ __forceinline__ int slot_rounds(const MixedArgs& m, const DevTile& t)
   __shared__ float4 ly[(LDS_ON) && (SECOND) ? (NODES) + 1 : 1]; \
   __shared__ float red[1024 / WAVE];
 #define PDEM_WINDOW(DIM, LDS_ON, t, gs) \
-  Win<DIM, LDS_ON> w{(const char*)lx, (const char*)lq, (const char*)ly, &s, &m, gs, t.ws, 1.f, {0., 0., 0.}}; \
+  Win<DIM, LDS_ON> w{(const char*)lx, (const char*)lq, (const char*)ly, &s, &m, gs, t.ws, 1.f, \
+                      1. / particle_scale(s, p), {0., 0., 0.}}; \
   for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
 
 // First pass of the open tiles (tiles that do not hold a whole particle:
@@ -738,7 +745,7 @@ __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_dilation(DS
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, LDS, t, gs)
-  if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
   const StateConsts c(s, p);
   const int nr = slot_rounds<LDS, LPN>(m, t);
   for (int it = 0; it < nr; it++) {
@@ -758,7 +765,7 @@ __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_force(DS s,
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, LDS, t, gs)
-  if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
   const StateConsts c(s, p);
   const int nr = slot_rounds<LDS, LPN>(m, t);
   for (int it = 0; it < nr; it++) {
@@ -778,7 +785,7 @@ __global__ void __launch_bounds__(TPB, TPB == 512 ? 6 : MIXED_WAVES_PER_SIMD) k_
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, true, t, gs)
-  w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, red);
+  w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
   const StateConsts c(s, p);
   const int nr = slot_rounds<true, 1>(m, t);
   for (int it = 0; it < nr; it++) {
