@@ -946,7 +946,7 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
     std::sort(open.begin(), open.end());
     open.erase(std::unique(open.begin(), open.end()), open.end());
     if (!c->mixed.open_pids) c->mixed.open_pids = c->dalloc<int>(std::max(1, c->np));
-    if (!c->mixed.pumax) c->mixed.pumax = c->dalloc<float>(std::max(1, c->np));
+    if (!c->mixed.pmax) c->mixed.pmax = c->dalloc<float4>(std::max(1, c->np));
     if (!open.empty())
       HIPCHK(hipMemcpy((void*)c->mixed.open_pids, open.data(), open.size() * sizeof(int), hipMemcpyHostToDevice));
     c->mixed.n_open_pids = (int)open.size();

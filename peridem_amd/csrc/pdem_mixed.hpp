@@ -105,11 +105,11 @@ struct MixedArgs {
   int geom;
   const float* fa;        // per node 2 alpha particle_scale, alpha = 15 G / m (constant, from set-up)
   float* fb;              // per node b particle_scale, b = theta ((3K/m) - alpha / 3), of the open tiles
-  // particles with open LDS tiles: max |u - u(first node)| over the particle
-  // (rounded up to float), for the fixed-point step of their windows
+  // particles with open LDS tiles: particle_max over the particle, for the
+  // fixed-point steps of their windows
   const int* open_pids;
   int n_open_pids;
-  float* pumax;           // [np]
+  float4* pmax;           // [np]
 };
 
 // The bond weights are read from the lists while the lists of the LDS tiles
@@ -174,19 +174,35 @@ __device__ __forceinline__ int block_id(const uint4& b, int t) {
 //       point (three int32 in units of a power-of-two step `us` chosen per
 //       particle so that every value stays below 2^29 in magnitude), and the
 //       node's alpha term (MixedArgs::fa)                     (first pass)
-//   ly  the FP32 current position relative to that of the particle's first
-//       node, and the node's b term                           (second pass)
+//   ly  the current position relative to that of the particle's first node,
+//       in FP32 or, where that would cost accuracy, in fixed point (as lq,
+//       with a step of its own), and the node's b term        (second pass)
 // A bond's relative displacement is the exact integer difference of two lq
 // records, rounded once to FP32 and scaled by us (exact): as accurate as
 // rounding the FP64 difference to FP32, plus a quantisation of 2^-29 of the
 // particle's largest relative displacement.  HBM tiles read the FP64 arrays
 // (us = 1).
 //
+// The second pass takes only the direction of the current bond vector, the
+// difference of two ly records.  While the particle is about as large as at
+// the start (FIXED_FROM), FP32 positions are as accurate as the reference
+// positions, which are FP32 throughout.  When its parts have flown apart
+// they are not (sphere of 1021 nodes in two halves 1 m apart, strain 0.2: RMS
+// force error 2.0e-5 of the largest force, 4.4e-6 in fixed point, which is the
+// error of the displacement records), and the tile takes fixed point.  Fixed
+// point throughout costs three conversions a bond: packing of 2000 spheres 3 %
+// of the step, 512-instance ensemble 1.6 %.
+//
 // The record after the window's last node (offset 16 (we - ws)) stands for
 // the list padding: a position so far off that its bond has no stretch, and
 // weight 0, so the entries that fill up a lane's last block add nothing and
 // the block loops need no test per bond.
 constexpr float PAD_POS = 1.0e18f;
+constexpr int PAD_Q = 1 << 30;  // its current position in fixed point (the nodes' are below 2^29)
+// fixed point from this ratio of the largest component of the current
+// positions to that of the reference positions on (a round body that turns
+// stays at 1, a box reaches 1.7)
+constexpr float FIXED_FROM = 1.25f;
 
 template <int DIM, bool LDS>
 struct Win {
@@ -240,87 +256,140 @@ struct Win {
       aj = m->fa[gs + e];
     }
   }
-  // current position relative to the particle's first node, and the b term
-  __device__ __forceinline__ float4 yb(int e) const {
-    if (LDS) return *(const float4*)(ly + e);
-    const int64_t j = gs + e;
-    float y[3] = {0.f, 0.f, 0.f};
-    for (int d = 0; d < DIM; d++) y[d] = (float)((s->xr[d][j] - org[d]) + (s->u[d][j] - s->u[d][gs]));
-    return make_float4(y[0], y[1], y[2], m->fb[j]);
+  // the node's own current position relative to the particle's first node
+  // (FP32, fixed point or, HBM tiles, FP64) and its b term
+  struct Cur {
+    int4 r;
+    double y[3];
+  };
+  __device__ __forceinline__ double pos(int64_t j, int d) const {
+    return (s->xr[d][j] - org[d]) + (s->u[d][j] - s->u[d][gs]);
+  }
+  __device__ __forceinline__ Cur cur(int e) const {
+    Cur o{};
+    if (LDS) {
+      o.r = *(const int4*)(ly + e);
+    } else {
+      for (int d = 0; d < DIM; d++) o.y[d] = pos(gs + e, d);
+      o.r.w = __float_as_int(m->fb[gs + e]);
+    }
+    return o;
+  }
+  // current bond vector to neighbor e (in the unit of the records) and the
+  // sum of the b terms
+  template <bool FIXED>
+  __device__ __forceinline__ void dy(int e, const Cur& o, float* out, float& b) const {
+    float bj;
+    if (LDS) {
+      const int4 r = *(const int4*)(ly + e);
+      auto diff = [](int x, int y) { return FIXED ? (float)(x - y) : __int_as_float(x) - __int_as_float(y); };
+      out[0] = diff(r.x, o.r.x);
+      out[1] = diff(r.y, o.r.y);
+      if (DIM == 3) out[2] = diff(r.z, o.r.z);
+      bj = __int_as_float(r.w);
+    } else {
+      for (int d = 0; d < DIM; d++) out[d] = (float)(pos(gs + e, d) - o.y[d]);
+      bj = m->fb[gs + e];
+    }
+    b = __int_as_float(o.r.w) + bj;
   }
 };
 
-// max |u - u(particle's first node)| over nodes [n0, n1) of the workgroup's
-// threads, as a float rounded up (the fixed-point step only has to bound it);
-// the maximum does not depend on the order, so every tile of a particle gets
-// the same value
-template <int DIM>
-__device__ __forceinline__ float particle_umax(const DS& s, int gs, int n0, int n1, float* red) {
-  double u0[3] = {0., 0., 0.};
-  for (int d = 0; d < DIM; d++) u0[d] = s.u[d][gs];
-  double mx = 0.;
-  for (int j = n0 + (int)threadIdx.x; j < n1; j += blockDim.x)
-    for (int d = 0; d < DIM; d++) mx = fmax(mx, fabs(s.u[d][j] - u0[d]));
-  float mf = (float)(mx * (1.0 + 0x1p-20));
-  for (int o = WAVE / 2; o > 0; o >>= 1) mf = fmaxf(mf, __shfl_xor(mf, o));
-  if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = mf;
-  __syncthreads();
-  mf = 0.f;
-  for (int w = 0; w < (int)(blockDim.x / WAVE); w++) mf = fmaxf(mf, red[w]);
-  __syncthreads();
-  return mf;
-}
+// Largest components over a particle's nodes, relative to its first node: the
+// displacement, the current and the reference position
+struct PartMax {
+  double u = 0., y = 0., x = 0.;
+  template <int DIM>
+  __device__ __forceinline__ void node(const double* xd, const double* du) {
+    for (int d = 0; d < DIM; d++) {
+      u = fmax(u, fabs(du[d]));
+      y = fmax(y, fabs(xd[d] + du[d]));
+      x = fmax(x, fabs(xd[d]));
+    }
+  }
+  // the workgroup's maxima as floats rounded up (the fixed-point steps only
+  // have to bound them); they do not depend on the order, so every tile of a
+  // particle gets the same values
+  __device__ __forceinline__ float4 group(float4* red) const {
+    auto up = [](double a) { return (float)(a * (1.0 + 0x1p-20)); };
+    float4 m = make_float4(up(u), up(y), up(x), 0.f);
+    auto join = [&](float a, float b, float c) {
+      m = make_float4(fmaxf(m.x, a), fmaxf(m.y, b), fmaxf(m.z, c), 0.f);
+    };
+    for (int o = WAVE / 2; o > 0; o >>= 1) join(__shfl_xor(m.x, o), __shfl_xor(m.y, o), __shfl_xor(m.z, o));
+    if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = m;
+    __syncthreads();
+    for (int w = 0; w < (int)(blockDim.x / WAVE); w++) join(red[w].x, red[w].y, red[w].z);
+    return m;
+  }
+};
 
-// the maximum for the particles with open LDS tiles: one workgroup each
+// the maxima of the particles with open LDS tiles: one workgroup each
 template <int DIM>
 __global__ void __launch_bounds__(256) k_mixed_umax(DS s, MixedArgs m) {
-  __shared__ float red[256 / WAVE];
+  __shared__ float4 red[256 / WAVE];
   const int pid = m.open_pids[blockIdx.x];
   const DevParticle& p = s.P[pid];
-  const float mf = particle_umax<DIM>(s, (int)p.glob_start, (int)p.glob_start, (int)p.glob_end, red);
-  if (threadIdx.x == 0) m.pumax[pid] = mf;
+  const int64_t gs = p.glob_start;
+  PartMax mx;
+  for (int64_t j = gs + threadIdx.x; j < p.glob_end; j += blockDim.x) {
+    double xd[3], du[3];
+    for (int d = 0; d < DIM; d++) {
+      xd[d] = s.xr[d][j] - s.xr[d][gs];
+      du[d] = s.u[d][j] - s.u[d][gs];
+    }
+    mx.node<DIM>(xd, du);
+  }
+  const float4 mf = mx.group(red);
+  if (threadIdx.x == 0) m.pmax[pid] = mf;
+}
+
+// the smallest power of two 2^e with mf / 2^e < 2^29 (e >= -126: a window at
+// rest keeps all zeros)
+__device__ __forceinline__ int fixed_exp(float mf) {
+  if (!(mf > 0.f)) return -126;
+  int ex;
+  frexpf(mf, &ex);  // mf < 2^ex
+  return ex - 29 > -126 ? ex - 29 : -126;
 }
 
 // Stage a tile's window in LDS: the records that the pass (or, FIRST and
-// SECOND, both passes) reads.  The fixed-point step us is the smallest power
-// of two with max |u - u_first| / us < 2^29 over the whole particle, so that
-// the records, and the results, do not depend on the tile shape; a closed
-// tile (the whole particle) takes the maximum over its window, an open tile
-// reads it from k_mixed_umax.  The b terms of the fused kernel are written by
-// its first pass; those of an open tile come from the other kernel.
-// Returns us.
+// SECOND, both passes) reads.  The fixed-point steps come from the largest
+// values of the whole particle, so that the records, and the results, do not
+// depend on the tile shape; a closed tile (the whole particle) takes them over
+// its window, an open tile reads them from k_mixed_umax.  The b terms of the
+// fused kernel are written by its first pass; those of an open tile come from
+// the other kernel.
+// Returns the displacements' step us; fixed: ly is in fixed point.
 template <int DIM, bool FIRST, bool SECOND, bool GEOM>
 __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, const DevTile& t, float4* lx,
-                                              int4* lq, float4* ly, const double* org, double inv_scale,
-                                              float* red) {
+                                              int4* lq, int4* ly, const double* org, double inv_scale,
+                                              float4* red, bool& fixed) {
   const int nw = t.we - t.ws;
   const int gs = (int)s.P[t.pid].glob_start;
   double u0[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) u0[d] = s.u[d][gs];
+  const bool closed = t.lds == 2;
+  PartMax mx;
   for (int q = threadIdx.x; q < nw; q += blockDim.x) {
     const int j = t.ws + q;
-    double xd[3] = {0., 0., 0.};
+    double xd[3] = {0., 0., 0.}, du[3] = {0., 0., 0.};
     for (int d = 0; d < DIM; d++) xd[d] = s.xr[d][j] - org[d];
     if (FIRST || GEOM)
       lx[q] = make_float4(2.f * (float)xd[0], 2.f * (float)xd[1], 2.f * (float)xd[2], (float)(s.vol[j] * inv_scale));
-    if (SECOND) {
-      float y[3] = {0.f, 0.f, 0.f};
-      for (int d = 0; d < DIM; d++) y[d] = (float)(xd[d] + (s.u[d][j] - u0[d]));
-      ly[q] = make_float4(y[0], y[1], y[2], FIRST ? 0.f : m.fb[j]);
+    if (closed || SECOND) {
+      for (int d = 0; d < DIM; d++) du[d] = s.u[d][j] - u0[d];
+      if (closed) mx.node<DIM>(xd, du);
     }
+    if (SECOND)
+      ly[q] = make_int4(__float_as_int((float)(xd[0] + du[0])), __float_as_int((float)(xd[1] + du[1])),
+                        __float_as_int((float)(xd[2] + du[2])), FIRST ? 0 : __float_as_int(m.fb[j]));
   }
-  float us = 1.f;
+  const float4 mf = closed ? mx.group(red) : m.pmax[t.pid];
+  fixed = __builtin_amdgcn_readfirstlane(mf.y > FIXED_FROM * mf.z);
+  const int eu = fixed_exp(mf.x);
   if (FIRST) {
-    const float mf = t.lds == 2 ? particle_umax<DIM>(s, gs, t.ws, t.we, red) : m.pumax[t.pid];
-    // us = 2^e with mf / us < 2^29 (e >= -126: a window at rest keeps all zeros)
-    int e = -126;
-    if (mf > 0.f) {
-      int ex;
-      frexpf(mf, &ex);  // mf < 2^ex
-      e = ex - 29 > -126 ? ex - 29 : -126;
-    }
-    us = ldexpf(1.f, e);
-    const double inv_us = ldexp(1., -e);
+    const double inv_us = ldexp(1., -eu);
     for (int q = threadIdx.x; q < nw; q += blockDim.x) {
       const int j = t.ws + q;
       int qq[3] = {0, 0, 0};
@@ -328,13 +397,23 @@ __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, c
       lq[q] = make_int4(qq[0], qq[1], qq[2], __float_as_int(m.fa[j]));
     }
   }
+  if (SECOND && fixed) {
+    const double inv_ys = ldexp(1., -fixed_exp(mf.y));
+    for (int q = threadIdx.x; q < nw; q += blockDim.x) {
+      const int j = t.ws + q;
+      int yy[3] = {0, 0, 0};
+      for (int d = 0; d < DIM; d++) yy[d] = (int)rint(((s.xr[d][j] - org[d]) + (s.u[d][j] - u0[d])) * inv_ys);
+      ly[q] = make_int4(yy[0], yy[1], yy[2], ly[q].w);
+    }
+  }
   if (threadIdx.x == 0) {  // the padding's record
+    const int pad = fixed ? PAD_Q : __float_as_int(PAD_POS);
     if (FIRST || GEOM) lx[nw] = make_float4(PAD_POS, PAD_POS, DIM == 3 ? PAD_POS : 0.f, 0.f);
     if (FIRST) lq[nw] = make_int4(0, 0, 0, 0);
-    if (SECOND) ly[nw] = make_float4(PAD_POS, PAD_POS, DIM == 3 ? PAD_POS : 0.f, 0.f);
+    if (SECOND) ly[nw] = make_int4(pad, pad, DIM == 3 ? pad : 0, 0);
   }
   __syncthreads();
-  return us;
+  return ldexpf(1.f, eu);
 }
 
 // Per-particle constants of the mixed bond loops (those of every bond in
@@ -399,7 +478,7 @@ __device__ __forceinline__ bool slack_bond(double r, double low) {
 // at hand, also sums the alpha part of the force and the repulsion of broken
 // bonds (into f), and the second pass only adds
 //   sum_j r J V_j^c (b_i + b_j) y / |y|
-// from the bond's weight and one record of current positions per neighbor.
+// from the bond's weight and the neighbors' current positions.
 //
 // The loops are bound by FP32 instruction issue and the latency of the list
 // reads.  Per bond in 3D they take 42 instructions in the first pass and 14 in
@@ -609,10 +688,10 @@ __device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m
 }
 
 // Second pass of one block: sum of 2 r J V^c (b_i + b_j) y / |y| into f
-template <int DIM, bool LDS, bool GEOM>
+template <int DIM, bool LDS, bool GEOM, bool FIXED>
 __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const StateConsts& c, const uint4& cur,
                                              const float4* wg, int left, unsigned wblk, const float* xi,
-                                             const float* yi, float bi, float (&f)[3]) {
+                                             const typename Win<DIM, LDS>::Cur& own, float (&f)[3]) {
 #pragma clang fp contract(fast)
   auto bond = [&](const int tt, const float wt, auto exact) {
     const int e = block_id<LDS>(cur, tt);
@@ -627,13 +706,11 @@ __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const State
       }
       wj = c.weight<decltype(exact)::value>(xx4 * rsqf_hw(xx4), xvj.w);
     }
-    const float4 ybj = w.yb(e);
-    const float yj[3] = {ybj.x, ybj.y, ybj.z};
-    float y[3];
-    for (int d = 0; d < DIM; d++) y[d] = yj[d] - yi[d];
+    float y[3], b;
+    w.template dy<FIXED>(e, own, y, b);
     float yy = y[0] * y[0];
     for (int d = 1; d < DIM; d++) yy += y[d] * y[d];
-    const float sf = wj * (bi + ybj.w) * rsqf_hw(yy);
+    const float sf = wj * b * rsqf_hw(yy);
     for (int d = 0; d < DIM; d++) f[d] += sf * y[d];
   };
   const std::false_type fast{};
@@ -663,7 +740,7 @@ __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const State
 }
 
 // Second pass of the node in thread slot q: adds the b terms to f.
-template <int DIM, bool LDS, bool GEOM, int LPN>
+template <int DIM, bool LDS, bool GEOM, bool FIXED, int LPN>
 __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m, const DevTile& t,
                                                  const Win<DIM, LDS>& w, const StateConsts& c, int q) {
   const uint32_t ln = m.lnode[t.node + q];
@@ -673,8 +750,9 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
   const uint4* cb = (const uint4*)(m.col16 + at) + q % WAVE;
   const float4* wb = (const float4*)(m.wgt + at) + q % WAVE;
   const unsigned* bw = s.bits + s.bptr[i / WAVE] + i % WAVE;
-  const float4 ybi = w.yb(w.entry(i)), xvi = GEOM ? w.x2(w.entry(i)) : ybi;
-  const float yi[3] = {ybi.x, ybi.y, ybi.z}, xi[3] = {xvi.x, xvi.y, xvi.z};
+  const auto own = w.cur(w.entry(i));
+  const float4 xvi = GEOM ? w.x2(w.entry(i)) : make_float4(0.f, 0.f, 0.f, 0.f);
+  const float xi[3] = {xvi.x, xvi.y, xvi.z};
   double force[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) force[d] = s.f[d][i];
   if (LPN == 1) {
@@ -685,8 +763,8 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
       const uint4 cur = blk;
       if (kb + KB < n) blk = cb[(kb / KB + 1) * WAVE];
       float fb[3] = {0.f, 0.f, 0.f};
-      second_block<DIM, LDS, GEOM>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb, (word >> (kb & 31)) & 0xffu, xi, yi,
-                                   ybi.w, fb);
+      second_block<DIM, LDS, GEOM, FIXED>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb, (word >> (kb & 31)) & 0xffu, xi, own,
+                                   fb);
       for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)fb[d];
     }
   } else {
@@ -694,8 +772,8 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
       const int kb = k0 + KB * sub;
       float fb[3] = {0.f, 0.f, 0.f};
       if (kb < n)
-        second_block<DIM, LDS, GEOM>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
-                                     (bw[(int64_t)(kb >> 5) * WAVE] >> (kb & 31)) & 0xffu, xi, yi, ybi.w, fb);
+        second_block<DIM, LDS, GEOM, FIXED>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
+                                     (bw[(int64_t)(kb >> 5) * WAVE] >> (kb & 31)) & 0xffu, xi, own, fb);
       for (int k = 0; k < LPN; k++)
         if (k0 + KB * k < n)
           for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)group_lane<LPN>(fb[d], k);
@@ -724,13 +802,30 @@ __device__ __forceinline__ int slot_rounds(const MixedArgs& m, const DevTile& t)
   return (t.te - t.ts + per - 1) / per;
 }
 
+// the second pass of a tile's nodes
+template <int DIM, bool LDS, bool GEOM, int LPN>
+__device__ __forceinline__ void second_pass(const DS& s, const MixedArgs& m, const DevTile& t, const Win<DIM, LDS>& w,
+                                            const StateConsts& c, bool fixed) {
+  const int nr = slot_rounds<LDS, LPN>(m, t);
+  auto run = [&](auto fx) {
+    for (int it = 0; it < nr; it++) {
+      const int q = slot_of<LDS, LPN>(m, it);
+      if (q < t.te - t.ts) second_pass_node<DIM, LDS, GEOM, decltype(fx)::value, LPN>(s, m, t, w, c, q);
+    }
+  };
+  if (LDS && fixed)
+    run(std::true_type{});
+  else
+    run(std::false_type{});
+}
+
 // LDS of the window records, one more than the window for the list padding
 // (LDS tiles), or a dummy (HBM tiles)
 #define PDEM_WINDOW_LDS(LDS_ON, NODES, FIRST, SECOND, GEOM)    \
   __shared__ float4 lx[(LDS_ON) && ((FIRST) || (GEOM)) ? (NODES) + 1 : 1]; \
   __shared__ int4 lq[(LDS_ON) && (FIRST) ? (NODES) + 1 : 1];   \
-  __shared__ float4 ly[(LDS_ON) && (SECOND) ? (NODES) + 1 : 1]; \
-  __shared__ float red[1024 / WAVE];
+  __shared__ int4 ly[(LDS_ON) && (SECOND) ? (NODES) + 1 : 1];  \
+  __shared__ float4 red[1024 / WAVE];
 #define PDEM_WINDOW(DIM, LDS_ON, t, gs) \
   Win<DIM, LDS_ON> w{(const char*)lx, (const char*)lq, (const char*)ly, &s, &m, gs, t.ws, 1.f, \
                       1. / particle_scale(s, p), {0., 0., 0.}}; \
@@ -745,7 +840,8 @@ __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_dilation(DS
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, LDS, t, gs)
-  if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
+  bool fixed = false;
+  if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
   const StateConsts c(s, p);
   const int nr = slot_rounds<LDS, LPN>(m, t);
   for (int it = 0; it < nr; it++) {
@@ -765,13 +861,10 @@ __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_force(DS s,
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, LDS, t, gs)
-  if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
+  bool fixed = false;
+  if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
   const StateConsts c(s, p);
-  const int nr = slot_rounds<LDS, LPN>(m, t);
-  for (int it = 0; it < nr; it++) {
-    const int q = slot_of<LDS, LPN>(m, it);
-    if (q < t.te - t.ts) second_pass_node<DIM, LDS, GEOM, LPN>(s, m, t, w, c, q);
-  }
+  second_pass<DIM, LDS, GEOM, LPN>(s, m, t, w, c, fixed);
 }
 
 // Both passes of a closed tile, a whole particle, so that every neighbor of
@@ -785,7 +878,8 @@ __global__ void __launch_bounds__(TPB, TPB == 512 ? 6 : MIXED_WAVES_PER_SIMD) k_
   const DevParticle& p = s.P[t.pid];
   const int gs = (int)p.glob_start;
   PDEM_WINDOW(DIM, true, t, gs)
-  w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red);
+  bool fixed;
+  w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
   const StateConsts c(s, p);
   const int nr = slot_rounds<true, 1>(m, t);
   for (int it = 0; it < nr; it++) {
@@ -793,13 +887,10 @@ __global__ void __launch_bounds__(TPB, TPB == 512 ? 6 : MIXED_WAVES_PER_SIMD) k_
     if (q >= t.te - t.ts) continue;
     int i;
     const float b = first_pass_node<DIM, true, GEOM, 1>(s, m, t, w, c, q, i);
-    ly[i - t.ws].w = b;
+    ly[i - t.ws].w = __float_as_int(b);
   }
   __syncthreads();
-  for (int it = 0; it < nr; it++) {
-    const int q = slot_of<true, 1>(m, it);
-    if (q < t.te - t.ts) second_pass_node<DIM, true, GEOM, 1>(s, m, t, w, c, q);
-  }
+  second_pass<DIM, true, GEOM, 1>(s, m, t, w, c, fixed);
 }
 
 #undef PDEM_WINDOW

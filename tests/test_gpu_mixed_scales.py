@@ -21,7 +21,7 @@ def _model(dim, n, nodes, R, inf, j_scale):
     depend on, so that the weighted volume of meshes below 0.07 mm stays in
     the accepted range."""
     rng = np.random.default_rng(21)
-    mat = configs.pdstate_material(inf=inf)
+    mat = configs.pdstate_material(K=5e7, inf=inf)  # K far from 5 G / 3, where the dilation has no force
     h = R * ((4.18879 / nodes) ** (1 / 3) if dim == 3 else (3.14159 / nodes / 0.866) ** 0.5)
     ref, vol = (ball_mesh if dim == 3 else disk_mesh)(R, h)
     b = ModelBuilder(dim, 1e-8, [ZoneDeck(mat)], {}, multi_particle=False)
