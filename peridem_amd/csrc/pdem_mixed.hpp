@@ -142,12 +142,13 @@ __device__ __forceinline__ float uniform(float x) {
   return __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(x)));
 }
 __device__ __forceinline__ float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
-// hardware square root and reciprocal square root (1 ulp, no denormal
-// rescaling): bond lengths squared are far from the FP32 denormal range.
-// The reciprocal square root yields both |v| = |v|^2 rsq(|v|^2) and 1 / |v|
-// from one transcendental (a quarter-rate instruction).
-__device__ __forceinline__ float sqrtf_hw(float x) { return __builtin_amdgcn_sqrtf(x); }
+// hardware reciprocal square root (1 ulp, no denormal rescaling): bond lengths
+// squared are far from the FP32 denormal range.  It yields both
+// |v| = |v|^2 rsq(|v|^2) and 1 / |v| from one transcendental (a quarter-rate
+// instruction).
 __device__ __forceinline__ float rsqf_hw(float x) { return __builtin_amdgcn_rsqf(x); }
+// the larger value, or NaN if either is one (v_maximum3_f32)
+__device__ __forceinline__ float max_nan(float a, float b) { return __builtin_elementwise_maximum(a, b); }
 // isGreater(a, b) with a, b >= 0 (util::isGreater, function.h, slack 1e-5 of
 // the larger operand) reduces to a (1 - 1e-5) > b: one compare against a
 // threshold scaled once per particle.
@@ -498,7 +499,7 @@ __device__ __forceinline__ bool slack_bond(double r, double low) {
 // doubled current bond vector
 template <int DIM>
 struct Stretch {
-  float xx4, r2, inv_r2, l2, inv_l2, c2, y2[3];
+  float xx4, yy4, r2, inv_r2, l2, inv_l2, c2, y2[3];
   // d2: twice the reference bond vector; q: relative displacement in units of us
   __device__ __forceinline__ Stretch(const float* d2, const float* q, float us) {
 #pragma clang fp contract(fast)
@@ -510,21 +511,28 @@ struct Stretch {
     }
     for (int d = 0; d < DIM; d++) y2[d] = d2[d] + 2.f * us * q[d];
     t *= us;                      // |y|^2 - |xi|^2
-    const float yy4 = xx4 + 4.f * t;
+    yy4 = xx4 + 4.f * t;
     inv_r2 = rsqf_hw(xx4);
     inv_l2 = rsqf_hw(yy4);
     r2 = xx4 * inv_r2;            // 2 |xi|
     l2 = yy4 * inv_l2;            // 2 |y|
     c2 = t * rcpf(l2 + r2);       // (|y| - |xi|) / 2
   }
-  __device__ __forceinline__ float s4() const { return fabsf(c2) * inv_r2; }  // |S| / 4
+  // a bond whose ends have met (|y| = 0 to rounding: l2 above is no number) has
+  // lost its whole length
+  __device__ __forceinline__ void met() {
+    if (yy4 <= 0.f) {
+      l2 = 0.f;
+      c2 = -0.25f * r2;
+    }
+  }
 };
 
 // the sums of one 8-bond block in the first pass
 struct Block1 {
   double theta;  // sum r c J V^c / particle_scale
   float f[3];
-  float z;       // largest |S| / 4
+  float z;       // largest |S| / 4, NaN if one is
 };
 
 // First pass of one block of a node's list: entries `cur`, weights at wg,
@@ -550,7 +558,7 @@ __device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const Stat
       const Stretch<DIM> b(d2, du, us);
       const float wj = GEOM ? c.weight<false>(b.r2, vj) : wt;
       const float p = b.c2 * b.inv_r2;  // S / 4
-      o.z = fmaxf(o.z, fabsf(p));
+      o.z = max_nan(o.z, fabsf(p));
       o.theta += (double)(b.c2 * wj);
       const float sf = p * wj * (own.a + aj) * b.inv_l2;
       for (int d = 0; d < DIM; d++) o.f[d] += sf * b.y2[d];
@@ -569,19 +577,20 @@ __device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const Stat
       bond(7, wb.w);
     }
     if (wblk == 0u && o.z <= c.thr4 && !(GEOM && (cur.x & SLACK_BLOCK))) return o;
-    o = Block1{0., {0.f, 0.f, 0.f}, o.z};
+    o = Block1{0., {0.f, 0.f, 0.f}, 0.f};
   }
-  // bond by bond: a bond of the block is broken, breaks now or (GEOM) is in
-  // the slack, and every block of an HBM tile
+  // bond by bond: a bond of the block is broken, breaks now, has no length left
+  // or (GEOM) is in the slack, and every block of an HBM tile
   const int nb = left < KB ? left : KB;
 #pragma unroll 1
   for (int tt = 0; tt < nb; tt++) {
     float d2[3], du[3], vj, aj;
     load(block_id<LDS>(cur, tt), d2, du, vj, aj);
-    const Stretch<DIM> b(d2, du, us);
+    Stretch<DIM> b(d2, du, us);
+    b.met();
     const float wj = GEOM ? c.weight<true>(b.r2, vj) : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4];
     const float p = b.c2 * b.inv_r2;
-    o.z = fmaxf(o.z, fabsf(p));
+    o.z = max_nan(o.z, fabsf(p));
     bool fs = ((wblk >> tt) & 1u) != 0u;
     if (!fs && fabsf(p) > c.thr4) {
       fs = true;
@@ -613,7 +622,7 @@ __device__ __forceinline__ T group_lane(T v, int k) {
 // First pass of the node in thread slot q: breaks bonds, writes theta, the
 // damage Z and the first part of the force, and returns the node's b term.
 // The damage Z_i (demModel.cpp:770-773) is the plain maximum of |S| / s0 over
-// the list, broken bonds included (the reference's running compare with a
+// the list, broken bonds included, NaN where a stretch is (the reference's running compare with a
 // 1e-5 relative slack keeps a value at most 1e-5 below it; FP32 bond
 // arithmetic is the larger difference).
 template <int DIM, bool LDS, bool GEOM, int LPN>
@@ -636,7 +645,7 @@ __device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m
   float Zs = 0.f;  // maximum of |S| / 4 over all bonds, broken ones included
   auto add = [&](const Block1& o, int k) {
     theta += group_lane<LPN>(o.theta, k);
-    Zs = fmaxf(Zs, group_lane<LPN>(o.z, k));
+    Zs = max_nan(Zs, group_lane<LPN>(o.z, k));
     for (int d = 0; d < DIM; d++) force[d] += (double)group_lane<LPN>(o.f[d], k);
   };
   if (LPN == 1) {
