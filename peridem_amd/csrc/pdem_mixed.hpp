@@ -428,12 +428,12 @@ struct StateConsts {
   float ja, jb, low2, inv_h2, up_h;
   __device__ StateConsts(const DS& s, const DevParticle& p) {
     thr4 = uniform(0.25f * ((float)(p.mat[2] + 1.0e-10) / REL_KEEP));
-    inv_s0 = (float)(1.0 / p.mat[2]);
-    Rc = (float)p.Rc;
+    inv_s0 = uniform((float)(1.0 / p.mat[2]));
+    Rc = uniform((float)p.Rc);
     K = p.mat[0];
     G = p.mat[1];
     scale = particle_scale(s, p);
-    Kn = (float)(p.Kn * scale);
+    Kn = uniform((float)(p.Kn * scale));
     ja = uniform((float)s.inf_p0);
     jb = uniform(s.inf_type == 1 ? (float)(0.5 * s.inf_p1 / p.horizon) : 0.f);
     low2 = uniform(2.f * ((float)(p.horizon - 0.5 * p.h) / REL_KEEP));
@@ -446,13 +446,13 @@ struct StateConsts {
   // the fourth power of the mesh size, is in v, which is 0 there.  The
   // correction is 1 at the distance horizon - h/2 from which it applies, so
   // clamping it to [0, 1], which the multiply-add does for nothing, saves the
-  // compare and the select (EXACT) for every bond but those in the slack of
+  // compare and the select (exact) for every bond but those in the slack of
   // the reference's compare (see slack_bond).
-  template <bool EXACT>
-  __device__ __forceinline__ float weight(float r2, float v) const {
+  __device__ __forceinline__ float weight(float r2, float v, bool exact) const {
 #pragma clang fp contract(fast)
     const float c = up_h - r2 * inv_h2;
-    const float k = EXACT ? (r2 > low2 ? c : 1.f) : __builtin_amdgcn_fmed3f(c, 0.f, 1.f);
+    float k = __builtin_amdgcn_fmed3f(c, 0.f, 1.f);
+    if (exact) k = r2 > low2 ? c : 1.f;
     return r2 * ((ja + jb * r2) * (v * k));
   }
 };
@@ -489,8 +489,16 @@ __device__ __forceinline__ bool slack_bond(double r, double low) {
 // before, 325 us now (kernel trace), 412 MB against 179 MB fetched.
 //
 // The loops take 4 bonds at a time without any test per bond: the lists are
-// padded to whole blocks (see Win), and a block with a bond that is broken, or
-// whose largest stretch says that one breaks now, is done again bond by bond.
+// padded to whole blocks (see Win), and a block whose largest stretch says that
+// a bond breaks now is done again with tests.  Where a lane of the wavefront
+// holds a broken bond among the 32 of a word, all its lanes take those blocks
+// with tests only, two bonds a round: doing the blocks twice there, lane by
+// lane and bond by bond, took 211 us for both passes of 400 spheres of 1021
+// nodes with 5 % of their bonds broken, 126 us now (104 us with none broken);
+// 2000 disks of 361 nodes 132 us, 89 now (77).  (A fully unrolled loop with
+// tests takes 120 us there, but its registers spill in the loop without tests:
+// 8 % on the intact packing of 2000 spheres, 26 % on the 512-instance ensemble.
+// The looking for broken bits costs 1 % of these steps.)
 // Every sum is taken per block (theta in FP64, forces in FP32) and the blocks
 // are added in list order in FP64, so the results do not depend on how blocks
 // are dealt to lanes.
@@ -537,75 +545,78 @@ struct Block1 {
 
 // First pass of one block of a node's list: entries `cur`, weights at wg,
 // `left` bonds to the list's end, broken bits wblk; brk gets the bonds that
-// break now.
+// break now.  `tests` (the same for the wavefront): some lane has a broken bond
+// here or hereabouts, and the block goes to the loop with tests at once.
 template <int DIM, bool LDS, bool GEOM>
-__device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const StateConsts& c, const uint4& cur,
+__device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const StateConsts& c, uint4 cur,
                                               const float4* wg, int left, unsigned wblk, const float* xi,
-                                              const typename Win<DIM, LDS>::Own& own, float us, unsigned& brk) {
+                                              const typename Win<DIM, LDS>::Own& own, float us, bool tests, unsigned& brk) {
 #pragma clang fp contract(fast)
   Block1 o{0., {0.f, 0.f, 0.f}, 0.f};
-  auto load = [&](int e, float* d2, float* du, float& vj, float& aj) {
+  const bool slack = GEOM && (cur.x & SLACK_BLOCK);
+  // one bond; SURE that it is whole and stays so
+  auto bond = [&](const int e, const float wt, const int tt, auto sure) {
+    constexpr bool SURE = decltype(sure)::value;
     const float4 xvj = w.x2(e);
     const float xj[3] = {xvj.x, xvj.y, xvj.z};
+    float d2[3], du[3], aj;
     w.du(e, own, du, aj);
     for (int d = 0; d < DIM; d++) d2[d] = xj[d] - xi[d];
-    vj = xvj.w;
-  };
-  if (LDS) {
-    auto bond = [&](const int tt, const float wt) {
-      float d2[3], du[3], vj, aj;
-      load(block_id<LDS>(cur, tt), d2, du, vj, aj);
-      const Stretch<DIM> b(d2, du, us);
-      const float wj = GEOM ? c.weight<false>(b.r2, vj) : wt;
-      const float p = b.c2 * b.inv_r2;  // S / 4
-      o.z = max_nan(o.z, fabsf(p));
-      o.theta += (double)(b.c2 * wj);
-      const float sf = p * wj * (own.a + aj) * b.inv_l2;
-      for (int d = 0; d < DIM; d++) o.f[d] += sf * b.y2[d];
-      if (tt % 2 == 1) pin(o.f, o.z);
-    };
-    const float4 wa = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[0];
-    const float4 wb = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[WAVE];
-    bond(0, wa.x);
-    bond(1, wa.y);
-    bond(2, wa.z);
-    bond(3, wa.w);
-    if (left > KB / 2) {
-      bond(4, wb.x);
-      bond(5, wb.y);
-      bond(6, wb.z);
-      bond(7, wb.w);
-    }
-    if (wblk == 0u && o.z <= c.thr4 && !(GEOM && (cur.x & SLACK_BLOCK))) return o;
-    o = Block1{0., {0.f, 0.f, 0.f}, 0.f};
-  }
-  // bond by bond: a bond of the block is broken, breaks now, has no length left
-  // or (GEOM) is in the slack, and every block of an HBM tile
-  const int nb = left < KB ? left : KB;
-#pragma unroll 1
-  for (int tt = 0; tt < nb; tt++) {
-    float d2[3], du[3], vj, aj;
-    load(block_id<LDS>(cur, tt), d2, du, vj, aj);
     Stretch<DIM> b(d2, du, us);
-    b.met();
-    const float wj = GEOM ? c.weight<true>(b.r2, vj) : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4];
-    const float p = b.c2 * b.inv_r2;
+    if (!SURE) b.met();
+    const float wj = GEOM ? c.weight(b.r2, xvj.w, !SURE && slack) : wt;
+    const float p = b.c2 * b.inv_r2;  // S / 4
     o.z = max_nan(o.z, fabsf(p));
-    bool fs = ((wblk >> tt) & 1u) != 0u;
-    if (!fs && fabsf(p) > c.thr4) {
-      fs = true;
-      brk |= 1u << tt;
-    }
-    float sf;
-    if (!fs) {
-      o.theta += (double)(b.c2 * wj);
-      sf = p * wj * (own.a + aj) * b.inv_l2;
+    const float th = b.c2 * wj;
+    float sf = p * wj * (own.a + aj) * b.inv_l2;
+    if (SURE) {
+      o.theta += (double)th;
     } else {
-      // Kn V (|y| - Rc) y / |y| where it repels (Kn with the scale of vj)
-      sf = c.Kn * vj * (0.5f * b.l2 - c.Rc) * b.inv_l2;
-      if (sf > 0.f) sf = 0.f;
+      bool fs = ((wblk >> tt) & 1u) != 0u;
+      if (!fs && fabsf(p) > c.thr4) {
+        fs = true;
+        brk |= 1u << tt;
+      }
+      if (!fs) {
+        o.theta += (double)th;
+      } else {
+        // Kn V (|y| - Rc) y / |y| where it repels (Kn with the scale of vj)
+        sf = c.Kn * xvj.w * (0.5f * b.l2 - c.Rc) * b.inv_l2;
+        if (sf > 0.f) sf = 0.f;
+      }
     }
     for (int d = 0; d < DIM; d++) o.f[d] += sf * b.y2[d];
+  };
+  if (LDS && !tests) {
+    auto half = [&](unsigned id0, unsigned id1, const float4& wt, const int t0) {
+      const std::true_type sure{};
+      bond((int)(id0 & 0x7fffu), wt.x, t0, sure);
+      bond((int)(id0 >> 16), wt.y, t0 + 1, sure);
+      pin(o.f, o.z);
+      bond((int)(id1 & 0xffffu), wt.z, t0 + 2, sure);
+      bond((int)(id1 >> 16), wt.w, t0 + 3, sure);
+      pin(o.f, o.z);
+    };
+    const float4 none = make_float4(0.f, 0.f, 0.f, 0.f);
+    const float4 wa = GEOM ? none : wg[0], wb = GEOM ? none : wg[WAVE];
+    half(cur.x, cur.y, wa, 0);
+    if (left > KB / 2) half(cur.z, cur.w, wb, KB / 2);
+    if (o.z <= c.thr4 && !slack) return o;
+    o = Block1{0., {0.f, 0.f, 0.f}, 0.f};
+  }
+  // with tests, two entries at a time: blocks with a bond that breaks now or
+  // has no length left or (GEOM) is in the slack, those of a wavefront that
+  // holds broken bonds, and every block of an HBM tile
+#pragma unroll 1
+  for (int tt = 0; tt < KB && tt < left; tt += 2) {
+    float2 wt = make_float2(0.f, 0.f);
+    if (!GEOM) wt = *(const float2*)((const float*)(wg + (tt / 4) * WAVE) + tt % 4);
+    bond((int)(cur.x & (LDS ? 0x7fffu : 0xffffu)), wt.x, tt, std::false_type{});
+    pin(o.f, o.z);
+    if (LDS || tt + 1 < left) bond((int)((cur.x >> 16) & 0xffffu), wt.y, tt + 1, std::false_type{});
+    cur.x = cur.y;
+    cur.y = cur.z;
+    cur.z = cur.w;
   }
   return o;
 }
@@ -650,18 +661,20 @@ __device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m
   };
   if (LPN == 1) {
     unsigned word = 0, wnew = 0;
+    bool tests = false;  // a lane of the wavefront holds a broken bond among these 32
     uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
     for (int kb = 0; kb < n; kb += KB) {
       if ((kb & 31) == 0) {
         if (kb > 0 && wnew != word) bw[(int64_t)((kb >> 5) - 1) * WAVE] = wnew;
         word = bw[(int64_t)(kb >> 5) * WAVE];
         wnew = word;
+        tests = __any(word != 0u);
       }
       const uint4 cur = blk;
       if (kb + KB < n) blk = cb[(kb / KB + 1) * WAVE];
       unsigned brk = 0;
       const Block1 o = first_block<DIM, LDS, GEOM>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb,
-                                             (word >> (kb & 31)) & 0xffu, xi, own, us, brk);
+                                             (word >> (kb & 31)) & 0xffu, xi, own, us, tests, brk);
       wnew |= brk << (kb & 31);
       add(o, 0);
     }
@@ -674,7 +687,7 @@ __device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m
       if (kb < n) {
         word = bw[(int64_t)(kb >> 5) * WAVE];
         o = first_block<DIM, LDS, GEOM>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
-                                  (word >> (kb & 31)) & 0xffu, xi, own, us, brk);
+                                  (word >> (kb & 31)) & 0xffu, xi, own, us, true, brk);
       }
       for (int k = 0; k < LPN; k++)
         if (k0 + KB * k < n) add(o, k);
@@ -700,9 +713,10 @@ __device__ __forceinline__ float first_pass_node(const DS& s, const MixedArgs& m
 template <int DIM, bool LDS, bool GEOM, bool FIXED>
 __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const StateConsts& c, const uint4& cur,
                                              const float4* wg, int left, unsigned wblk, const float* xi,
-                                             const typename Win<DIM, LDS>::Cur& own, float (&f)[3]) {
+                                             const typename Win<DIM, LDS>::Cur& own, bool tests, float (&f)[3]) {
 #pragma clang fp contract(fast)
-  auto bond = [&](const int tt, const float wt, auto exact) {
+  // one bond (whole: SURE that it is not broken)
+  auto bond = [&](const int tt, const float wt, auto whole, auto exact) {
     const int e = block_id<LDS>(cur, tt);
     float wj = wt;
     if (GEOM) {
@@ -713,39 +727,42 @@ __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const State
         d2 = xj[d] - xi[d];
         xx4 += d2 * d2;
       }
-      wj = c.weight<decltype(exact)::value>(xx4 * rsqf_hw(xx4), xvj.w);
+      wj = c.weight(xx4 * rsqf_hw(xx4), xvj.w, decltype(exact)::value);
     }
     float y[3], b;
     w.template dy<FIXED>(e, own, y, b);
     float yy = y[0] * y[0];
     for (int d = 1; d < DIM; d++) yy += y[d] * y[d];
-    const float sf = wj * b * rsqf_hw(yy);
+    float sf = wj * b * rsqf_hw(yy);
+    if (!decltype(whole)::value) sf = ((wblk >> tt) & 1u) ? 0.f : sf;  // (broken bonds: in the first pass)
     for (int d = 0; d < DIM; d++) f[d] += sf * y[d];
   };
-  const std::false_type fast{};
-  if (LDS && wblk == 0u && !(GEOM && (cur.x & SLACK_BLOCK))) {
+  const std::true_type yes{};
+  const std::false_type no{};
+  if (LDS && !(GEOM && (cur.x & SLACK_BLOCK))) {
     const float4 wa = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[0];
     const float4 wb = GEOM ? make_float4(0.f, 0.f, 0.f, 0.f) : wg[WAVE];
-    bond(0, wa.x, fast);
-    bond(1, wa.y, fast);
-    if (GEOM) pin(f, f[0]);
-    bond(2, wa.z, fast);
-    bond(3, wa.w, fast);
-    pin(f, f[0]);
-    if (left > KB / 2) {
-      bond(4, wb.x, fast);
-      bond(5, wb.y, fast);
+    auto half = [&](int t0, const float4& wt, auto whole) {
+      bond(t0, wt.x, whole, no);
+      bond(t0 + 1, wt.y, whole, no);
       if (GEOM) pin(f, f[0]);
-      bond(6, wb.z, fast);
-      bond(7, wb.w, fast);
-    }
+      bond(t0 + 2, wt.z, whole, no);
+      bond(t0 + 3, wt.w, whole, no);
+    };
+    auto block = [&](auto whole) {
+      half(0, wa, whole);
+      pin(f, f[0]);
+      if (left > KB / 2) half(KB / 2, wb, whole);
+    };
+    if (!tests)
+      block(yes);
+    else if (wblk != (left < KB ? (1u << left) - 1u : 0xffu))  // (not all of them broken)
+      block(no);
     return;
   }
   const int nb = left < KB ? left : KB;
 #pragma unroll 1
-  for (int tt = 0; tt < nb; tt++)  // broken bonds: in the first pass
-    if (!((wblk >> tt) & 1u))
-      bond(tt, GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], std::true_type{});
+  for (int tt = 0; tt < nb; tt++) bond(tt, GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], no, yes);
 }
 
 // Second pass of the node in thread slot q: adds the b terms to f.
@@ -766,14 +783,18 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
   for (int d = 0; d < DIM; d++) force[d] = s.f[d][i];
   if (LPN == 1) {
     unsigned word = 0;
+    bool tests = false;
     uint4 blk = n > 0 ? cb[0] : make_uint4(0, 0, 0, 0);
     for (int kb = 0; kb < n; kb += KB) {
-      if ((kb & 31) == 0) word = bw[(int64_t)(kb >> 5) * WAVE];
+      if ((kb & 31) == 0) {
+        word = bw[(int64_t)(kb >> 5) * WAVE];
+        tests = __any(word != 0u);
+      }
       const uint4 cur = blk;
       if (kb + KB < n) blk = cb[(kb / KB + 1) * WAVE];
       float fb[3] = {0.f, 0.f, 0.f};
       second_block<DIM, LDS, GEOM, FIXED>(w, c, cur, wb + (kb / KB) * 2 * WAVE, n - kb, (word >> (kb & 31)) & 0xffu, xi, own,
-                                   fb);
+                                   tests, fb);
       for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)fb[d];
     }
   } else {
@@ -782,7 +803,7 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
       float fb[3] = {0.f, 0.f, 0.f};
       if (kb < n)
         second_block<DIM, LDS, GEOM, FIXED>(w, c, cb[(kb / KB) * WAVE], wb + (kb / KB) * 2 * WAVE, n - kb,
-                                     (bw[(int64_t)(kb >> 5) * WAVE] >> (kb & 31)) & 0xffu, xi, own, fb);
+                                     (bw[(int64_t)(kb >> 5) * WAVE] >> (kb & 31)) & 0xffu, xi, own, true, fb);
       for (int k = 0; k < LPN; k++)
         if (k0 + KB * k < n)
           for (int d = 0; d < DIM; d++) force[d] += 0.5 * (double)group_lane<LPN>(fb[d], k);
