@@ -299,15 +299,19 @@ struct Launch {
   }
   static void hbm_first(pdem_ctx* c, hipStream_t st) {
     const MixedArgs& ma = c->mixed;
-    if (ma.ntiles_hbm)
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB>), dim3((unsigned)(ma.ntiles_hbm * ma.hbm_split)),
-                         dim3(HBM_TPB), 0, st, c->ds, ma);
+    const dim3 g(hbm_blocks(ma)), t(HBM_TPB);
+    if (ma.ntiles_hbm && ma.hbm_lpn == 8)
+      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB, LDS_NODES, 8>), g, t, 0, st, c->ds, ma);
+    else if (ma.ntiles_hbm)
+      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB, LDS_NODES, 4>), g, t, 0, st, c->ds, ma);
   }
   static void hbm_second(pdem_ctx* c, hipStream_t st) {
     const MixedArgs& ma = c->mixed;
-    if (ma.ntiles_hbm)
-      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB>), dim3((unsigned)(ma.ntiles_hbm * ma.hbm_split)),
-                         dim3(HBM_TPB), 0, st, c->ds, ma);
+    const dim3 g(hbm_blocks(ma)), t(HBM_TPB);
+    if (ma.ntiles_hbm && ma.hbm_lpn == 8)
+      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB, LDS_NODES, 8>), g, t, 0, st, c->ds, ma);
+    else if (ma.ntiles_hbm)
+      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB, LDS_NODES, 4>), g, t, 0, st, c->ds, ma);
   }
   template <int T, bool GEOM>
   static void mixed_state(pdem_ctx* c) {
@@ -826,13 +830,15 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
       t.node = (int)lnode.size();
       t.slice = (int)lslice.size();
       t.data = data;
-      // slots: nodes by their count of half blocks (most first), then by id
+      // slots: nodes by their count of half blocks (most first), then by id;
+      // HBM tiles: by id
       const int* deg = c->h_deg.data() + t.ts;
       order.resize(n);
       for (int q = 0; q < n; q++) order[q] = q;
-      std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
-        return (deg[a] + KB / 2 - 1) / (KB / 2) > (deg[b] + KB / 2 - 1) / (KB / 2);
-      });
+      if (t.lds)
+        std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
+          return (deg[a] + KB / 2 - 1) / (KB / 2) > (deg[b] + KB / 2 - 1) / (KB / 2);
+        });
       int64_t len = 0;
       for (int q = 0; q < n; q += WAVE) {
         lslice.push_back((int)len);
@@ -959,7 +965,10 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
   c->mixed.small = maxw <= LDS_SMALL ? 1 : 0;
   c->mixed.mid = maxw <= LDS_MID ? 1 : 0;
   c->mixed.ntiles_hbm = c->ntiles_global;
-  c->mixed.hbm_split = std::max(1, (int)(tile_max * HBM_LPN / HBM_TPB));
+  int64_t hbm_nodes = 0;
+  for (auto& t : tiles) hbm_nodes += t.lds ? 0 : t.te - t.ts;
+  c->mixed.hbm_lpn = hbm_nodes > HBM_LPN8_NODES ? 4 : 8;
+  c->mixed.hbm_split = std::max(1, (int)(tile_max * c->mixed.hbm_lpn / HBM_TPB));
   c->tile_nodes = (int)tile_max;
   c->mixed.tiles = c->d_tiles;
   build_lists(c, tiles);

@@ -30,7 +30,7 @@
 // bonds (0.9 GB) shrink to a few of 0.4 MB.  A tile whose list matches no
 // other keeps its own.
 //
-// Threads take nodes in slot order: inside every tile the nodes are ordered
+// Threads take nodes in slot order: inside every LDS tile the nodes are ordered
 // by their number of 4-bond half blocks (most first, node id second), so the
 // 64 lanes of a wavefront run lists of about the same length (a wavefront
 // runs as long as its longest list; surface nodes have far fewer bonds than
@@ -62,15 +62,26 @@ constexpr int LDS_SMALL = 384;
 // 2000 spheres of 1021 nodes: 0.541 to 0.516 ms per step).
 constexpr int LDS_MID = 1120;
 constexpr int KB = 8;             // neighbor ids per 16-byte block
-// HBM tiles: workgroup size and lanes per node.  They are few (a meshed wall)
-// and wait on gathers, so a node's list is dealt to 8 lanes and a tile to
-// several workgroups (top wall of the packing, 17 tiles: 273 us for both
-// passes with a lane per node and a workgroup per tile, 114 us now, beside
-// the fused kernel's 325 us).
-constexpr int HBM_TPB = 256, HBM_LPN = 8;
+// HBM tiles (a meshed wall, a particle of many nodes) wait on gathers.  A tile
+// goes to several workgroups of HBM_TPB threads, all on one XCD (see
+// hbm_tile), whose L2 then holds its neighbors' data once; its nodes keep
+// their order, so that neighboring lanes gather neighboring nodes; and a
+// node's list is dealt to 8 lanes, or to 4 in models of more than HBM_LPN8_NODES
+// nodes in such tiles, which have enough wavefronts without.  Both passes, us,
+// before there were lanes to a node / 8 lanes of tiles over all XCDs / 8 / 4:
+//   sphere of 9.9k nodes            286    94    89   102
+//   sphere of 40k                   391   261   207   214
+//   10 of 9.9k                      343   377   258   264
+//   10 of 40k                      1005  1640  1100   972
+//   40 of 40k                      4615  6400  4106  3466
+//   10 of 9.9k, nodes in any order  913   650   591   576
+constexpr int HBM_TPB = 256;
+constexpr int64_t HBM_LPN8_NODES = 1 << 17;
 // waves per SIMD the bond kernels are compiled for (at most 64 VGPRs): two
 // 1024-thread workgroups per CU, so one stages its window while the other computes
 constexpr int MIXED_WAVES_PER_SIMD = 8;
+// the first pass of HBM tiles, whose positions are FP64, would spill
+constexpr int HBM_WAVES_PER_SIMD = 6;
 
 struct DevTile {
   int ts, te;     // nodes [ts, te)
@@ -92,7 +103,7 @@ struct DevTile {
 struct MixedArgs {
   const DevTile* tiles;   // closed LDS tiles, then open LDS tiles, then HBM tiles
   int ntiles_closed, ntiles_lds, ntiles_hbm;
-  int hbm_split;          // workgroups per HBM tile
+  int hbm_lpn, hbm_split; // HBM tiles: lanes per node, workgroups per tile
   int small;              // every LDS window holds at most LDS_SMALL nodes
   int mid;                // every LDS window holds at most LDS_MID nodes
   // the lists (see DevTile)
@@ -815,16 +826,25 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
 
 // Tile ranges of MixedArgs::tiles: closed LDS tiles (whole particles, fused
 // kernel), open LDS tiles, HBM tiles.  An HBM tile is shared by hbm_split
-// workgroups of HBM_TPB threads (there is no window to stage).
+// workgroups of HBM_TPB threads (there is no window to stage).  Workgroups go
+// to the 8 XCDs in turn, so those of a tile are 8 apart; the last group of 8
+// tiles may be incomplete (hbm_blocks() workgroups, hbm_tile() beyond the tiles).
+constexpr int XCDS = 8;
+__host__ inline unsigned hbm_blocks(const MixedArgs& m) {
+  return (unsigned)((m.ntiles_hbm + XCDS - 1) / XCDS * XCDS * m.hbm_split);
+}
+__device__ __forceinline__ int hbm_tile(const MixedArgs& m) {
+  return (int)blockIdx.x / (XCDS * m.hbm_split) * XCDS + (int)blockIdx.x % XCDS;
+}
 template <bool LDS>
 __device__ __forceinline__ const DevTile& tile_of(const MixedArgs& m) {
-  return m.tiles[LDS ? m.ntiles_closed + (int)blockIdx.x
-                     : m.ntiles_closed + m.ntiles_lds + (int)blockIdx.x / m.hbm_split];
+  return m.tiles[m.ntiles_closed + (LDS ? (int)blockIdx.x : m.ntiles_lds + hbm_tile(m))];
 }
 // thread slot of the workgroup's round `it` over the tile's slots (LPN lanes per slot)
 template <bool LDS, int LPN>
 __device__ __forceinline__ int slot_of(const MixedArgs& m, int it) {
-  return ((LDS ? it : it * m.hbm_split + (int)blockIdx.x % m.hbm_split) * (int)blockDim.x + (int)threadIdx.x) / LPN;
+  const int part = LDS ? 0 : (int)blockIdx.x / XCDS % m.hbm_split;
+  return ((LDS ? it : it * m.hbm_split + part) * (int)blockDim.x + (int)threadIdx.x) / LPN;
 }
 template <bool LDS, int LPN>
 __device__ __forceinline__ int slot_rounds(const MixedArgs& m, const DevTile& t) {
@@ -863,8 +883,9 @@ __device__ __forceinline__ void second_pass(const DS& s, const MixedArgs& m, con
 
 // First pass of the open tiles (tiles that do not hold a whole particle:
 // the second pass of a tile reads the b terms of nodes of other tiles).
-template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = LDS ? 1 : HBM_LPN>
-__global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_dilation(DS s, MixedArgs m) {
+template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = 1>
+__global__ void __launch_bounds__(TPB, LDS ? MIXED_WAVES_PER_SIMD : HBM_WAVES_PER_SIMD) k_mixed_dilation(DS s, MixedArgs m) {
+  if (!LDS && hbm_tile(m) >= m.ntiles_hbm) return;
   PDEM_WINDOW_LDS(LDS, NODES, true, false, GEOM)
   const DevTile t = tile_of<LDS>(m);
   const DevParticle& p = s.P[t.pid];
@@ -884,8 +905,9 @@ __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_dilation(DS
 }
 
 // Second pass of the open tiles.
-template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = LDS ? 1 : HBM_LPN>
+template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = 1>
 __global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_force(DS s, MixedArgs m) {
+  if (!LDS && hbm_tile(m) >= m.ntiles_hbm) return;
   PDEM_WINDOW_LDS(LDS, NODES, false, true, GEOM)
   const DevTile t = tile_of<LDS>(m);
   const DevParticle& p = s.P[t.pid];
