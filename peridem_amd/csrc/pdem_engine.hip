@@ -1233,7 +1233,10 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     s.inv_cell = 1. / cell;
     s.ncells = ncells;
     s.ncell_blocks = (ncells + CELL_BLOCK - 1) / CELL_BLOCK;
-    s.cells_in_ctrl = N <= CTRL_CELLS_NODES && ncells <= CTRL_CELLS ? 1 : 0;
+    s.cells_in_ctrl = N <= CTRL_CELLS_NODES && ncells <= CTRL_CELLS &&
+                              (N - 1) / CTRL_CELLS_NODES_PER_STEP + 1 < d->neigh_update_interval
+                          ? 1
+                          : 0;
     s.cell_count = c->dalloc<int>(ncells + 1);
     s.cell_owner = c->dalloc<int>(ncells + 1);
     hipLaunchKernelGGL(k_cells_init, dim3((unsigned)std::min<int64_t>(blocks(ncells), 4096)), dim3(TPB), 0,

@@ -422,18 +422,20 @@ __device__ void ctrl_decide(Ctrl* cg) {
 // and runs the controller; all workgroups pack the non-wall particles' centre
 // data (and clear the closure's per-step flags).  The cell table is cleared
 // after each rebuild's query (k_contact_force), so no step clears it here.
-// For models of at most CTRL_CELLS_NODES nodes and CTRL_CELLS cells, workgroup 0
-// also builds the cell list on a rebuild step (cells_build_one): three launches
-// and a side stream less in every step, of which most find nothing to do.  With
-// them a small model's step waits for the side stream's fork, three kernels
-// that return at once and the join, about 26 us, whatever the bond kernel
-// takes (two-particle collision of 734 nodes: 56 us per step with the side
-// stream, 49 without; 3D packing of 10.4k nodes: 70 and 62).  The one workgroup
-// takes about 4 us per 1024 nodes, so at 16384 nodes it breaks even when every
-// third step rebuilds the list (11k nodes: 37 us per step against 54 with
-// rebuilds every 40 steps, 164 against 119 with one in every step).
+// For models of at most CTRL_CELLS_NODES nodes and CTRL_CELLS cells that do not
+// rebuild it too often (CTRL_CELLS_NODES_PER_STEP), workgroup 0 also builds the
+// cell list on a rebuild step (cells_build_one): three launches less in every
+// step, of which most find nothing to do.  The one workgroup takes about 6 us
+// per 1024 nodes and rebuild, the three launches 4 us of a step that rebuilds
+// nothing, so it pays where the list is rebuilt every 1 + 1.5 N / 1024 steps or
+// less often by the deck's interval (the controller shortens that only where
+// nodes move a tenth of the contact radius in a step).  2D bed of 12k nodes, us
+// per step, one workgroup / three launches: 131 / 64 with a rebuild in every
+// step, 54 / 44 in every 5th, 41 / 39 in every 10th, 32 / 36 in every 40th; 1.2k
+// nodes 77 / 77 in every step; 3D packing of 10.5k nodes 140 / 82 in every step.
 constexpr int CTRL_BLOCKS = 64;
 constexpr int64_t CTRL_CELLS_NODES = 16384, CTRL_CELLS = 65536;
+constexpr int64_t CTRL_CELLS_NODES_PER_STEP = 700;  // N <= this (interval - 1)
 template <int DIM>
 __device__ void cells_build_one(const DS& s, int* lds);
 
