@@ -66,7 +66,6 @@ __global__ void k_zero_u32(unsigned* p, int n) {
 }
 }  // namespace
 
-// multi-particle models up to this many nodes use the fused step kernels
 // Up to this size the cell list's kernels follow the bond forces on the
 // engine's queue.  Beside them on a side stream, the fork, the three kernels
 // and the join take about 36 us of a step, more than the bond forces of a
@@ -76,6 +75,7 @@ __global__ void k_zero_u32(unsigned* p, int n) {
 // 87 -> 91).
 constexpr int64_t CELLS_INLINE_NODES = int64_t(1) << 16;
 constexpr int64_t LIGHT_2D_MIN_NODES = int64_t(1) << 17;  // 2D models from this size use the light-node contact kernel
+// multi-particle models up to this many nodes use the fused step kernels
 constexpr int64_t FUSE_MAX_NODES = (int64_t)1 << 20;
 
 struct pdem_ctx {
@@ -131,7 +131,6 @@ struct pdem_ctx {
   bool graph_verlet = false;  // the captured step is integrateVerlet
   // bond-based RNP pair-tile kernel (FP64, all force-computing particles RNP)
   RnpTileArgs rt{};
-  bool lists_in_rnp = false;  // this RNP pass's launch also takes the candidate query (set around it)
   bool rnp_tile = false;  // use it (by size, RNP_TILE_NODES; autotuned)
   bool nf_zeroed = false;  // inside a step whose node update zeroed f of the non-force nodes
   int step_fusion = 1;  // fused step kernels: 0 never, 1 models up to FUSE_MAX_NODES, 2 any size
@@ -358,13 +357,14 @@ struct Launch {
       HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
     }
   }
-  // lanes per node of the lane-group RNP kernel (RNP16_NODES)
+  // the lane-group RNP kernel (lanes per node: RNP16_NODES); lists: its launch
+  // also takes the candidate query and the damping partner lists
   template <int INF>
-  static void rnp(pdem_ctx* c, int tpb) {
+  static void rnp(pdem_ctx* c, int tpb, bool lists) {
     const int lpn = c->N <= RNP16_NODES ? 16 : 4;
     const unsigned nb = blocks(c->N * lpn, tpb);
     if (lpn == 16) {
-      const unsigned db = c->lists_in_rnp ? list_dblocks(c, tpb) : 0, qb = c->lists_in_rnp ? blocks(c->N, tpb) : 0;
+      const unsigned db = lists ? list_dblocks(c, tpb) : 0, qb = lists ? blocks(c->N, tpb) : 0;
       hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 16>), dim3(nb + db + qb), dim3(tpb), 0, c->stream, c->ds, (int)nb, (int)db);
     } else {
       hipLaunchKernelGGL((k_pd_rnp<DIM, INF, 4>), dim3(nb), dim3(tpb), 0, c->stream, c->ds, (int)nb, 0);
@@ -376,13 +376,13 @@ struct Launch {
     return (unsigned)std::min<int64_t>((std::max(c->ds.n_nonwall, 1) + w - 1) / w, 1024);
   }
   template <int INF>
-  static void pd_inf(pdem_ctx* c) {
+  static void pd_inf(pdem_ctx* c, bool lists) {
     hipStream_t st = c->stream;
     const unsigned nb = blocks(c->N);
     if (c->precision == PDEM_PREC_MIXED && c->ntiles > 0) {
       if (c->ds.n_noforce > 0 && !c->nf_zeroed)
         hipLaunchKernelGGL(k_zero_noforce<DIM>, dim3(std::min<unsigned>(nb, BZ_BLOCKS)), dim3(TPB), 0, st, c->ds);
-      if (c->rnp_any) rnp<INF>(c, TPB);
+      if (c->rnp_any) rnp<INF>(c, TPB, false);
       if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(nb), dim3(TPB), 0, st, c->ds);
       if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(nb), dim3(TPB), 0, st, c->ds);
       // timed inside: both state-based passes (dilation and force), all tiles
@@ -401,19 +401,19 @@ struct Launch {
       hipLaunchKernelGGL((k_pd_rnp_tile<DIM, INF>), dim3(c->rt.ntiles), dim3(RT_THREADS), c->rt.lds_bytes, st,
                          c->ds, c->rt);
     else if (c->rnp_any || !(c->state_any || c->pmb_any || c->elastic_any))
-      rnp<INF>(c, c->pd_tpb);
+      rnp<INF>(c, c->pd_tpb, lists);
     if (c->pmb_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 2>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->elastic_any) hipLaunchKernelGGL((k_pd_bond<DIM, INF, 3>), dim3(pnb), dim3(pb), 0, st, c->ds);
     if (c->state_any) hipLaunchKernelGGL((k_pd_state<DIM, INF>), dim3(qnb), dim3(pb), 0, st, c->ds);
     ev_end(c, ev, st, c->ev_next_group++);
   }
-  static void pd_forces(pdem_ctx* c) {
+  static void pd_forces(pdem_ctx* c, bool lists = false) {
     if (c->ds.inf_type == 0)
-      pd_inf<0>(c);
+      pd_inf<0>(c, lists);
     else if (c->ds.inf_type == 1)
-      pd_inf<1>(c);
+      pd_inf<1>(c, lists);
     else
-      pd_inf<2>(c);
+      pd_inf<2>(c, lists);
   }
   // the cell list of a rebuild step (counting sort by cell key); every
   // kernel returns at once on other steps
@@ -435,13 +435,11 @@ struct Launch {
   static void pd_forces_and_cells(pdem_ctx* c) {
     if (!c->multi || c->ds.cells_in_ctrl || c->N <= CELLS_INLINE_NODES) {
       // (FP64 RNP models whose cell list is there: the query rides in the bond pass's launch)
-      c->lists_in_rnp = c->multi && c->ds.cells_in_ctrl && c->N <= RNP16_NODES && c->rnp_any && !c->rnp_tile &&
-                        !(c->precision == PDEM_PREC_MIXED && c->ntiles > 0);
-      const bool done = c->lists_in_rnp;
-      pd_forces(c);
-      c->lists_in_rnp = false;
+      const bool in_rnp = c->multi && c->ds.cells_in_ctrl && c->N <= RNP16_NODES && c->rnp_any && !c->rnp_tile &&
+                          !(c->precision == PDEM_PREC_MIXED && c->ntiles > 0);
+      pd_forces(c, in_rnp);
       if (c->multi && !c->ds.cells_in_ctrl) cells_build(c, c->stream);
-      if (c->multi && !done) rebuild_lists(c, c->stream);
+      if (c->multi && !in_rnp) rebuild_lists(c, c->stream);
       return;
     }
     HIPCHK(hipEventRecord(c->ev_fork2, c->stream));

@@ -958,10 +958,13 @@ __device__ __forceinline__ unsigned group_bits(bool on) {
 //   14.6k         29 / 14 /  14        98k   34 / 36 / 58
 //     21k         28 / 18 /  19       191k   51 / 58 / 106
 constexpr int64_t RNP16_NODES = 16384, RNP_TILE_NODES = 81920;
-// With `lists` (small models, whose cell list the controller has built), the
-// workgroups from pdblocks on are those of k_rebuild_lists: the candidate
-// query of a rebuild step needs nothing of this pass, and a launch of its own
-// costs 4 us of every step (734 nodes 29.6 to 28.1 us, 6926 nodes 34 to 32).
+// The workgroups from pdblocks on (small models, whose cell list the controller
+// has built) are those of k_rebuild_lists: the candidate query of a rebuild step
+// needs nothing of this pass, and a launch of its own costs 4 us of every step
+// (2D beds of 734 nodes 29.6 to 28.1 us, 6926 nodes 34 to 32, 13.4k 33.9 to 32.5;
+// balls in 3D, 610 nodes 34.1 to 32.2, 8.2k 44.4 to 42.2, 13.3k 55.6 to 54.1).  The
+// registers are the bond pass's own, 157 in 2D and 197 in 3D with the query and
+// 156 and 196 without.
 template <int DIM>
 __device__ void rebuild_lists_block(const DS& s, int block, int nblocks, int dblocks);
 template <int DIM, int INF, int LPN>
