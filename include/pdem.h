@@ -331,10 +331,10 @@ int pdem_set_launch_config(pdem_ctx *ctx, int32_t pd_tpb, int32_t mixed_tpb, int
  * shape introspection for tuning and tests). */
 int pdem_get_tile_counts(pdem_ctx *ctx, int32_t *lds_tiles, int32_t *hbm_tiles);
 
-/* Bond lists of the tiles above: the number of distinct lists and of their
- * entries, and whether the LDS tiles evaluate their bond weights (1) instead
- * of reading them beside the lists (0). */
-int pdem_get_list_info(pdem_ctx *ctx, int64_t *lists, int64_t *entries, int32_t *evaluated);
+/* Bond lists of the tiles above: the number of distinct lists, of their
+ * entries and of the bond weights stored beside them, and whether the LDS
+ * tiles evaluate their weights (1) instead of reading them (0). */
+int pdem_get_list_info(pdem_ctx *ctx, int64_t *lists, int64_t *entries, int64_t *weights, int32_t *evaluated);
 
 /* Contact kernel selection: at each candidate rebuild, nodes with at most
  * light_max candidates (0..16) go to the lane-per-node contact kernel, the

@@ -444,7 +444,7 @@ def engine_library():
         lib.pdem_set_launch_config.argtypes = [C.c_void_p] + [C.c_int32] * 3
         lib.pdem_get_tile_counts.restype = C.c_int
         lib.pdem_get_list_info.restype = C.c_int
-        lib.pdem_get_list_info.argtypes = [C.c_void_p] + [C.POINTER(C.c_int64)] * 2 + [C.POINTER(C.c_int32)]
+        lib.pdem_get_list_info.argtypes = [C.c_void_p] + [C.POINTER(C.c_int64)] * 3 + [C.POINTER(C.c_int32)]
         lib.pdem_set_contact_light_max.restype = C.c_int
         lib.pdem_set_contact_light_max.argtypes = [C.c_void_p, C.c_int32]
         lib.pdem_get_tile_counts.argtypes = [C.c_void_p] + [C.POINTER(C.c_int32)] * 2
@@ -554,10 +554,11 @@ class GpuEngine(Engine):
 
     def list_info(self):
         """Bond lists of the mixed-precision tiles: (distinct lists, their
-        entries, whether the LDS tiles evaluate their bond weights)."""
-        n, k, e = C.c_int64(), C.c_int64(), C.c_int32()
-        self._check(self.lib.pdem_get_list_info(self.ctx, C.byref(n), C.byref(k), C.byref(e)), "list_info")
-        return n.value, k.value, bool(e.value)
+        entries, whether the LDS tiles evaluate their bond weights, weights
+        stored)."""
+        n, k, w, e = C.c_int64(), C.c_int64(), C.c_int64(), C.c_int32()
+        self._check(self.lib.pdem_get_list_info(self.ctx, *[C.byref(x) for x in (n, k, w, e)]), "list_info")
+        return n.value, k.value, bool(e.value), w.value
 
     def set_step_fusion(self, on=True):
         """Fused step kernels: False never; True (default) for multi-particle

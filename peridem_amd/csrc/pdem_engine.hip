@@ -122,7 +122,7 @@ struct pdem_ctx {
   uint32_t* d_lnode = nullptr;
   int* d_lslice = nullptr;
   size_t col16_cap = 0, wgt_cap = 0, lnode_cap = 0, lslice_cap = 0;
-  int64_t n_lists = 0, n_list_entries = 0;
+  int64_t n_lists = 0, n_list_entries = 0, n_list_weights = 0;
   // learned pair-contact closure
   bool cl_ready = false;        // closure data allocated (pdem_closure_setup)
   ClosureArgs ca{};
@@ -785,7 +785,9 @@ void build_rnp_tiles(pdem_ctx* c) {
 // Lists of the mixed tiles (DevTile).  Tiles with equal lists (the copies of
 // one mesh) share one: tiles are grouped by a hash of their degrees and
 // entries, the first of a group gives its list, and every tile's own list is
-// compared with the one it is given; a tile that differs gets its own.
+// compared with the one it is given; a tile that differs gets its own.  Where
+// the LDS tiles evaluate their weights (GEOM_MIN_ENTRIES), only the entries are
+// stored for them and compared; the HBM tiles' lists come first, with theirs.
 void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
   const size_t nt = tiles.size();
   if (nt == 0) return;
@@ -796,7 +798,9 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
   };
   put_tiles();
   std::vector<unsigned long long> hash(nt);
-  std::vector<int> diff(nt, 0), which;
+  std::vector<int> diff(nt, 0), which, lslice, order;
+  std::vector<uint32_t> lnode;
+  int64_t data = 0, hbm_data = 0;  // entries of all lists, of the HBM tiles'
   unsigned long long* d_hash = c->dalloc<unsigned long long>(nt, false);
   int* d_int = c->dalloc<int>(nt, false);
   const dim3 gt((unsigned)nt), tb(256);
@@ -804,13 +808,15 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
   check_launch(c);
   HIPCHK(hipMemcpyAsync(hash.data(), d_hash, nt * 8, hipMemcpyDeviceToHost, c->stream));
   HIPCHK(hipStreamSynchronize(c->stream));
-  for (int round = 0; round < 2; round++) {
+  // the lists of the groups and of the tiles in `diff`, laid out
+  auto lay_out = [&] {
     std::map<std::array<int64_t, 6>, size_t> first;
-    std::vector<uint32_t> lnode;
-    std::vector<int> lslice, order;
     which.clear();
-    int64_t data = 0, lds_data = 0;  // entries, of all lists and of the LDS tiles'
-    for (size_t k = 0; k < nt; k++) {
+    lslice.clear();
+    lnode.clear();
+    data = hbm_data = 0;
+    for (size_t q = 0; q < nt; q++) {
+      const size_t k = (q + nt - c->ntiles_global) % nt;  // (HBM tiles are the last)
       DevTile& t = tiles[k];
       const int n = t.te - t.ts, gs = (int)c->hp[t.pid].glob_start;
       const auto at = first.emplace(
@@ -846,11 +852,27 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
         len += (int64_t)((w + KB - 1) / KB) * KB * WAVE;
       }
       data += len;
-      if (t.lds) lds_data += len;
+      if (!t.lds) hbm_data = data;
       for (int q = 0; q < n; q++) lnode.push_back((uint32_t)order[q] | ((uint32_t)deg[order[q]] << 16));
     }
+  };
+  bool geom = false;
+  for (int round = 0;; round++) {
+    lay_out();
+    if (!geom && s.inf_type != 2 && data - hbm_data > GEOM_MIN_ENTRIES) {
+      // (tiles of equal entries and other weights then share their lists)
+      geom = true;
+      if (round > 0) {
+        std::fill(diff.begin(), diff.end(), 0);
+        round = 0;
+        lay_out();
+      }
+    }
+    c->n_lists = (int64_t)which.size();
+    c->n_list_entries = data;
+    c->n_list_weights = geom ? hbm_data : data;
     c->grow(c->d_col16, c->col16_cap, (size_t)data + 8);
-    c->grow(c->d_wgt, c->wgt_cap, (size_t)data + 8);
+    c->grow(c->d_wgt, c->wgt_cap, (size_t)c->n_list_weights + 8);
     c->grow(c->d_lnode, c->lnode_cap, lnode.size());
     c->grow(c->d_lslice, c->lslice_cap, lslice.size());
     HIPCHK(hipMemcpy(c->d_lnode, lnode.data(), lnode.size() * sizeof(uint32_t), hipMemcpyHostToDevice));
@@ -861,9 +883,7 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
     c->mixed.lslice = c->d_lslice;
     c->mixed.col16 = c->d_col16;
     c->mixed.wgt = c->d_wgt;
-    c->mixed.geom = lds_data > GEOM_MIN_ENTRIES && s.inf_type != 2 ? 1 : 0;
-    c->n_lists = (int64_t)which.size();
-    c->n_list_entries = data;
+    c->mixed.geom = geom ? 1 : 0;
     const dim3 gw((unsigned)which.size());
     dispatch(
         c,
@@ -2494,11 +2514,12 @@ int pdem_get_tile_counts(pdem_ctx* c, int32_t* lds_tiles, int32_t* hbm_tiles) {
   });
 }
 
-int pdem_get_list_info(pdem_ctx* c, int64_t* lists, int64_t* entries, int32_t* evaluated) {
+int pdem_get_list_info(pdem_ctx* c, int64_t* lists, int64_t* entries, int64_t* weights, int32_t* evaluated) {
   return guarded(c, [&] {
-    if (!lists || !entries || !evaluated) throw HipError{"null output pointer"};
+    if (!lists || !entries || !weights || !evaluated) throw HipError{"null output pointer"};
     *lists = c->n_lists;
     *entries = c->n_list_entries;
+    *weights = c->n_list_weights;
     *evaluated = c->mixed.geom;
   });
 }

@@ -1023,8 +1023,8 @@ __global__ void __launch_bounds__(256) k_list_fill(DS s, MixedArgs m, const int*
         const unsigned e = k < n ? (unsigned)list_entry(t, gs, j) : t.lds ? (unsigned)(t.we - t.ws) * 16u : 0u;
         if (k == kb) id0 = e;
         id[k - kb] = (uint16_t)e;
-        wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] =
-            k < n ? (float)bond_weight<DIM>(s, p, inv_scale, i, j, slack) : 0.f;
+        const double w = k < n ? bond_weight<DIM>(s, p, inv_scale, i, j, slack) : 0.;
+        if (!(m.geom && t.lds)) wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] = (float)w;
       }
       if (slack && t.lds) id[0] = (uint16_t)(id0 | SLACK_BLOCK);
     }
@@ -1032,7 +1032,7 @@ __global__ void __launch_bounds__(256) k_list_fill(DS s, MixedArgs m, const int*
 }
 
 // whether the tiles' own lists equal the ones they are given (degrees and
-// entries the same, weights within an ulp): diff[tile] is set where not
+// entries the same, weights, where they are read, within an ulp): diff[tile] is set where not
 template <int DIM>
 __global__ void __launch_bounds__(256) k_list_check(DS s, MixedArgs m, int* diff) {
   const DevTile t = m.tiles[blockIdx.x];
@@ -1057,7 +1057,9 @@ __global__ void __launch_bounds__(256) k_list_check(DS s, MixedArgs m, int* diff
         const int j = c[(int64_t)k * WAVE];
         const double w = bond_weight<DIM>(s, p, inv_scale, i, j, slack);
         bad |= (id[k - kb] & mask) != (unsigned)list_entry(t, gs, j);
-        bad |= !(fabs((double)m.wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] - w) <= 0x1p-23 * fabs(w));
+        if (!(m.geom && t.lds))
+          bad |= !(fabs((double)m.wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] - w) <=
+                   0x1p-23 * fabs(w));
       }
       bad |= t.lds && ((id[0] & SLACK_BLOCK) != 0) != slack;
     }
