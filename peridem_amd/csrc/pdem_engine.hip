@@ -296,21 +296,27 @@ struct Launch {
     else if (ma.ntiles_lds)
       hipLaunchKernelGGL((k_mixed_force<DIM, true, GEOM, T>), g, t, 0, st, c->ds, ma);
   }
-  static void hbm_first(pdem_ctx* c, hipStream_t st) {
+  // HBM tiles: lanes per node (MixedArgs::hbm_lpn); they read their weights
+  // with the Gaussian influence function only
+  template <int LPN>
+  static void hbm_lanes(pdem_ctx* c, hipStream_t st, bool first) {
     const MixedArgs& ma = c->mixed;
     const dim3 g(hbm_blocks(ma)), t(HBM_TPB);
-    if (ma.ntiles_hbm && ma.hbm_lpn == 8)
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB, LDS_NODES, 8>), g, t, 0, st, c->ds, ma);
-    else if (ma.ntiles_hbm)
-      hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB, LDS_NODES, 4>), g, t, 0, st, c->ds, ma);
+    if (c->ds.inf_type == 2) {
+      if (first)
+        hipLaunchKernelGGL((k_mixed_dilation<DIM, false, false, HBM_TPB, LDS_NODES, LPN>), g, t, 0, st, c->ds, ma);
+      else
+        hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB, LDS_NODES, LPN>), g, t, 0, st, c->ds, ma);
+    } else {
+      if (first)
+        hipLaunchKernelGGL((k_mixed_dilation<DIM, false, true, HBM_TPB, LDS_NODES, LPN>), g, t, 0, st, c->ds, ma);
+      else
+        hipLaunchKernelGGL((k_mixed_force<DIM, false, true, HBM_TPB, LDS_NODES, LPN>), g, t, 0, st, c->ds, ma);
+    }
   }
-  static void hbm_second(pdem_ctx* c, hipStream_t st) {
-    const MixedArgs& ma = c->mixed;
-    const dim3 g(hbm_blocks(ma)), t(HBM_TPB);
-    if (ma.ntiles_hbm && ma.hbm_lpn == 8)
-      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB, LDS_NODES, 8>), g, t, 0, st, c->ds, ma);
-    else if (ma.ntiles_hbm)
-      hipLaunchKernelGGL((k_mixed_force<DIM, false, false, HBM_TPB, LDS_NODES, 4>), g, t, 0, st, c->ds, ma);
+  static void hbm_pass(pdem_ctx* c, hipStream_t st, bool first) {
+    if (!c->mixed.ntiles_hbm) return;
+    c->mixed.hbm_lpn == 8 ? hbm_lanes<8>(c, st, first) : hbm_lanes<1>(c, st, first);
   }
   template <int T, bool GEOM>
   static void mixed_state(pdem_ctx* c) {
@@ -322,7 +328,7 @@ struct Launch {
       for (int pass = 0; pass < 2; pass++) {
         if (ma.ntiles_hbm) {
           fork(c);
-          pass == 0 ? hbm_first(c, c->side) : hbm_second(c, c->side);
+          hbm_pass(c, c->side, pass == 0);
           HIPCHK(hipEventRecord(c->ev_join, c->side));
         }
         pass == 0 ? open_first<T, GEOM>(c, c->stream) : open_second<T, GEOM>(c, c->stream);
@@ -349,9 +355,9 @@ struct Launch {
       auto es = ev_begin(c, c->side);
       mixed_umax(c, c->side);
       open_first<T, GEOM>(c, c->side);
-      hbm_first(c, c->side);
+      hbm_pass(c, c->side, true);
       open_second<T, GEOM>(c, c->side);
-      hbm_second(c, c->side);
+      hbm_pass(c, c->side, false);
       ev_end(c, es, c->side, grp);
       HIPCHK(hipEventRecord(c->ev_join, c->side));
       HIPCHK(hipStreamWaitEvent(c->stream, c->ev_join, 0));
@@ -785,9 +791,9 @@ void build_rnp_tiles(pdem_ctx* c) {
 // Lists of the mixed tiles (DevTile).  Tiles with equal lists (the copies of
 // one mesh) share one: tiles are grouped by a hash of their degrees and
 // entries, the first of a group gives its list, and every tile's own list is
-// compared with the one it is given; a tile that differs gets its own.  Where
-// the LDS tiles evaluate their weights (GEOM_MIN_ENTRIES), only the entries are
-// stored for them and compared; the HBM tiles' lists come first, with theirs.
+// compared with the one it is given; a tile that differs gets its own.  Only
+// lists that have weights (has_weights) are compared by them; those of the LDS
+// tiles come first.
 void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
   const size_t nt = tiles.size();
   if (nt == 0) return;
@@ -800,7 +806,7 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
   std::vector<unsigned long long> hash(nt);
   std::vector<int> diff(nt, 0), which, lslice, order;
   std::vector<uint32_t> lnode;
-  int64_t data = 0, hbm_data = 0;  // entries of all lists, of the HBM tiles'
+  int64_t data = 0, lds_data = 0;  // entries of all lists, of the LDS tiles'
   unsigned long long* d_hash = c->dalloc<unsigned long long>(nt, false);
   int* d_int = c->dalloc<int>(nt, false);
   const dim3 gt((unsigned)nt), tb(256);
@@ -814,9 +820,8 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
     which.clear();
     lslice.clear();
     lnode.clear();
-    data = hbm_data = 0;
-    for (size_t q = 0; q < nt; q++) {
-      const size_t k = (q + nt - c->ntiles_global) % nt;  // (HBM tiles are the last)
+    data = lds_data = 0;
+    for (size_t k = 0; k < nt; k++) {
       DevTile& t = tiles[k];
       const int n = t.te - t.ts, gs = (int)c->hp[t.pid].glob_start;
       const auto at = first.emplace(
@@ -834,12 +839,14 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
       t.node = (int)lnode.size();
       t.slice = (int)lslice.size();
       t.data = data;
-      // slots: nodes by their count of half blocks (most first), then by id;
-      // HBM tiles: by id
+      // slots: nodes by their count of half blocks (most first), then by id; HBM
+      // tiles of particles numbered in some order by id (see HBM_TPB)
       const int* deg = c->h_deg.data() + t.ts;
       order.resize(n);
       for (int q = 0; q < n; q++) order[q] = q;
-      if (t.lds)
+      int64_t span = 0;
+      for (int i = t.ts; i < t.te; i++) span += c->nbr_hi[i] - c->nbr_lo[i];
+      if (t.lds || span > (int64_t)(0.75 * n * (c->hp[t.pid].glob_end - gs)))
         std::stable_sort(order.begin(), order.end(), [&](int a, int b) {
           return (deg[a] + KB / 2 - 1) / (KB / 2) > (deg[b] + KB / 2 - 1) / (KB / 2);
         });
@@ -852,14 +859,14 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
         len += (int64_t)((w + KB - 1) / KB) * KB * WAVE;
       }
       data += len;
-      if (!t.lds) hbm_data = data;
+      if (t.lds) lds_data = data;
       for (int q = 0; q < n; q++) lnode.push_back((uint32_t)order[q] | ((uint32_t)deg[order[q]] << 16));
     }
   };
   bool geom = false;
   for (int round = 0;; round++) {
     lay_out();
-    if (!geom && s.inf_type != 2 && data - hbm_data > GEOM_MIN_ENTRIES) {
+    if (!geom && s.inf_type != 2 && lds_data > GEOM_MIN_ENTRIES) {
       // (tiles of equal entries and other weights then share their lists)
       geom = true;
       if (round > 0) {
@@ -870,7 +877,7 @@ void build_lists(pdem_ctx* c, std::vector<DevTile>& tiles) {
     }
     c->n_lists = (int64_t)which.size();
     c->n_list_entries = data;
-    c->n_list_weights = geom ? hbm_data : data;
+    c->n_list_weights = s.inf_type == 2 ? data : geom ? 0 : lds_data;
     c->grow(c->d_col16, c->col16_cap, (size_t)data + 8);
     c->grow(c->d_wgt, c->wgt_cap, (size_t)c->n_list_weights + 8);
     c->grow(c->d_lnode, c->lnode_cap, lnode.size());
@@ -985,7 +992,7 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
   c->mixed.ntiles_hbm = c->ntiles_global;
   int64_t hbm_nodes = 0;
   for (auto& t : tiles) hbm_nodes += t.lds ? 0 : t.te - t.ts;
-  c->mixed.hbm_lpn = hbm_nodes > HBM_LPN8_NODES ? 4 : 8;
+  c->mixed.hbm_lpn = hbm_nodes > HBM_LPN8_NODES ? 1 : 8;
   c->mixed.hbm_split = std::max(1, (int)(tile_max * c->mixed.hbm_lpn / HBM_TPB));
   c->tile_nodes = (int)tile_max;
   c->mixed.tiles = c->d_tiles;

@@ -63,25 +63,34 @@ constexpr int LDS_SMALL = 384;
 constexpr int LDS_MID = 1120;
 constexpr int KB = 8;             // neighbor ids per 16-byte block
 // HBM tiles (a meshed wall, a particle of many nodes) wait on gathers.  A tile
-// goes to several workgroups of HBM_TPB threads, all on one XCD (see
-// hbm_tile), whose L2 then holds its neighbors' data once; its nodes keep
-// their order, so that neighboring lanes gather neighboring nodes; and a
-// node's list is dealt to 8 lanes, or to 4 in models of more than HBM_LPN8_NODES
-// nodes in such tiles, which have enough wavefronts without.  Both passes, us,
-// before there were lanes to a node / 8 lanes of tiles over all XCDs / 8 / 4:
-//   sphere of 9.9k nodes            286    94    89   102
-//   sphere of 40k                   391   261   207   214
-//   10 of 9.9k                      343   377   258   264
-//   10 of 40k                      1005  1640  1100   972
-//   40 of 40k                      4615  6400  4106  3466
-//   10 of 9.9k, nodes in any order  913   650   591   576
+// goes to several workgroups of HBM_TPB threads, an eighth of the tiles to each
+// XCD (see hbm_tile), whose L2 then holds a particle's data once.  Bonds are
+// gathered 8 at a time, and their weights evaluated: read from the lists, they
+// would be three times the bytes that pass through the caches (the Gaussian
+// influence function's are read).  In models of up to HBM_LPN8_NODES nodes in
+// such tiles, a node's list is dealt to 8 lanes, for lack of wavefronts; above,
+// a lane each, so that neighboring lanes gather neighboring nodes.  For that
+// the nodes keep their order, unless it is an arbitrary one (lists that span
+// more than 3/4 of the particle), where lists of equal length go together.
+// Both passes, us: without lanes, a workgroup of 1024 a tile / 8 lanes, weights
+// read, tiles dealt to all XCDs / now; 8 lanes and one at the line:
+//   sphere of 9.9k nodes              286    94    87
+//   4 of 9.9k                         302   177   130 (one lane 204)
+//   10 of 9.9k                        342   377   209 (8 lanes 245)
+//   10 of 40k                        1005  1640   640
+//   40 of 40k                        4600  6400  2247
+//   20 disks of 40k                   323   727   292
+//   10 spheres of 9.9k, any order     916   650   502
+//   300 of 2.5k, any order           1700  4460  1740
 constexpr int HBM_TPB = 256;
-constexpr int64_t HBM_LPN8_NODES = 1 << 17;
+constexpr int64_t HBM_LPN8_NODES = 1 << 16;
 // waves per SIMD the bond kernels are compiled for (at most 64 VGPRs): two
 // 1024-thread workgroups per CU, so one stages its window while the other computes
 constexpr int MIXED_WAVES_PER_SIMD = 8;
-// the first pass of HBM tiles, whose positions are FP64, would spill
-constexpr int HBM_WAVES_PER_SIMD = 6;
+// HBM tiles, whose positions are FP64 and which take 8 bonds at once: first and
+// second pass (at 8 the registers spill: 10 spheres of 40k nodes 807 us for both
+// passes, 640 now)
+constexpr int HBM_WAVES_PER_SIMD = 4, HBM_WAVES2_PER_SIMD = 6;
 
 struct DevTile {
   int ts, te;     // nodes [ts, te)
@@ -165,11 +174,10 @@ __device__ __forceinline__ float max_nan(float a, float b) { return __builtin_el
 // threshold scaled once per particle.
 constexpr float REL_KEEP = 1.f - 1e-5f;
 
-// entry t of a block; in LDS tiles the first entry's top bit is a mark of the block
-template <bool LDS>
+// entry t of a block
 __device__ __forceinline__ int block_id(const uint4& b, int t) {
   const unsigned w = t < 2 ? b.x : t < 4 ? b.y : t < 6 ? b.z : b.w;
-  return (int)((w >> ((t & 1) * 16)) & (LDS ? 0x7fffu : 0xffffu));
+  return (int)((w >> ((t & 1) * 16)) & 0xffffu);
 }
 
 // Node data of the bond loops: the LDS window (LDS) or HBM.
@@ -564,7 +572,7 @@ __device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const Stat
                                               const typename Win<DIM, LDS>::Own& own, float us, bool tests, unsigned& brk) {
 #pragma clang fp contract(fast)
   Block1 o{0., {0.f, 0.f, 0.f}, 0.f};
-  const bool slack = GEOM && (cur.x & SLACK_BLOCK);
+  const bool slack = GEOM && (!LDS || (cur.x & SLACK_BLOCK));
   // one bond; SURE that it is whole and stays so
   auto bond = [&](const int e, const float wt, const int tt, auto sure) {
     constexpr bool SURE = decltype(sure)::value;
@@ -615,16 +623,22 @@ __device__ __forceinline__ Block1 first_block(const Win<DIM, LDS>& w, const Stat
     if (o.z <= c.thr4 && !slack) return o;
     o = Block1{0., {0.f, 0.f, 0.f}, 0.f};
   }
+  if (!LDS) {
+#pragma unroll
+    for (int tt = 0; tt < KB; tt++)
+      if (tt < left) bond(block_id(cur, tt), GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], tt, std::false_type{});
+    return o;
+  }
   // with tests, two entries at a time: blocks with a bond that breaks now or
-  // has no length left or (GEOM) is in the slack, those of a wavefront that
-  // holds broken bonds, and every block of an HBM tile
+  // has no length left or (GEOM) is in the slack, and those of a wavefront that
+  // holds broken bonds
 #pragma unroll 1
   for (int tt = 0; tt < KB && tt < left; tt += 2) {
     float2 wt = make_float2(0.f, 0.f);
     if (!GEOM) wt = *(const float2*)((const float*)(wg + (tt / 4) * WAVE) + tt % 4);
-    bond((int)(cur.x & (LDS ? 0x7fffu : 0xffffu)), wt.x, tt, std::false_type{});
+    bond((int)(cur.x & 0x7fffu), wt.x, tt, std::false_type{});
     pin(o.f, o.z);
-    if (LDS || tt + 1 < left) bond((int)((cur.x >> 16) & 0xffffu), wt.y, tt + 1, std::false_type{});
+    bond((int)(cur.x >> 16), wt.y, tt + 1, std::false_type{});
     cur.x = cur.y;
     cur.y = cur.z;
     cur.z = cur.w;
@@ -728,7 +742,7 @@ __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const State
 #pragma clang fp contract(fast)
   // one bond (whole: SURE that it is not broken)
   auto bond = [&](const int tt, const float wt, auto whole, auto exact) {
-    const int e = block_id<LDS>(cur, tt);
+    const int e = block_id(cur, tt) & (LDS ? 0x7fff : 0xffff);  // (the first entry's top bit in LDS tiles: SLACK_BLOCK)
     float wj = wt;
     if (GEOM) {
       const float4 xvj = w.x2(e);
@@ -771,9 +785,15 @@ __device__ __forceinline__ void second_block(const Win<DIM, LDS>& w, const State
       block(no);
     return;
   }
-  const int nb = left < KB ? left : KB;
+  if (!LDS) {
+#pragma unroll
+    for (int tt = 0; tt < KB; tt++)
+      if (tt < left && !((wblk >> tt) & 1u))
+        bond(tt, GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], yes, yes);
+    return;
+  }
 #pragma unroll 1
-  for (int tt = 0; tt < nb; tt++) bond(tt, GEOM ? 0.f : ((const float*)(wg + (tt / 4) * WAVE))[tt % 4], no, yes);
+  for (int tt = 0; tt < KB && tt < left; tt++) bond(tt, 0.f, no, yes);  // (GEOM, in the slack)
 }
 
 // Second pass of the node in thread slot q: adds the b terms to f.
@@ -827,14 +847,14 @@ __device__ __forceinline__ void second_pass_node(const DS& s, const MixedArgs& m
 // Tile ranges of MixedArgs::tiles: closed LDS tiles (whole particles, fused
 // kernel), open LDS tiles, HBM tiles.  An HBM tile is shared by hbm_split
 // workgroups of HBM_TPB threads (there is no window to stage).  Workgroups go
-// to the 8 XCDs in turn, so those of a tile are 8 apart; the last group of 8
-// tiles may be incomplete (hbm_blocks() workgroups, hbm_tile() beyond the tiles).
+// to the 8 XCDs in turn; an XCD takes an eighth of the tiles, one after the
+// other with all of their workgroups (the last may find fewer: hbm_blocks()
+// workgroups, hbm_tile() beyond the tiles).
 constexpr int XCDS = 8;
-__host__ inline unsigned hbm_blocks(const MixedArgs& m) {
-  return (unsigned)((m.ntiles_hbm + XCDS - 1) / XCDS * XCDS * m.hbm_split);
-}
+__host__ __device__ inline int hbm_per_xcd(const MixedArgs& m) { return (m.ntiles_hbm + XCDS - 1) / XCDS; }
+__host__ inline unsigned hbm_blocks(const MixedArgs& m) { return (unsigned)(XCDS * hbm_per_xcd(m) * m.hbm_split); }
 __device__ __forceinline__ int hbm_tile(const MixedArgs& m) {
-  return (int)blockIdx.x / (XCDS * m.hbm_split) * XCDS + (int)blockIdx.x % XCDS;
+  return (int)blockIdx.x % XCDS * hbm_per_xcd(m) + (int)blockIdx.x / XCDS / m.hbm_split;
 }
 template <bool LDS>
 __device__ __forceinline__ const DevTile& tile_of(const MixedArgs& m) {
@@ -906,7 +926,7 @@ __global__ void __launch_bounds__(TPB, LDS ? MIXED_WAVES_PER_SIMD : HBM_WAVES_PE
 
 // Second pass of the open tiles.
 template <int DIM, bool LDS, bool GEOM, int TPB, int NODES = LDS_NODES, int LPN = 1>
-__global__ void __launch_bounds__(TPB, MIXED_WAVES_PER_SIMD) k_mixed_force(DS s, MixedArgs m) {
+__global__ void __launch_bounds__(TPB, LDS ? MIXED_WAVES_PER_SIMD : HBM_WAVES2_PER_SIMD) k_mixed_force(DS s, MixedArgs m) {
   if (!LDS && hbm_tile(m) >= m.ntiles_hbm) return;
   PDEM_WINDOW_LDS(LDS, NODES, false, true, GEOM)
   const DevTile t = tile_of<LDS>(m);
@@ -961,6 +981,12 @@ __global__ void k_zero_noforce(DS s) {
 }
 
 // Set-up of the lists (see DevTile).
+
+// whether a tile's list has weights: where it reads them (HBM tiles evaluate
+// theirs but for the Gaussian influence function's)
+__device__ __forceinline__ bool has_weights(const DS& s, const MixedArgs& m, const DevTile& t) {
+  return s.inf_type == 2 || (t.lds && !m.geom);
+}
 
 // weight 2 r J(r) V_j^c / particle_scale of a bond (materialUtil.cpp:21-73, m_x's terms)
 template <int DIM>
@@ -1024,7 +1050,7 @@ __global__ void __launch_bounds__(256) k_list_fill(DS s, MixedArgs m, const int*
         if (k == kb) id0 = e;
         id[k - kb] = (uint16_t)e;
         const double w = k < n ? bond_weight<DIM>(s, p, inv_scale, i, j, slack) : 0.;
-        if (!(m.geom && t.lds)) wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] = (float)w;
+        if (has_weights(s, m, t)) wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] = (float)w;
       }
       if (slack && t.lds) id[0] = (uint16_t)(id0 | SLACK_BLOCK);
     }
@@ -1057,7 +1083,7 @@ __global__ void __launch_bounds__(256) k_list_check(DS s, MixedArgs m, int* diff
         const int j = c[(int64_t)k * WAVE];
         const double w = bond_weight<DIM>(s, p, inv_scale, i, j, slack);
         bad |= (id[k - kb] & mask) != (unsigned)list_entry(t, gs, j);
-        if (!(m.geom && t.lds))
+        if (has_weights(s, m, t))
           bad |= !(fabs((double)m.wgt[at + (int64_t)(k / 4) * WAVE * 4 + (q % WAVE) * 4 + k % 4] - w) <=
                    0x1p-23 * fabs(w));
       }

@@ -1,9 +1,10 @@
 """HBM tiles of the mixed bond kernels (particles whose numbering spreads their
-neighbors): 8 lanes a node or, in large models, 4, tiles dealt to workgroups of
-one XCD in groups of 8.  Tile counts around the groups and both lane counts
-against the FP64 oracle (tolerances as in test_gpu_mixed.py: 1e-4 max, 1e-5
-RMS of the largest force), and a particle's results bit for bit the same in a
-model of one particle and in one that takes 4 lanes."""
+neighbors): 8 lanes a node or, in large models, one; an eighth of the tiles to
+an XCD; nodes in mesh order or in any; weights evaluated, or read with the
+Gaussian influence function.  Against the FP64 oracle (tolerances as in
+test_gpu_mixed.py: 1e-4 max, 1e-5 RMS of the largest force), and a particle's
+results bit for bit the same in a model of one particle and in one that takes
+one lane."""
 import numpy as np
 import pytest
 
@@ -15,13 +16,14 @@ import oracle
 pytestmark = pytest.mark.gpu
 
 
-def _model(copies, nodes):
+def _model(copies, nodes, shuffle=True, inf=capi.INF_LINEAR):
     rng = np.random.default_rng(41)
     R = 1e-3
     h = R * (4.18879 / nodes) ** (1 / 3)
     x, vol = ball_mesh(R, h)
-    x = x[rng.permutation(len(x))]
-    b = ModelBuilder(3, 1e-9, [ZoneDeck(configs.pdstate_material(K=5e7))], {}, multi_particle=False)
+    if shuffle:
+        x = x[rng.permutation(len(x))]
+    b = ModelBuilder(3, 1e-9, [ZoneDeck(configs.pdstate_material(K=5e7, inf=inf))], {}, multi_particle=False)
     for k in range(copies):
         b.add_particle(0, x + np.array([5 * R * k, 0.0, 0.0]), vol, center_node(x, (0, 0, 0), R), R)
     return b.build(name="hbm", h_override=[h] * copies)
@@ -47,10 +49,13 @@ def _run(e, spec):
     return tuple(e.field(k) for k in (capi.FIELD_F, capi.FIELD_THETA, capi.FIELD_Z, capi.FIELD_BONDS))
 
 
-@pytest.mark.parametrize("copies,nodes", [(1, 2200), (4, 1500), (5, 2200), (50, 2800)])
-def test_hbm_tiles(copies, nodes):
-    spec = _model(copies, nodes)
-    print(f"[hbm] {copies} x {nodes}: {spec.n_nodes} nodes", flush=True)
+@pytest.mark.parametrize("copies,nodes,shuffle,inf", [
+    (1, 2200, True, capi.INF_LINEAR), (4, 1500, True, capi.INF_LINEAR), (5, 2200, True, capi.INF_CONST),
+    (2, 4000, False, capi.INF_LINEAR), (3, 2200, True, capi.INF_GAUSSIAN), (30, 2800, True, capi.INF_LINEAR),
+    (20, 4000, False, capi.INF_LINEAR), (30, 2800, True, capi.INF_GAUSSIAN)])
+def test_hbm_tiles(copies, nodes, shuffle, inf):
+    spec = _model(copies, nodes, shuffle, inf)
+    print(f"[hbm] {copies} x {nodes} shuffle={shuffle} inf={inf}: {spec.n_nodes} nodes", flush=True)
     g = capi.GpuEngine(spec, capi.PREC_MIXED)
     assert g.tile_counts()[0] == 0
     r = oracle.OracleEngine(spec, 8)
@@ -66,12 +71,14 @@ def test_hbm_tiles(copies, nodes):
     r.close()
 
 
-def test_lanes_agree():
-    one, many = _model(1, 2800), _model(50, 2800)
-    assert one.n_nodes <= 131072 < many.n_nodes
+@pytest.mark.parametrize("shuffle,inf", [(True, capi.INF_LINEAR), (False, capi.INF_LINEAR), (True, capi.INF_GAUSSIAN)])
+def test_lanes_agree(shuffle, inf):
+    one, many = _model(1, 4000, shuffle, inf), _model(20, 4000, shuffle, inf)
+    assert one.n_nodes <= 65536 < many.n_nodes
     out = []
     for spec in (one, many):
         g = capi.GpuEngine(spec, capi.PREC_MIXED)
+        assert g.tile_counts()[0] == 0
         n = one.n_nodes
         out.append([a[:n] for a in _run(g, spec)[:3]])
         g.close()

@@ -1,6 +1,7 @@
-"""Which bond weights a mixed-precision model stores: those of every distinct
-list while the LDS tiles read them, and none for LDS tiles where they evaluate
-them.  Tiles with the same entries then share a list whatever their weights."""
+"""Which bond weights a mixed-precision model stores: those of the LDS tiles'
+distinct lists while the tiles read them, none where they evaluate them, and
+HBM tiles' with the Gaussian influence function only.  Tiles with the same
+entries share a list whatever their weights where these are evaluated."""
 import numpy as np
 import pytest
 
@@ -38,7 +39,9 @@ def _model(kinds, inf=capi.INF_LINEAR):
     ("cvv", capi.INF_LINEAR, 3, False, "all"),
     ("v" * 40, capi.INF_LINEAR, 1, True, "none"),          # 40 lists would be evaluated; then they are one
     ("m" * 40 + "vvc", capi.INF_CONST, 41, True, "none"),
-    ("m" * 40 + "ch", capi.INF_LINEAR, 44, True, "hbm"),   # 3 HBM tiles
+    ("m" * 40 + "ch", capi.INF_LINEAR, 44, True, "none"),  # 3 HBM tiles
+    ("vch", capi.INF_LINEAR, 5, False, "lds"),
+    ("hvch", capi.INF_GAUSSIAN, 8, False, "all"),
     ("v" * 40, capi.INF_GAUSSIAN, 40, False, "all"),
 ])
 def test_stored_weights(kinds, inf, lists, evaluated, weights):
@@ -48,10 +51,9 @@ def test_stored_weights(kinds, inf, lists, evaluated, weights):
     n, entries, ev, w = g.list_info()
     print(f"[weights]   {n} lists of {entries} entries, {w} weights, evaluated={ev} tiles {g.tile_counts()}", flush=True)
     assert ev == evaluated and n == lists
-    if weights == "hbm":
-        p = spec.particles[-1]
+    if weights == "lds":  # whole slices of 64 nodes and blocks of 8 bonds
         rp, _ = g.neighbors(capi.NEIGH_PD)
-        bonds = rp[p["glob_end"]] - rp[p["glob_start"]]
+        bonds = rp[spec.particles[1]["glob_end"]]
         assert bonds <= w < 2 * bonds < entries
     else:
         assert w == (entries if weights == "all" else 0)
