@@ -268,7 +268,7 @@ struct Launch {
   }
   static void mixed_umax(pdem_ctx* c, hipStream_t st) {
     if (c->mixed.n_open_pids > 0)
-      hipLaunchKernelGGL(k_mixed_umax<DIM>, dim3(c->mixed.n_open_pids), dim3(256), 0, st, c->ds, c->mixed);
+      hipLaunchKernelGGL(k_mixed_umax<DIM>, dim3(c->mixed.n_open_pids), dim3(1024), 0, st, c->ds, c->mixed);
   }
   // The state-based passes of the mixed kernels: closed tiles (whole
   // particles) in the fused kernel on the engine stream; open LDS tiles and

@@ -346,8 +346,8 @@ struct PartMax {
 
 // the maxima of the particles with open LDS tiles: one workgroup each
 template <int DIM>
-__global__ void __launch_bounds__(256) k_mixed_umax(DS s, MixedArgs m) {
-  __shared__ float4 red[256 / WAVE];
+__global__ void __launch_bounds__(1024) k_mixed_umax(DS s, MixedArgs m) {
+  __shared__ float4 red[1024 / WAVE];
   const int pid = m.open_pids[blockIdx.x];
   const DevParticle& p = s.P[pid];
   const int64_t gs = p.glob_start;
@@ -389,7 +389,9 @@ __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, c
   const int gs = (int)s.P[t.pid].glob_start;
   double u0[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) u0[d] = s.u[d][gs];
-  const bool closed = t.lds == 2;
+  constexpr bool CLOSED = FIRST && SECOND;
+  float4 mf = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (!CLOSED) mf = m.pmax[t.pid];
   PartMax mx;
   for (int q = threadIdx.x; q < nw; q += blockDim.x) {
     const int j = t.ws + q;
@@ -397,15 +399,14 @@ __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, c
     for (int d = 0; d < DIM; d++) xd[d] = s.xr[d][j] - org[d];
     if (FIRST || GEOM)
       lx[q] = make_float4(2.f * (float)xd[0], 2.f * (float)xd[1], 2.f * (float)xd[2], (float)(s.vol[j] * inv_scale));
-    if (closed || SECOND) {
+    if (SECOND) {
       for (int d = 0; d < DIM; d++) du[d] = s.u[d][j] - u0[d];
-      if (closed) mx.node<DIM>(xd, du);
-    }
-    if (SECOND)
+      if (CLOSED) mx.node<DIM>(xd, du);
       ly[q] = make_int4(__float_as_int((float)(xd[0] + du[0])), __float_as_int((float)(xd[1] + du[1])),
                         __float_as_int((float)(xd[2] + du[2])), FIRST ? 0 : __float_as_int(m.fb[j]));
+    }
   }
-  const float4 mf = closed ? mx.group(red) : m.pmax[t.pid];
+  if (CLOSED) mf = mx.group(red);
   fixed = __builtin_amdgcn_readfirstlane(mf.y > FIXED_FROM * mf.z);
   const int eu = fixed_exp(mf.x);
   if (FIRST) {
