@@ -977,7 +977,7 @@ void build_tiles(pdem_ctx* c, int64_t tile_max) {
     std::sort(open.begin(), open.end());
     open.erase(std::unique(open.begin(), open.end()), open.end());
     if (!c->mixed.open_pids) c->mixed.open_pids = c->dalloc<int>(std::max(1, c->np));
-    if (!c->mixed.pmax) c->mixed.pmax = c->dalloc<float4>(std::max(1, c->np));
+    if (!c->mixed.pmax) c->mixed.pmax = c->dalloc<float2>(std::max(1, c->np));
     if (!open.empty())
       HIPCHK(hipMemcpy((void*)c->mixed.open_pids, open.data(), open.size() * sizeof(int), hipMemcpyHostToDevice));
     c->mixed.n_open_pids = (int)open.size();
@@ -1415,6 +1415,10 @@ void build(pdem_ctx* c, const pdem_desc* d) {
     hipLaunchKernelGGL(k_mixed_alpha, dim3(blocks(N)), dim3(TPB), 0, c->stream, s, fa);
     check_launch(c);
     c->mixed.fa = fa;
+    PartConst* part = c->dalloc<PartConst>(std::max(1, c->np));
+    if (c->np > 0) hipLaunchKernelGGL(k_mixed_part, dim3(c->np), dim3(256), 0, c->stream, s, dim, part);
+    check_launch(c);
+    c->mixed.part = part;
   }
   if (c->multi) {
     Ctrl h2 = h;

@@ -109,7 +109,16 @@ struct DevTile {
   int64_t data;
 };
 
+// constants of a particle (set-up): particle_scale and its reciprocal, the
+// largest component of the reference positions relative to the first node's
+// (rounded up)
+struct PartConst {
+  double scale, inv_scale;
+  float xmax;
+};
+
 struct MixedArgs {
+  const PartConst* part;  // [np]
   const DevTile* tiles;   // closed LDS tiles, then open LDS tiles, then HBM tiles
   int ntiles_closed, ntiles_lds, ntiles_hbm;
   int hbm_lpn, hbm_split; // HBM tiles: lanes per node, workgroups per tile
@@ -129,7 +138,7 @@ struct MixedArgs {
   // fixed-point steps of their windows
   const int* open_pids;
   int n_open_pids;
-  float4* pmax;           // [np]
+  float2* pmax;           // [np]
 };
 
 // The bond weights are read from the lists while the lists of the LDS tiles
@@ -315,31 +324,28 @@ struct Win {
   }
 };
 
+__device__ __forceinline__ float round_up(double a) { return (float)(a * (1.0 + 0x1p-20)); }
 // Largest components over a particle's nodes, relative to its first node: the
-// displacement, the current and the reference position
+// displacement and the current position
 struct PartMax {
-  double u = 0., y = 0., x = 0.;
+  double u = 0., y = 0.;
   template <int DIM>
   __device__ __forceinline__ void node(const double* xd, const double* du) {
     for (int d = 0; d < DIM; d++) {
       u = fmax(u, fabs(du[d]));
       y = fmax(y, fabs(xd[d] + du[d]));
-      x = fmax(x, fabs(xd[d]));
     }
   }
   // the workgroup's maxima as floats rounded up (the fixed-point steps only
   // have to bound them); they do not depend on the order, so every tile of a
   // particle gets the same values
-  __device__ __forceinline__ float4 group(float4* red) const {
-    auto up = [](double a) { return (float)(a * (1.0 + 0x1p-20)); };
-    float4 m = make_float4(up(u), up(y), up(x), 0.f);
-    auto join = [&](float a, float b, float c) {
-      m = make_float4(fmaxf(m.x, a), fmaxf(m.y, b), fmaxf(m.z, c), 0.f);
-    };
-    for (int o = WAVE / 2; o > 0; o >>= 1) join(__shfl_xor(m.x, o), __shfl_xor(m.y, o), __shfl_xor(m.z, o));
+  __device__ __forceinline__ float2 group(float2* red) const {
+    float2 m = make_float2(round_up(u), round_up(y));
+    auto join = [&](float a, float b) { m = make_float2(fmaxf(m.x, a), fmaxf(m.y, b)); };
+    for (int o = WAVE / 2; o > 0; o >>= 1) join(__shfl_xor(m.x, o), __shfl_xor(m.y, o));
     if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = m;
     __syncthreads();
-    for (int w = 0; w < (int)(blockDim.x / WAVE); w++) join(red[w].x, red[w].y, red[w].z);
+    for (int w = 0; w < (int)(blockDim.x / WAVE); w++) join(red[w].x, red[w].y);
     return m;
   }
 };
@@ -347,7 +353,7 @@ struct PartMax {
 // the maxima of the particles with open LDS tiles: one workgroup each
 template <int DIM>
 __global__ void __launch_bounds__(1024) k_mixed_umax(DS s, MixedArgs m) {
-  __shared__ float4 red[1024 / WAVE];
+  __shared__ float2 red[1024 / WAVE];
   const int pid = m.open_pids[blockIdx.x];
   const DevParticle& p = s.P[pid];
   const int64_t gs = p.glob_start;
@@ -360,7 +366,7 @@ __global__ void __launch_bounds__(1024) k_mixed_umax(DS s, MixedArgs m) {
     }
     mx.node<DIM>(xd, du);
   }
-  const float4 mf = mx.group(red);
+  const float2 mf = mx.group(red);
   if (threadIdx.x == 0) m.pmax[pid] = mf;
 }
 
@@ -384,13 +390,13 @@ __device__ __forceinline__ int fixed_exp(float mf) {
 template <int DIM, bool FIRST, bool SECOND, bool GEOM>
 __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, const DevTile& t, float4* lx,
                                               int4* lq, int4* ly, const double* org, double inv_scale,
-                                              float4* red, bool& fixed) {
+                                              float2* red, bool& fixed) {
   const int nw = t.we - t.ws;
   const int gs = (int)s.P[t.pid].glob_start;
   double u0[3] = {0., 0., 0.};
   for (int d = 0; d < DIM; d++) u0[d] = s.u[d][gs];
   constexpr bool CLOSED = FIRST && SECOND;
-  float4 mf = make_float4(0.f, 0.f, 0.f, 0.f);
+  float2 mf = make_float2(0.f, 0.f);
   if (!CLOSED) mf = m.pmax[t.pid];
   PartMax mx;
   for (int q = threadIdx.x; q < nw; q += blockDim.x) {
@@ -407,7 +413,7 @@ __device__ __forceinline__ float stage_window(const DS& s, const MixedArgs& m, c
     }
   }
   if (CLOSED) mf = mx.group(red);
-  fixed = __builtin_amdgcn_readfirstlane(mf.y > FIXED_FROM * mf.z);
+  fixed = __builtin_amdgcn_readfirstlane(mf.y > FIXED_FROM * m.part[t.pid].xmax);
   const int eu = fixed_exp(mf.x);
   if (FIRST) {
     const double inv_us = ldexp(1., -eu);
@@ -446,13 +452,14 @@ struct StateConsts {
   // GEOM: J = ja + jb r2 (constant and linear influence functions), volume
   // correction up_h - r2 inv_h2 where r2 > low2
   float ja, jb, low2, inv_h2, up_h;
-  __device__ StateConsts(const DS& s, const DevParticle& p) {
+  __device__ StateConsts(const DS& s, const MixedArgs& m, int pid) {
+    const DevParticle& p = s.P[pid];
     thr4 = uniform(0.25f * ((float)(p.mat[2] + 1.0e-10) / REL_KEEP));
     inv_s0 = uniform((float)(1.0 / p.mat[2]));
     Rc = uniform((float)p.Rc);
     K = p.mat[0];
     G = p.mat[1];
-    scale = particle_scale(s, p);
+    scale = m.part[pid].scale;
     Kn = uniform((float)(p.Kn * scale));
     ja = uniform((float)s.inf_p0);
     jb = uniform(s.inf_type == 1 ? (float)(0.5 * s.inf_p1 / p.horizon) : 0.f);
@@ -896,10 +903,10 @@ __device__ __forceinline__ void second_pass(const DS& s, const MixedArgs& m, con
   __shared__ float4 lx[(LDS_ON) && ((FIRST) || (GEOM)) ? (NODES) + 1 : 1]; \
   __shared__ int4 lq[(LDS_ON) && (FIRST) ? (NODES) + 1 : 1];   \
   __shared__ int4 ly[(LDS_ON) && (SECOND) ? (NODES) + 1 : 1];  \
-  __shared__ float4 red[1024 / WAVE];
+  __shared__ float2 red[1024 / WAVE];
 #define PDEM_WINDOW(DIM, LDS_ON, t, gs) \
   Win<DIM, LDS_ON> w{(const char*)lx, (const char*)lq, (const char*)ly, &s, &m, gs, t.ws, 1.f, \
-                      1. / particle_scale(s, p), {0., 0., 0.}}; \
+                      m.part[t.pid].inv_scale, {0., 0., 0.}}; \
   for (int d = 0; d < DIM; d++) w.org[d] = s.xr[d][gs];
 
 // First pass of the open tiles (tiles that do not hold a whole particle:
@@ -914,7 +921,7 @@ __global__ void __launch_bounds__(TPB, LDS ? MIXED_WAVES_PER_SIMD : HBM_WAVES_PE
   PDEM_WINDOW(DIM, LDS, t, gs)
   bool fixed = false;
   if (LDS) w.us = stage_window<DIM, true, false, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
-  const StateConsts c(s, p);
+  const StateConsts c(s, m, t.pid);
   const int nr = slot_rounds<LDS, LPN>(m, t);
   for (int it = 0; it < nr; it++) {
     const int q = slot_of<LDS, LPN>(m, it);
@@ -936,7 +943,7 @@ __global__ void __launch_bounds__(TPB, LDS ? MIXED_WAVES_PER_SIMD : HBM_WAVES2_P
   PDEM_WINDOW(DIM, LDS, t, gs)
   bool fixed = false;
   if (LDS) stage_window<DIM, false, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
-  const StateConsts c(s, p);
+  const StateConsts c(s, m, t.pid);
   second_pass<DIM, LDS, GEOM, LPN>(s, m, t, w, c, fixed);
 }
 
@@ -953,7 +960,7 @@ __global__ void __launch_bounds__(TPB, TPB == 512 ? 6 : MIXED_WAVES_PER_SIMD) k_
   PDEM_WINDOW(DIM, true, t, gs)
   bool fixed;
   w.us = stage_window<DIM, true, true, GEOM>(s, m, t, lx, lq, ly, w.org, w.inv_scale, red, fixed);
-  const StateConsts c(s, p);
+  const StateConsts c(s, m, t.pid);
   const int nr = slot_rounds<true, 1>(m, t);
   for (int it = 0; it < nr; it++) {
     const int q = slot_of<true, 1>(m, it);
@@ -1092,6 +1099,23 @@ __global__ void __launch_bounds__(256) k_list_check(DS s, MixedArgs m, int* diff
     }
   }
   if (bad) diff[blockIdx.x] = 1;
+}
+
+// the particles' constants (set-up); a workgroup each
+__global__ void __launch_bounds__(256) k_mixed_part(DS s, int dim, PartConst* out) {
+  __shared__ float red[256 / WAVE];
+  const DevParticle& p = s.P[blockIdx.x];
+  const int64_t gs = p.glob_start;
+  double x = 0.;
+  for (int64_t j = gs + threadIdx.x; j < p.glob_end; j += blockDim.x)
+    for (int d = 0; d < dim; d++) x = fmax(x, fabs(s.xr[d][j] - s.xr[d][gs]));
+  float mf = round_up(x);
+  for (int o = WAVE / 2; o > 0; o >>= 1) mf = fmaxf(mf, __shfl_xor(mf, o));
+  if ((threadIdx.x & (WAVE - 1)) == 0) red[threadIdx.x / WAVE] = mf;
+  __syncthreads();
+  if (threadIdx.x != 0 || p.glob_end <= gs) return;
+  const double c = particle_scale(s, p);
+  out[blockIdx.x] = PartConst{c, 1. / c, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]))};
 }
 
 // the nodes' constant alpha terms (set-up)
