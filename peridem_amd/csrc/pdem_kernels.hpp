@@ -852,7 +852,12 @@ __global__ void k_fbc(DS s, DevBc bc) {
 // a y by its exact remainder (Markstein, IBM J. Res. Dev. 34, 1990: the first
 // leaves the quotient within an ulp, the second rounds it), 5 instructions
 // where a division of its own takes about 15.  For divisors that several
-// quotients share.
+// quotients share.  Holds while the remainder is no subnormal number, |a| above
+// 2^-969, and a, b and y are finite and not 0: lengths, mesh sizes, horizons.
+// The RNP law's numerator falls below that where a bond that does not break is
+// drawn to 36 times its critical stretch (a force of 1e-290 of its scale, which
+// may then differ in its last digit); a critical stretch of 0 or infinity gives
+// NaN instead of infinity or 0, and neither is stored as damage.
 __device__ __forceinline__ double div_by(double a, double b, double y) {
   double q = a * y;
   q = __builtin_fma(__builtin_fma(-b, q, a), y, q);
