@@ -206,6 +206,16 @@ dim3 grad_grid(int64_t nwg) {
 // at most; 100000 rows: 469 us a call before, 326 kept).
 constexpr int64_t PIN_ROWS = 16384, KEEP_ROWS = 1 << 18;
 
+// whether p is memory that the host cannot read (device rows go through copies)
+bool device_memory(const void* p) {
+  hipPointerAttribute_t a{};
+  if (hipPointerGetAttributes(&a, p) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return a.type == hipMemoryTypeDevice;
+}
+
 mlp::Net net_of(const pdem_mlp* m) { return mlp::make_net(m->wb, m->wtb, m->p, m->norm); }
 
 void ensure_partial(pdem_mlp* m, int64_t nwg) {
@@ -354,6 +364,7 @@ int pdem_mlp_forward(pdem_mlp* m, const float* x, int64_t n, float* y) {
   return mguard(m, [&] {
     if (n < 0) throw HipError{"negative row count"};
     if (n == 0) return;
+    if (!x || !y) throw HipError{"null row pointer"};
     const size_t bx = n * mlp::NIN * sizeof(float), by = n * mlp::NOUT * sizeof(float);
     auto infer = [&](const float* X, float* Y) {
       hipLaunchKernelGGL(mlp::k_mlp_infer, dim3((unsigned)((n + 63) / 64)), dim3(256), 0, m->stream, net_of(m), X, n, Y);
@@ -361,7 +372,7 @@ int pdem_mlp_forward(pdem_mlp* m, const float* x, int64_t n, float* y) {
     };
     // the kept buffers serve one call at a time; a call beside it brings its own
     std::unique_lock<std::mutex> own(m->io, std::try_to_lock);
-    if (own && n <= PIN_ROWS) {
+    if (own && n <= PIN_ROWS && !device_memory(x) && !device_memory(y)) {
       if (n > m->pin_rows) {
         int64_t rows = 256;
         while (rows < n) rows *= 2;
