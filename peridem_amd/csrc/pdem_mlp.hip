@@ -372,7 +372,7 @@ int pdem_mlp_forward(pdem_mlp* m, const float* x, int64_t n, float* y) {
     };
     // the kept buffers serve one call at a time; a call beside it brings its own
     std::unique_lock<std::mutex> own(m->io, std::try_to_lock);
-    if (own && n <= PIN_ROWS && !device_memory(x) && !device_memory(y)) {
+    if (own && n <= PIN_ROWS && !device_memory(x)) {
       if (n > m->pin_rows) {
         int64_t rows = 256;
         while (rows < n) rows *= 2;
@@ -385,8 +385,10 @@ int pdem_mlp_forward(pdem_mlp* m, const float* x, int64_t n, float* y) {
       float *px = (float*)m->pin, *py = px + n * mlp::NIN;
       std::memcpy(px, x, bx);
       infer(px, py);
+      const bool copy = device_memory(y);  // (asked while the kernel runs)
+      if (copy) HIPCHK(hipMemcpyAsync(y, py, by, hipMemcpyHostToDevice, m->stream));
       HIPCHK(hipStreamSynchronize(m->stream));
-      std::memcpy(y, py, by);
+      if (!copy) std::memcpy(y, py, by);
       return;
     }
     const bool keep = own && n <= KEEP_ROWS;
