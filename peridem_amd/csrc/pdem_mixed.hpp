@@ -15,20 +15,21 @@
 //
 // Neighbor ids are 16-bit, stored in blocks of KB = 8 per lane: one 16-byte
 // load yields a lane's next 8 ids and the block loop is unrolled so each id is
-// a compile-time lane of the block.  Beside each id lies the bond's constant
-// weight (its reference geometry: r J(r) V_j^c), so the loops evaluate only
-// what moves.
-//
-// (Models of many different meshes evaluate the weights instead, see
-// GEOM_MIN_ENTRIES.)
+// a compile-time lane of the block.  In models of few different meshes the
+// bond's constant weight (its reference geometry: r J(r) V_j^c) lies beside
+// each id, so the loops evaluate only what moves; models of many evaluate the
+// weights (GEOM_MIN_ENTRIES), and so do HBM tiles.
 //
 // Lists are shared: the particles of a model are mostly scaled and turned
 // copies of a few meshes, whose tiles then have the same relative ids and,
 // up to the particle's scale h V, the same weights.  Set-up finds such tiles
 // (by hash, then by comparing every entry) and stores one list for all of
-// them, which stays in L2: on the packing of 2000 spheres the lists of 1.4e8
-// bonds (0.9 GB) shrink to a few of 0.4 MB.  A tile whose list matches no
-// other keeps its own.
+// them.  512-instance ensemble: 17167 particles, 78 lists of 0.54M entries (3 MB
+// with the weights, which stay in L2).  Packing of 2000 spheres, 1.4e8 bonds:
+// 101 lists of 7.3M entries (15 MB of ids), nearly all of them of one sphere
+// each, whose bonds as long as the horizon fall on either side of it by the
+// rounding of its turn; that is too many to read weights, and its tiles
+// evaluate them.  A tile whose list matches no other keeps its own.
 //
 // Threads take nodes in slot order: inside every LDS tile the nodes are ordered
 // by their number of 4-bond half blocks (most first, node id second), so the
@@ -145,8 +146,9 @@ struct MixedArgs {
 // hold at most this many entries (6 bytes each; an XCD's L2 holds 4 MB) and
 // evaluated from the reference positions beyond it, where their lists would
 // come from HBM in both passes (constant and linear influence functions; the
-// Gaussian one costs an exponential, so its weights are always read).
-// Measured with the particles' lists shared by 1 / 16 / 64 / 256 / no others,
+// Gaussian one costs an exponential, so its weights are always read).  Lists
+// that read none have none stored (has_weights).
+// Measured with 1 / 16 / 64 / 256 lists of equal use and one for each particle,
 // step in us, read and evaluated: packing of 2000 spheres of 1021 nodes (76k
 // entries each) 478, 499, 521, 562, 645 against 486, 488, 490, 499, 518;
 // 512-instance ensemble of particles of up to 367 nodes (12k entries)
@@ -509,11 +511,13 @@ __device__ __forceinline__ bool slack_bond(double r, double low) {
 // from the bond's weight and the neighbors' current positions.
 //
 // The loops are bound by FP32 instruction issue and the latency of the list
-// reads.  Per bond in 3D they take 42 instructions in the first pass and 14 in
-// the second (of which 3 and 1 are half-rate transcendentals); with the
-// reference geometry evaluated in both passes and the alpha part in the second
-// they took 57 each.  Packing of 2000 spheres, both passes of a step: 409 us
-// before, 325 us now (kernel trace), 412 MB against 179 MB fetched.
+// reads.  Per bond in 3D they take 42 VALU instructions in the first pass and 14
+// in the second with weights from the lists, 47 and 28 evaluating them (of which
+// 3 and 1 or 2 are half-rate transcendentals); with the reference geometry
+// evaluated in both passes and the alpha part in the second they took 57 each.
+// Packing of 2000 spheres (weights evaluated), both passes of a step: 409 us with
+// the alpha part in the second, 328 us now (kernel trace), 412 MB against 134 MB
+// fetched.
 //
 // The loops take 4 bonds at a time without any test per bond: the lists are
 // padded to whole blocks (see Win), and a block whose largest stretch says that
